@@ -18,11 +18,10 @@ everything else FP64).  The max relative error of
 Anderson loop over 1.6 GB state vectors is outside the timed path).  `value` is the FP32-MFMA path's
 iterations/s when every error is <= 1e-6, else the FP64 path's (`config.value_path`).
 
-`roofline` is the BSE contraction, the iteration's largest kernel family (BSE_L_K3! + BSE_K3!, four
-launches per iteration): on the FP32 path HBM-bound, algorithmic 168 B per K3 element of the three
-channels per iteration (gemm_roofline) over the launches' HIP-event time, with `traffic` the rocprofv3
-FETCH + WRITE bytes per launch (profiles/c2_bse_gemm_traffic.txt); on the FP64 path MFMA-bound
-(executed flops 8 BM BN Nν3 per computed tile).  `roofline_bubble` is the lattice bubble kernel
+`roofline` is the BSE contraction, the iteration's largest kernel (k_bse3: BSE_L_K3! and BSE_K3! of the three
+channels in one launch): MFMA-bound (executed flops 8 BM BN Nν3 per computed tile over the launch's HIP-event
+time), with its algorithmic bytes beside (gemm_roofline) and `traffic` the rocprofv3 FETCH + WRITE bytes per
+launch (profiles/c2_bse_gemm_traffic.txt).  `roofline_bubble` is the lattice bubble kernel
 (k_bubble_nl, bubbles_real_space!): G(R) read once, Πpp and Πph written on the band chunks and the
 chunk sums, over its HIP-event time; `traffic` from profiles/c2_bubble_nl_traffic.txt.  `cpu_baseline` times the CPU
 restatement of the reference loops (oracle/) on a stated bounded sample of the same workload, at one
@@ -300,22 +299,16 @@ def tune_gemm_grid(S, grids=(0, 256, 512, 768, 1024), lk3_grids=(0, 160, 192, 22
 
 
 def gemm_roofline(head, P, gemm_peak, traffic, n3P):
-    """Roofline object of the BSE contraction GEMMs.  FP32 path: HBM-bound (their epilogues and FP32 operands
-    move 168 B per K3 element of the three channels per iteration, every K3 array in FP32: FL.K3 and the
-    FP32 right operand written by BSE_L_K3! (24 + 24), FL.a read for its t post-processing (8); BSE_K3! reads
-    A32, R32, FL.K3, FL.a for the t self term and Fbuff.a for the t post-processing (24 + 24 + 24 + 8 + 8) and
-    writes Fbuff.K3 (24)); the MFMA rate is stated beside.  FP64 path: MFMA-bound (executed flops)."""
+    """Roofline object of the BSE contractions, one kernel for both equations of the three channels (k_bse3):
+    MFMA-bound (executed flops); its algorithmic bytes (F.K3 read once, FL.K3 and Fbuff.K3 written once: nine
+    values of 8 B, FP64 path 16 B, per K3 element) and HBM rate beside."""
     t = P["t_gemm"]
     mfma = P["f_exec"] / t
-    kern = ("k_lk3_pb64 (BSE_L_K3!) + zgemm_tiles_t (BSE_K3!), FP32 MFMA" if head == "fp32"
-            else "zgemm_tiles_t (FP64 MFMA, BSE_L_K3! + BSE_K3!)")
-    common = {"kernel": kern + ", 4 launches per iteration",
-              "launches_per_iteration": 4, "ms_per_iteration": t * 1e3, "traffic": traffic,
-              "executed_flops_per_iteration": P["f_exec"], "mfma_tflops": mfma / 1e12, "mfma_frac": mfma / gemm_peak}
-    if head == "fp32":
-        b = 168.0 * n3P / 4
-        return dict({"bound": "hbm", "achieved": b / (t / 4) / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
-                     "frac": b / (t / 4) / HBM_PEAK, "algorithmic_bytes_per_launch": b}, **common)
+    b = (72.0 if head == "fp32" else 144.0) * n3P
+    common = {"kernel": f"k_bse3 (BSE_L_K3! + BSE_K3!), {head.upper()} MFMA, one launch per iteration",
+              "launches_per_iteration": 1, "ms_per_iteration": t * 1e3, "traffic": traffic,
+              "executed_flops_per_iteration": P["f_exec"], "mfma_tflops": mfma / 1e12, "mfma_frac": mfma / gemm_peak,
+              "algorithmic_bytes_per_launch": b, "hbm_gbs": b / t / 1e9}
     return dict({"bound": "mfma", "achieved": mfma / 1e12, "peak": gemm_peak / 1e12, "unit": "TFLOP/s",
                  "frac": mfma / gemm_peak}, **common)
 
@@ -396,8 +389,7 @@ def main_c2(args):
                             "bse_tflops_dense_equiv": paths["fp64"]["bse_tflops_dense_equiv"],
                             "stage_ms": paths["fp64"]["st"]},
                    "speedup_fp32_over_fp64": paths["fp64"]["ms"] / paths["fp32"]["ms"]},
-        # the dominant kernel: the BSE contraction GEMMs (four launches per iteration: BSE_L_K3! p+a and t,
-        # BSE_K3! p+a and t), over their summed durations (HIP events, one kernel at a time)
+        # the dominant kernel: the BSE contractions (HIP events, one kernel at a time)
         "roofline": gemm_roofline(head, P, gemm_peak, gemm_traffic, NW3 * NV3 * NV3 * NP),
         "roofline_bubble": {"bound": "hbm", "achieved": b_bubble / t_bub / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                             "frac": b_bubble / t_bub / HBM_PEAK,
@@ -457,9 +449,9 @@ def main_c4(args):
     G.set_timing(False)
     # algorithmic flops of one grouped launch: 3 channels x 8 flop per complex MAC, dense per point
     f_launch = sum(3 * 8.0 * (2 * w["nK3"][0] - 1) * w["L"] ** 2 * (2 * w["nK3"][1]) ** 3 for w in ws)
-    tf_l, tf_k = f_launch / (gl * 1e-3) / 1e12, f_launch / (gk * 1e-3) / 1e12
-    log(f"bench c4: {ms:.1f} ms per sweep iteration; grouped GEMMs {gl:.2f} ms ({tf_l:.1f} TFLOP/s) and "
-        f"{gk:.2f} ms ({tf_k:.1f} TFLOP/s)")
+    # (both equations of the members on k_bse3 count with the second time)
+    tf = 2 * f_launch / ((gl + gk) * 1e-3) / 1e12
+    log(f"bench c4: {ms:.1f} ms per sweep iteration; contractions {gl + gk:.2f} ms ({tf:.1f} TFLOP/s)")
     G.close()
     solo = []
     for Sk in S:   # the same points one after the other (eager, each alone)
@@ -472,9 +464,8 @@ def main_c4(args):
         "steps": args.steps, "warmup": args.warmup,
         "sweep_ms_per_iteration": ms, "sweep_iters_per_s": 1000.0 / ms,
         "points_one_after_another_ms": sum(solo),
-        "grouped_gemm": {"L_K3_ms": gl, "K3_ms": gk, "flops_per_launch": f_launch,
-                         "L_K3_tflops": tf_l, "K3_tflops": tf_k, "peak_tflops_fp32": peak,
-                         "roofline_frac": max(tf_l, tf_k) / peak},
+        "contractions": {"ms": gl + gk, "flops": 2 * f_launch, "tflops": tf, "peak_tflops_fp32": peak,
+                         "roofline_frac": tf / peak},
         "autotuned": tuned}), flush=True)
 
 

@@ -17,6 +17,7 @@
 #include "../../include/fdga.h"
 #include "fdga_kernels.h"
 #include "fdga_adjoint.h"
+#include "fdga_bse3.h"
 #include "fdga_forms.h"
 #include "fdga_sym.h"
 
@@ -1317,6 +1318,30 @@ static int launch_k3(fdga_ctx* c, const int* chans, int n, bool mfrg = false) {
     return k3_finish(c, c->Fb, chans, n, false, sym, t_epi);
 }
 
+// BSE_L_K3! and BSE_K3! of the three channels in one kernel (k_bse3): the lattice fdPA iterations without
+// K3 symmetry groups, in FP64, or in FP32 with every K3 array in its FP32 form
+static bool bse3_fused(const fdga_ctx* c) {
+    if (c->NP == 1 || c->NV3 > bse3_max(c->d.precision == FDGA_FP32)) return false;
+    if (k3_sym(c, kChansAll, 3, true) || k3_sym(c, kChansAll, 3, false)) return false;
+    return c->d.precision == FDGA_FP64 || fl32_mode(c);
+}
+// (fl_prepare has put FL.K3, F.K3 and Fbuff.K3 into the form of the context's iterations)
+static int launch_bse3(fdga_ctx* c) {
+    auto chan = [&](int ch) {
+        return Bse3Chan{c->cache[idx_gamma(ch)], c->cache[idx_f0(ch)], c->cache[ch == PCH ? 0 : ch == ACH ? 10 : 11],
+                        c->cache[idx_fbase(ch)], pi_of(c, ch, false), pi_of(c, ch, true), c->F[ch].K2, c->F[ch].K3,
+                        c->FL[ch].K3, c->Fb[ch].K3};
+    };
+    const Bse3Args a{k3geom(c), c->d.T, chan(PCH), chan(ACH), chan(TCH)};
+    c->r32_fresh = 0;
+    kernel_begin(c);
+    const hipError_t e = c->d.precision == FDGA_FP32 ? bse3_launch<true>(a, (size_t)c->kgrid[1], c->run)
+                                                     : bse3_launch<false>(a, (size_t)c->kgrid[1], c->run);
+    if (e != hipSuccess) return fail(c, "BSE_L_K3 / BSE_K3 launch failed", -3);
+    kernel_end(c, 10);
+    return 0;
+}
+
 // ---------------------------------------------------------------------------------------
 // the is_mfRG forms of BSE_K1!/BSE_K2! and the _new forms (fdga_forms.h): one wave per output class
 template <int FORM, int CH>
@@ -2076,8 +2101,12 @@ static int iterate_two_chains(fdga_ctx* c, int32_t strategy, int32_t update_sigm
     if (rc) return -3;
     // chain A on st
     if (fdga_build_k3_cache(c)) return -3;
-    if (strategy == FDGA_FDPA && launch_lk3(c, all, 3)) return -3;
-    if (launch_k3(c, all, 3)) return -3;
+    if (strategy == FDGA_FDPA && bse3_fused(c)) {
+        if (launch_bse3(c)) return -3;
+    } else {
+        if (strategy == FDGA_FDPA && launch_lk3(c, all, 3)) return -3;
+        if (launch_k3(c, all, 3)) return -3;
+    }
     // join
     HIPCHK(c, hipEventRecord(c->evjoin, c->st2));
     HIPCHK(c, hipStreamWaitEvent(c->st, c->evjoin, 0));
@@ -2096,13 +2125,14 @@ static int iterate_new(fdga_ctx* c, int32_t strategy, int32_t update_sigma, int3
     stage_begin(c);
     if (fdga_build_k3_cache(c)) return -3;
     stage_end(c, 1);
-    if (strategy == FDGA_FDPA_NEW) {
+    const bool fused = strategy == FDGA_FDPA_NEW && bse3_fused(c);
+    if (strategy == FDGA_FDPA_NEW && !fused) {
         stage_begin(c);
         if (launch_lk3(c, all, 3)) return -3;
         stage_end(c, 3);
     }
     stage_begin(c);
-    if (launch_k3(c, all, 3)) return -3;
+    if (fused ? launch_bse3(c) : launch_k3(c, all, 3)) return -3;
     stage_end(c, 6);
     stage_begin(c);
     for (int ch : all)
@@ -2177,13 +2207,14 @@ static int iterate_eager(fdga_ctx* c, int32_t strategy, int32_t update_sigma, in
     stage_begin(c);
     if (fdga_build_k3_cache(c)) return -3;
     stage_end(c, 1);
+    const bool fused = strategy == FDGA_FDPA && bse3_fused(c);   // both K3 equations in stage 6
     if (strategy == FDGA_FDPA) {
         stage_begin(c);
         if (launch_lk2_pa(c) || fdga_bse_l_k2(c, TCH)) return -3;
         stage_end(c, 2);
         stage_begin(c);
         const int all[3] = {PCH, ACH, TCH};
-        if (launch_lk3(c, all, 3)) return -3;
+        if (!fused && launch_lk3(c, all, 3)) return -3;
         stage_end(c, 3);
     }
     stage_begin(c);
@@ -2200,7 +2231,7 @@ static int iterate_eager(fdga_ctx* c, int32_t strategy, int32_t update_sigma, in
     stage_begin(c);
     {
         const int all[3] = {PCH, ACH, TCH};
-        if (launch_k3(c, all, 3)) return -3;
+        if (fused ? launch_bse3(c) : launch_k3(c, all, 3)) return -3;
     }
     stage_end(c, 6);
     stage_begin(c);
@@ -2556,7 +2587,9 @@ struct fdga_group {
     std::string err;
     int* boff = nullptr;             // first batch of each member in the launch's batch space
     std::vector<int> boff_h;
-    GroupItems gi[TILE_N];
+    GroupItems gi[TILE_N];     // every member's items
+    GroupItems giu[TILE_N];    // the items of the members outside k_bse3 (the fdPA contractions)
+    int nfused = 0;            // members whose fdPA contractions run in k_bse3
     // per-member functors on the device: BSE_L_K3! (independent of the F/Fbuff state) and BSE_K3!
     // for each F/Fbuff pointer state
     LK3_Aop* lk3a = nullptr;
@@ -2595,14 +2628,16 @@ bool has_k3_groups(const fdga_ctx* c) {
 }
 
 // work items of one tile shape: members in order of decreasing box (the larger items first), each
-// member's batches in chunks of 8 with the tiles of a batch on one XCD (item index mod 8)
-int group_build_items(fdga_group* g, int tile) {
-    GroupItems& gi = g->gi[tile];
-    if (gi.items) return 0;
+// member's batches in chunks of 8 with the tiles of a batch on one XCD (item index mod 8); unfused: only
+// the members outside k_bse3
+int group_build_list(fdga_group* g, int tile, bool unfused) {
+    GroupItems& gi = unfused ? g->giu[tile] : g->gi[tile];
+    if (gi.geo) return 0;
     const int BM = tile_bm(tile), BN = tile_bn(tile);
     std::vector<GemmGroupGeom> geo((size_t)g->n);
-    std::vector<int> order((size_t)g->n);
-    for (int j = 0; j < g->n; ++j) order[(size_t)j] = j;
+    std::vector<int> order;
+    for (int j = 0; j < g->n; ++j)
+        if (!unfused || !bse3_fused(g->m[(size_t)j])) order.push_back(j);
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return g->m[(size_t)a]->NV3 > g->m[(size_t)b]->NV3; });
     std::vector<int> items, items_t;
     int64_t computed = 0;
@@ -2633,10 +2668,10 @@ int group_build_items(fdga_group* g, int tile) {
             add(items, j, tiles, 0, nb);
         }
     }
-    GHIPCHK(g, hipMalloc((void**)&gi.items, items.size() * sizeof(int)));
-    GHIPCHK(g, hipMalloc((void**)&gi.geo, geo.size() * sizeof(GemmGroupGeom)));
-    GHIPCHK(g, hipMemcpy(gi.items, items.data(), items.size() * sizeof(int), hipMemcpyHostToDevice));
-    GHIPCHK(g, hipMemcpy(gi.geo, geo.data(), geo.size() * sizeof(GemmGroupGeom), hipMemcpyHostToDevice));
+    if (!items.empty()) {
+        GHIPCHK(g, hipMalloc((void**)&gi.items, items.size() * sizeof(int)));
+        GHIPCHK(g, hipMemcpy(gi.items, items.data(), items.size() * sizeof(int), hipMemcpyHostToDevice));
+    }
     if (!items_t.empty()) {
         GHIPCHK(g, hipMalloc((void**)&gi.items_t, items_t.size() * sizeof(int)));
         GHIPCHK(g, hipMemcpy(gi.items_t, items_t.data(), items_t.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -2644,7 +2679,13 @@ int group_build_items(fdga_group* g, int tile) {
     gi.nitems = (int)items.size();
     gi.nitems_t = (int)items_t.size();
     gi.computed = computed;
+    GHIPCHK(g, hipMalloc((void**)&gi.geo, geo.size() * sizeof(GemmGroupGeom)));
+    GHIPCHK(g, hipMemcpy(gi.geo, geo.data(), geo.size() * sizeof(GemmGroupGeom), hipMemcpyHostToDevice));
     return 0;
+}
+int group_build_items(fdga_group* g, int tile) {
+    if (group_build_list(g, tile, false)) return -2;
+    return g->nfused ? group_build_list(g, tile, true) : 0;
 }
 
 template <class T>
@@ -2714,11 +2755,7 @@ void group_graphs_invalidate(fdga_group* g) {
             }
 }
 
-size_t group_grid(const fdga_group* g, int which, bool t_launch = false) {
-    const GroupItems& gi = g->gi[g->tile[which]];
-    const size_t n = (size_t)(t_launch ? gi.nitems_t : gi.nitems);
-    return g->grid[which] ? std::min(g->grid[which], n) : n;
-}
+size_t group_grid(const fdga_group* g, int which, size_t n) { return g->grid[which] ? std::min(g->grid[which], n) : n; }
 
 // one launch of the grouped contraction `which` (0 BSE_L_K3!, 1 BSE_K3!) over the item list `sc`
 hipError_t group_gemm_launch(fdga_group* g, int which, const GemmSchedGroup& sc, size_t grid) {
@@ -2746,18 +2783,20 @@ hipError_t group_gemm_launch(fdga_group* g, int which, const GemmSchedGroup& sc,
 }
 
 // the grouped contraction `which` (0 BSE_L_K3!, 1 BSE_K3!) on the group's stream: one launch, or for
-// lattice groups the p and a channels and then the t channel
-int group_gemm(fdga_group* g, int which) {
-    const GroupItems& gi = g->gi[g->tile[which]];
+// lattice groups the p and a channels and then the t channel; unfused: of the members outside k_bse3
+int group_gemm(fdga_group* g, int which, bool unfused = false) {
+    const GroupItems& gi = unfused && g->nfused ? g->giu[g->tile[which]] : g->gi[g->tile[which]];
     if (which == 1) {
         const int s = g->m[0]->swap_state;
         for (const fdga_ctx* c : g->m)
             if (c->swap_state != s) return gfail(g, "group members are not at the same iteration (F/Fbuff state)");
     }
     if (g->timing) GHIPCHK(g, hipEventRecord(g->tev[0], g->st));
-    hipError_t e = group_gemm_launch(g, which, GemmSchedGroup{gi.items, gi.geo, gi.nitems}, group_grid(g, which));
+    hipError_t e = group_gemm_launch(g, which, GemmSchedGroup{gi.items, gi.geo, gi.nitems},
+                                     group_grid(g, which, (size_t)gi.nitems));
     if (e == hipSuccess && gi.nitems_t)
-        e = group_gemm_launch(g, which, GemmSchedGroup{gi.items_t, gi.geo, gi.nitems_t}, group_grid(g, which, true));
+        e = group_gemm_launch(g, which, GemmSchedGroup{gi.items_t, gi.geo, gi.nitems_t},
+                              group_grid(g, which, (size_t)gi.nitems_t));
     if (e != hipSuccess) return gfail(g, std::string("grouped GEMM launch: ") + hipGetErrorString(e), -3);
     if (g->timing) {
         GHIPCHK(g, hipEventRecord(g->tev[1], g->st));
@@ -2785,27 +2824,50 @@ int group_join(fdga_group* g) {
 }
 int member_err(fdga_group* g, const fdga_ctx* c) { return gfail(g, std::string("member: ") + c->err, -3); }
 
-// one iterate_solver! of every member (src/solve.jl:4-116), the contractions grouped
+// the fdPA contractions of the members on k_bse3: each on its own stream, or (event timing on) one after
+// the other on the group's stream, their time counted with the grouped BSE_K3!
+int group_bse3(fdga_group* g, fdga_ctx* c) {
+    if (!g->timing) return launch_bse3(c) ? member_err(g, c) : 0;
+    c->run = g->st;
+    GHIPCHK(g, hipEventRecord(g->tev[0], g->st));
+    const int rc = launch_bse3(c);
+    c->run = c->st;
+    if (rc) return member_err(g, c);
+    GHIPCHK(g, hipEventRecord(g->tev[1], g->st));
+    GHIPCHK(g, hipEventSynchronize(g->tev[1]));
+    float ms = 0.f;
+    GHIPCHK(g, hipEventElapsedTime(&ms, g->tev[0], g->tev[1]));
+    g->gemm_ms[1] += ms;
+    return 0;
+}
+
+// one iterate_solver! of every member (src/solve.jl:4-116): the contractions of the fdPA members that
+// qualify in one k_bse3 launch each on the member's stream (as on the member alone), the others' grouped
 int group_iterate_eager(fdga_group* g, int strategy, int update_sigma) {
     const int all[3] = {PCH, ACH, TCH};
+    const bool fd = strategy == FDGA_FDPA;
+    std::vector<char> fused;
     for (fdga_ctx* c : g->m) {
         if (has_k3_groups(c)) return gfail(g, "group members must not have K3 symmetry groups installed");
         c->run = c->st;
+        fused.push_back(fd && bse3_fused(c));
     }
+    const bool gemms = !fd || g->nfused < g->n;
     if (group_fork(g)) return -2;
     for (fdga_ctx* c : g->m) {
         if (update_sigma && (fdga_dyson(c) || fdga_bubbles(c))) return member_err(g, c);
         if (fdga_build_k3_cache(c)) return member_err(g, c);
-        if (strategy == FDGA_FDPA)
+        if (fd)
             for (int ch : {PCH, ACH, TCH})
                 if (fdga_bse_l_k2(c, ch)) return member_err(g, c);
     }
-    if (strategy == FDGA_FDPA) {
-        if (group_join(g) || group_gemm(g, 0) || group_fork(g)) return -3;
-        for (fdga_ctx* c : g->m)
-            if (k3_finish(c, c->FL, all, 3, true, false, g->nonlocal)) return member_err(g, c);
+    if (fd && gemms) {
+        if (group_join(g) || group_gemm(g, 0, true) || group_fork(g)) return -3;
+        for (size_t j = 0; j < fused.size(); ++j)
+            if (!fused[j] && k3_finish(g->m[j], g->m[j]->FL, all, 3, true, false, g->nonlocal)) return member_err(g, g->m[j]);
     }
-    for (fdga_ctx* c : g->m) {
+    for (size_t j = 0; j < fused.size(); ++j) {
+        fdga_ctx* c = g->m[j];
         if (launch_w_all(c)) return member_err(g, c);
         c->w_fresh = 1;
         int rc = 0;
@@ -2813,13 +2875,24 @@ int group_iterate_eager(fdga_group* g, int strategy, int update_sigma) {
         rc = rc ? rc : launch_k2_all(c);
         c->w_fresh = 0;
         if (rc) return member_err(g, c);
+        if (fused[j]) {
+            if (!g->timing && group_bse3(g, c)) return -3;
+            continue;
+        }
         // fdPA: the grouped BSE_L_K3! epilogue wrote the FP32 lattice right operands
-        const bool skipR = strategy == FDGA_FDPA && g->lk3_ro;
+        const bool skipR = fd && g->lk3_ro;
         if (k3_rhs(c, k3_set(c, all, 3, false, false), 3, false, skipR)) return member_err(g, c);
     }
-    if (group_join(g) || group_gemm(g, 1) || group_fork(g)) return -3;
-    for (fdga_ctx* c : g->m) {
-        if (k3_finish(c, c->Fb, all, 3, false, false, g->nonlocal)) return member_err(g, c);
+    if (gemms || g->timing) {
+        if (group_join(g)) return -3;
+        if (gemms && group_gemm(g, 1, fd)) return -3;
+        for (size_t j = 0; j < fused.size(); ++j)
+            if (fused[j] && g->timing && group_bse3(g, g->m[j])) return -3;
+        if (group_fork(g)) return -3;
+    }
+    for (size_t j = 0; j < fused.size(); ++j) {
+        fdga_ctx* c = g->m[j];
+        if (!fused[j] && k3_finish(c, c->Fb, all, 3, false, false, g->nonlocal)) return member_err(g, c);
         if (fdga_update_F(c)) return member_err(g, c);
         if (update_sigma && fdga_sde(c, strategy, 1)) return member_err(g, c);
     }
@@ -2890,7 +2963,10 @@ int fdga_group_create(fdga_group** out, fdga_ctx* const* members, int32_t n) {
         g->boff_h[(size_t)j + 1] = g->boff_h[(size_t)j] + (int)nb;
     }
     if (group_upload(g, &g->boff, g->boff_h)) return -2;
-    for (fdga_ctx* c : g->m) GHIPCHK(g, hipStreamSynchronize(c->st));
+    for (fdga_ctx* c : g->m) {
+        g->nfused += bse3_fused(c);
+        GHIPCHK(g, hipStreamSynchronize(c->st));
+    }
     if (group_build_items(g, TILE_64x64) || group_build_functors(g)) return -2;
     return 0;
 }
@@ -2899,11 +2975,12 @@ int fdga_group_destroy(fdga_group* g) {
     if (!g) return 0;
     if (g->st) (void)hipStreamSynchronize(g->st);
     group_graphs_invalidate(g);
-    for (auto& gi : g->gi) {
-        if (gi.items) (void)hipFree(gi.items);
-        if (gi.items_t) (void)hipFree(gi.items_t);
-        if (gi.geo) (void)hipFree(gi.geo);
-    }
+    for (GroupItems* list : {g->gi, g->giu})
+        for (int t = 0; t < TILE_N; ++t) {
+            if (list[t].items) (void)hipFree(list[t].items);
+            if (list[t].items_t) (void)hipFree(list[t].items_t);
+            if (list[t].geo) (void)hipFree(list[t].geo);
+        }
     for (void* p : {(void*)g->boff, (void*)g->lk3a, (void*)g->lk3b, (void*)g->lk3e, (void*)g->lk3er, g->k3a[0], g->k3a[1], g->k3b[0],
                     g->k3b[1], (void*)g->k3e[0], (void*)g->k3e[1]})
         if (p) (void)hipFree(p);
