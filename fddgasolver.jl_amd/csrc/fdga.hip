@@ -2251,9 +2251,25 @@ int64_t fdga_flat_size_F(const fdga_ctx* c) { return (int64_t)(3 * (c->n1 + c->n
 }  // extern "C"
 
 namespace {
+FlatArgs flat_args(fdga_ctx* c) {
+    FlatArgs a{};
+    for (int r = 0; r < 3; ++r) {
+        a.K1[r] = c->F[r].K1;
+        a.K2[r] = c->F[r].K2;
+        a.K3[r] = c->F[r].K3;
+    }
+    a.Sig = c->Sig;
+    a.n1 = c->n1 * c->NP;
+    a.n2 = c->n2 * c->NP;
+    a.n3 = c->n3 * c->NP;
+    a.NW = c->NW3;
+    a.NV = c->NV3;
+    a.k3f = c->fk32;
+    return a;
+}
 // x (host, reference layout [γp; γt; γa] of K1, K2, K3, then Σ when `sigma`) into the device arrays;
 // the vertex part is multiplied by `scale`
-// `buf`: the staging buffer (nullptr: the context's, allocated on first use)
+// `buf`: the staging buffer (nullptr: the context's, allocated on first use); it holds x afterwards
 int unflatten_into(fdga_ctx* c, const double* x, bool sigma, double scale, double2* buf = nullptr) {
     const size_t n = (size_t)(sigma ? fdga_flat_size(c) : fdga_flat_size_F(c));
     if (!buf) {
@@ -2261,49 +2277,24 @@ int unflatten_into(fdga_ctx* c, const double* x, bool sigma, double scale, doubl
         buf = c->stage;
     }
     HIPCHK(c, hipMemcpyAsync(buf, x, n * sizeof(double2), hipMemcpyHostToDevice, c->st));
-    if (scale != 1.0) {
-        const size_t nf = (size_t)fdga_flat_size_F(c);
-        k_axpby<<<cdiv(nf, 256), 256, 0, c->run>>>(buf, buf, scale, 0.0, nf);
-        LAUNCHCHK(c);
-    }
-    size_t off = 0;
-    for (int r = 0; r < 3; ++r) {
-        HIPCHK(c, hipMemcpyAsync(c->F[r].K1, buf + off, c->n1 * c->NP * sizeof(double2), hipMemcpyDeviceToDevice, c->st));
-        off += c->n1 * c->NP;
-        HIPCHK(c, hipMemcpyAsync(c->F[r].K2, buf + off, c->n2 * c->NP * sizeof(double2), hipMemcpyDeviceToDevice, c->st));
-        off += c->n2 * c->NP;
-        if (c->fk32)
-            k_k3_to_dev32<<<cdiv(c->n3 * c->NP, 256), 256, 0, c->run>>>(reinterpret_cast<float2*>(c->F[r].K3), buf + off,
-                                                                          c->NW3, c->NV3, c->NP);
-        else k_k3_to_dev<<<cdiv(c->n3 * c->NP, 256), 256, 0, c->run>>>(c->F[r].K3, buf + off, c->NW3, c->NV3, c->NP);
-        LAUNCHCHK(c);
-        off += c->n3 * c->NP;
-    }
-    if (sigma) HIPCHK(c, hipMemcpyAsync(c->Sig, buf + off, c->nGel * sizeof(double2), hipMemcpyDeviceToDevice, c->st));
+    k_unflatten<<<cdiv(n, 256), 256, 0, c->run>>>(flat_args(c), buf, scale, n);
+    LAUNCHCHK(c);
     if (refresh_avg(c)) return -3;
     return 0;
 }
-// the device arrays into x (host, the same layout); synchronises the stream
-int flatten_from(fdga_ctx* c, double* x, bool sigma, double2* buf = nullptr) {
+// the device arrays into x (host, the same layout); synchronises the stream.  op 1: the residual arrays - x,
+// op 2: x - arrays / f, with the argument x still in the staging buffer from unflatten_into
+int flatten_from(fdga_ctx* c, double* x, bool sigma, double2* buf = nullptr, int op = 0, double f = 1.0) {
     const size_t n = (size_t)(sigma ? fdga_flat_size(c) : fdga_flat_size_F(c));
     if (!buf) {
         if (ensure_stage(c, n)) return -2;
         buf = c->stage;
     }
-    size_t off = 0;
-    for (int r = 0; r < 3; ++r) {
-        HIPCHK(c, hipMemcpyAsync(buf + off, c->F[r].K1, c->n1 * c->NP * sizeof(double2), hipMemcpyDeviceToDevice, c->st));
-        off += c->n1 * c->NP;
-        HIPCHK(c, hipMemcpyAsync(buf + off, c->F[r].K2, c->n2 * c->NP * sizeof(double2), hipMemcpyDeviceToDevice, c->st));
-        off += c->n2 * c->NP;
-        if (c->fk32)
-            k_k3_to_ref32<<<cdiv(c->n3 * c->NP, 256), 256, 0, c->run>>>(buf + off, reinterpret_cast<const float2*>(c->F[r].K3),
-                                                                          c->NW3, c->NV3, c->NP);
-        else k_k3_to_ref<<<cdiv(c->n3 * c->NP, 256), 256, 0, c->run>>>(buf + off, c->F[r].K3, c->NW3, c->NV3, c->NP);
-        LAUNCHCHK(c);
-        off += c->n3 * c->NP;
-    }
-    if (sigma) HIPCHK(c, hipMemcpyAsync(buf + off, c->Sig, c->nGel * sizeof(double2), hipMemcpyDeviceToDevice, c->st));
+    const FlatArgs a = flat_args(c);
+    if (op == 0) k_flatten<0><<<cdiv(n, 256), 256, 0, c->run>>>(a, buf, f, n);
+    else if (op == 1) k_flatten<1><<<cdiv(n, 256), 256, 0, c->run>>>(a, buf, f, n);
+    else k_flatten<2><<<cdiv(n, 256), 256, 0, c->run>>>(a, buf, f, n);
+    LAUNCHCHK(c);
     HIPCHK(c, hipMemcpyAsync(x, buf, n * sizeof(double2), hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     return 0;
@@ -2320,10 +2311,7 @@ int fdga_fixed_point(fdga_ctx* c, double* R, const double* x, int32_t strategy, 
     if (!c || !R || !x) return -1;
     if (unflatten_into(c, x, update_sigma != 0, 1.0)) return -3;
     if (fdga_iterate(c, strategy, update_sigma, compute_hartree)) return -3;
-    if (flatten_from(c, R, update_sigma != 0)) return -3;
-    const size_t n = 2 * (size_t)(update_sigma ? fdga_flat_size(c) : fdga_flat_size_F(c));
-    for (size_t i = 0; i < n; ++i) R[i] -= x[i];
-    return 0;
+    return flatten_from(c, R, update_sigma != 0, nullptr, 1) ? -3 : 0;
 }
 
 int fdga_fixed_point_noalloc(fdga_ctx* c, double* R, const double* x, int32_t strategy, int32_t update_sigma,
@@ -2340,9 +2328,7 @@ int fdga_fixed_point_noalloc(fdga_ctx* c, double* R, const double* x, int32_t st
     // always the eager launches: capturing and instantiating a hipGraph allocates
     c->caches_mfrg = 0;
     if (fl_prepare(c) || iterate_eager(c, strategy, update_sigma, compute_hartree)) return -3;
-    if (flatten_from(c, R, update_sigma != 0, c->scratch)) return -3;
-    for (size_t i = 0; i < 2 * n; ++i) R[i] -= x[i];
-    return 0;
+    return flatten_from(c, R, update_sigma != 0, c->scratch, 1) ? -3 : 0;
 }
 
 int fdga_mfrg_apply(fdga_ctx* c, double* y, const double* x, int32_t strategy, int32_t is_first) {
@@ -2372,10 +2358,7 @@ int fdga_mfrg_apply(fdga_ctx* c, double* y, const double* x, int32_t strategy, i
     if (launch_lk3(c, all, 3)) return -3;
     if (launch_k3(c, all, 3, true)) return -3;
     if (fdga_update_F(c)) return -3;
-    if (flatten_from(c, y, false)) return -3;
-    const size_t n = 2 * (size_t)fdga_flat_size_F(c);
-    for (size_t i = 0; i < n; ++i) y[i] = x[i] - y[i] / factor;
-    return 0;
+    return flatten_from(c, y, false, nullptr, 2, factor) ? -3 : 0;   // y = x - G_lin(x / 100) * 100
 }
 
 int fdga_sync(fdga_ctx* c) {

@@ -3453,6 +3453,66 @@ __global__ void k_k3_to_ref(double2* __restrict__ out, const double2* __restrict
     size_t p = r / NV;
     out[e] = in[(size_t)i + (size_t)NV * ((size_t)j + (size_t)NV * ((size_t)iW + (size_t)NW * p))];
 }
+// The solver vector x = [γp(K1, K2, K3); γt; γa; Σ] between the reference layout and the device arrays in one
+// launch (K1, K2 and Σ have the same layout in both; K3 as k_k3_to_dev / k_k3_to_ref).  A launch per array was
+// ten launches with as many gaps each way (fixed-point evaluation of boxes 33, (16, 16), (8, 8): 236 -> 161 µs), and
+// the subtraction of x on the host cost 2.3 of 7.9 ms at 47 MB.
+struct FlatArgs {
+    double2* K1[3];
+    double2* K2[3];
+    double2* K3[3];   // FP32 values when k3f
+    double2* Sig;
+    size_t n1, n2, n3;   // elements of K1, K2, K3 (all momenta)
+    int NW, NV, k3f;
+};
+// array element of x's entry e: its channel, class (0 K1, 1 K2, 2 K3, 3 Σ) and device index
+__device__ __forceinline__ int flat_find(const FlatArgs& a, size_t e, int& r, size_t& i) {
+    const size_t per = a.n1 + a.n2 + a.n3;
+    r = e < per ? 0 : e < 2 * per ? 1 : e < 3 * per ? 2 : 3;
+    i = e - per * r;
+    if (r == 3) return 3;
+    if (i < a.n1) return 0;
+    i -= a.n1;
+    if (i < a.n2) return 1;
+    i -= a.n2;
+    // reference [Ω, ν, νp, P] -> device [ν, νp, Ω, P]
+    const size_t q = i / a.NW, iW = i - q * a.NW, nn = (size_t)a.NV * a.NV, p = q / nn;
+    i = (q - p * nn) + nn * (iW + (size_t)a.NW * p);
+    return 2;
+}
+__device__ __forceinline__ double2* flat_sel(double2* const* k, int r) { return r == 0 ? k[0] : r == 1 ? k[1] : k[2]; }
+// x -> arrays, the vertex part times scale
+__global__ __launch_bounds__(256) void k_unflatten(FlatArgs a, const double2* __restrict__ x, double scale, size_t n) {
+    const size_t e = blockIdx.x * (size_t)256 + threadIdx.x;
+    if (e >= n) return;
+    int r;
+    size_t i;
+    const int cls = flat_find(a, e, r, i);
+    const double2 v = x[e];
+    if (cls == 3) { a.Sig[i] = v; return; }
+    const double2 w = scale == 1.0 ? v : cscale(v, scale);
+    if (cls == 2 && a.k3f) reinterpret_cast<float2*>(flat_sel(a.K3, r))[i] = make_float2((float)w.x, (float)w.y);
+    else flat_sel(cls == 0 ? a.K1 : cls == 1 ? a.K2 : a.K3, r)[i] = w;
+}
+// arrays -> x (OP 0), the residual x = arrays - x of a fixed-point evaluation (OP 1), or the linear map's
+// x = x - arrays / f (OP 2), x holding the argument
+template <int OP>
+__global__ __launch_bounds__(256) void k_flatten(FlatArgs a, double2* __restrict__ x, double f, size_t n) {
+    const size_t e = blockIdx.x * (size_t)256 + threadIdx.x;
+    if (e >= n) return;
+    int r;
+    size_t i;
+    const int cls = flat_find(a, e, r, i);
+    double2 v;
+    if (cls == 3) v = a.Sig[i];
+    else if (cls == 2 && a.k3f) {
+        const float2 q = reinterpret_cast<const float2*>(flat_sel(a.K3, r))[i];
+        v = cmk(q.x, q.y);
+    } else v = flat_sel(cls == 0 ? a.K1 : cls == 1 ? a.K2 : a.K3, r)[i];
+    if (OP == 1) v = csub(v, x[e]);
+    if (OP == 2) { const double2 y = x[e]; v = cmk(y.x - v.x / f, y.y - v.y / f); }
+    x[e] = v;
+}
 // bubble: ref [Ω, ν, P] <-> dev [ν, Ω, P]
 __global__ void k_pi_to_dev(double2* __restrict__ out, const double2* __restrict__ in, int NW, int NV, int NP) {
     size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
