@@ -12,6 +12,7 @@
 #include <string>
 #include <future>
 #include <mutex>
+#include <numeric>
 #include <vector>
 
 #include "../../include/fdga.h"
@@ -19,6 +20,7 @@
 #include "fdga_adjoint.h"
 #include "fdga_bse3.h"
 #include "fdga_forms.h"
+#include "fdga_local.h"
 #include "fdga_sym.h"
 
 using namespace fdga;
@@ -96,6 +98,10 @@ struct fdga_ctx {
     size_t ntail = 0;                                               // elements of one tail-sum array
     double2* pchunk[2] = {nullptr, nullptr};   // lattice bubble: chunk sums of the last Πpp / Πph [P, chunk, Ω]
     int w_fresh = 0;                                                // Wc valid for the current iteration
+    double2* seg[6] = {};                                           // local solver: K2 of F (p, t, a) and F0 along diagonals
+    double2* wtot = nullptr;                                        // local solver: Σ_ω W per (Ω, channel)
+    int tot_fresh = 0;                                              // wtot valid for the current iteration
+    int seg_fresh = 0;                                              // seg valid for the current iteration
     // lattice BSE_K2! / BSE_L_K2! tables and GEMM result (s-wave solver only)
     double2 *k2x = nullptr, *k2xf = nullptr, *k2y = nullptr, *lk2x = nullptr;
     double2 *sde0 = nullptr;
@@ -589,6 +595,9 @@ int sde_hartree(fdga_ctx* c, double2* S, const double2* G, double sign) {
     return 0;
 }
 
+// a channel's classes for the segment kernels (without the diagonal copy of K2)
+SegCh seg_of(const ChanV& v) { return SegCh{v.K1, v.K2, v.K3, nullptr, v.n1, v.n2b, v.n2f, v.n3b, v.n3f}; }
+
 // Lpp/Lph of one level (lattice solver: plus a second Vertex level `lv2` of the same scale, summed
 // in the same pass); `zero` selects the reference system's groups SG0pp2/SG0ph2
 int sde_level_L(fdga_ctx* c, const Level& lv, const double2* Pp, const double2* Ph, bool zero,
@@ -652,15 +661,26 @@ int sde_level_L(fdga_ctx* c, const Level& lv, const double2* Pp, const double2* 
         if (sym_fill(c, c->Lpp, spp.ncls ? c->sg[idp].repop : nullptr, nout)) return -3;
         return sym_fill(c, c->Lph, sph.ncls ? c->sg[idh].repop : nullptr, nout);
     }
-    if (!spp.ncls && !sph.ncls) {
-        k_sde_L<<<cdiv(nout * WAVE, 256), 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, lv.g[0], lv.g[1], lv.g[2], ref,
-                                                           lv.kind, d.nK2b, d.nK2f, d.nK1, c->nVP, c->wb, c->NP,
-                                                           lv.chanNP, TU, NK, spp);
+    if (lv.kind == 0) {   // local solver, Vertex level
+        SegSde a{};
+        a.p = seg_of(lv.g[PCH]);
+        a.t = seg_of(lv.g[TCH]);
+        a.a = seg_of(lv.g[ACH]);
+        a.Pp = Pp; a.Ph = Ph; a.Tp = Tpp; a.Th = Tph;
+        a.Lpp = c->Lpp; a.Lph = c->Lph;
+        a.TU = TU;
+        a.n2b = d.nK2b; a.n2f = d.nK2f; a.nWP = d.nK1; a.nVP = c->nVP; a.wb = c->wb;
+        a.sp = spp; a.sh = sph;
+        a.npp = (int)nclass(spp, nout);
+        a.nph = (int)nclass(sph, nout);
+        k_seg_sde<<<cdiv((size_t)(a.npp + a.nph) * WAVE, 256), 256, 0, c->run>>>(a);
+    } else if (!spp.ncls && !sph.ncls) {
+        k_sde_L<<<cdiv(nout * WAVE, 256), 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, ref, d.nK2b, d.nK2f, d.nK1,
+                                                           c->nVP, c->wb, c->NP, TU, NK, spp);
     } else {
         const size_t nw = nclass(spp, nout) + nclass(sph, nout);
-        k_sde_L_pair<<<cdiv(nw * WAVE, 256), 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, lv.g[0], lv.g[1], lv.g[2], ref,
-                                                               lv.kind, d.nK2b, d.nK2f, d.nK1, c->nVP, c->wb, c->NP,
-                                                               lv.chanNP, TU, NK, spp, sph);
+        k_sde_L_pair<<<cdiv(nw * WAVE, 256), 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, ref, d.nK2b, d.nK2f, d.nK1,
+                                                               c->nVP, c->wb, c->NP, TU, NK, spp, sph);
     }
     LAUNCHCHK(c);
     return 0;
@@ -731,6 +751,94 @@ int idx_fbase(int ch) { return ch == PCH ? 7 : ch == ACH ? 8 : 9; }
 // classes of the channel's K2 (SGpp[2] = SGppL[2] for p, SGph[2] = SGphL[2] for a and t)
 static SymCls sym_k2(const fdga_ctx* c, int ch) { return symcls(c, ch == PCH ? SG_PP2 : SG_PH2); }
 
+static WTail wtail(fdga_ctx* c, int ch);
+static SegTot seg_tot_args(fdga_ctx* c) {
+    SegTot a{};
+    for (int ch = 0; ch < 3; ++ch) {
+        a.W[ch] = c->Wc[ch];
+        a.T[ch] = wtail(c, ch);
+    }
+    a.out = c->wtot;
+    a.n2b = c->d.nK2b; a.nWP = c->d.nK1; a.wb = c->wb;
+    return a;
+}
+// the local solver's K2 copies along diagonals (F, and F0 when it is a Vertex; once per iteration), and for the
+// channels in `left` (bit ch) the weights of BSE_L_K2! into Wc, in one launch
+static int launch_seg_prep(fdga_ctx* c, int left) {
+    const fdga_dims& d = c->d;
+    SegPrep a{};
+    unsigned blk = 0;
+    const bool copies = !c->seg_fresh;
+    const F0V f0 = f0_view(c);
+    if (copies)
+        for (int v = 0; v < (d.ref_kind == 1 ? 2 : 1); ++v)
+            for (int r = 0; r < 3; ++r) {
+                SegCh g = seg_of(v == 0 ? chanF(c, c->F[r]) : f0.g[r]);
+                g.S = c->seg[3 * v + r];
+                a.ch[a.nch] = g;
+                a.plus[a.nch] = r != PCH;
+                a.blk[a.nch++] = blk;
+                blk += cdiv((size_t)2 * g.n2f * g.rows(), 256);
+            }
+    a.wblk = blk;
+    a.wper = cdiv((size_t)2 * c->wb * c->NWP, 256);
+    int nw = 0;
+    for (int ch = 0; ch < 3; ++ch)
+        if (left >> ch & 1) {
+            a.W[nw] = c->Wc[ch];
+            a.Pi0[nw] = pi_of(c, ch, true);
+            a.wch[nw++] = ch;
+        }
+    a.f0 = f0;
+    a.nWP = d.nK1; a.nVP = c->nVP; a.wb = c->wb;
+    blk += nw * a.wper;
+    if (blk) k_seg_prep<<<blk, 256, 0, c->run>>>(a);
+    LAUNCHCHK(c);
+    return 0;
+}
+// BSE_K2! (LEFT: BSE_L_K2!) of the local solver for the channels in `chs` (bit ch)
+template <bool LEFT>
+static int launch_seg_k2(fdga_ctx* c, int chs) {
+    if (launch_seg_prep(c, LEFT ? chs : 0)) return -3;
+    const fdga_dims& d = c->d;
+    SegK2 a{};
+    const F0V f0 = f0_view(c);
+    SegCh* dst[2][3] = {{&a.F.p, &a.F.t, &a.F.a}, {&a.F0.p, &a.F0.t, &a.F0.a}};
+    for (int r = 0; r < 3; ++r) {
+        *dst[0][r] = seg_of(chanF(c, c->F[r]));
+        dst[0][r]->S = c->seg[r];
+        if (d.ref_kind == 1) {
+            *dst[1][r] = seg_of(f0.g[r]);
+            dst[1][r]->S = c->seg[3 + r];
+        }
+    }
+    a.ref = f0.ref;
+    a.Wp = c->Wc[PCH]; a.Wt = c->Wc[TCH]; a.Wa = c->Wc[ACH];
+    if (!LEFT) {
+        if (!c->tot_fresh) {
+            k_seg_tot<<<cdiv((size_t)3 * c->NW2 * WAVE, 256), 256, 0, c->run>>>(seg_tot_args(c));
+            LAUNCHCHK(c);
+        }
+        a.tot = c->wtot;
+        a.Lp = c->FL[PCH].K2; a.Lt = c->FL[TCH].K2; a.La = c->FL[ACH].K2;
+    }
+    DevChan* out = LEFT ? c->FL : c->Fb;
+    a.Kp = out[PCH].K2; a.Kt = out[TCH].K2; a.Ka = out[ACH].K2;
+    a.n2b = d.nK2b; a.n2f = d.nK2f; a.nWP = d.nK1; a.nVP = c->nVP; a.wb = c->wb;
+    a.T = d.T;
+    a.sp = symcls(c, SG_PP2);
+    a.sat = symcls(c, SG_PH2);
+    a.np = (chs >> PCH & 1) ? (int)nclass(a.sp, c->n2) : 0;
+    a.at = (chs >> ACH & 1) | (chs >> TCH & 1) << 1;
+    a.nat = a.at ? (int)nclass(a.sat, c->n2) : 0;
+    a.bat = (int)cdiv((size_t)a.nat * WAVE, 8 * SEG_NT);
+    const unsigned nb = 8 * (a.bat + cdiv((size_t)a.np * WAVE, 8 * SEG_NT));
+    if (!LEFT && d.ref_kind == 1) k_seg_k2<false, true><<<nb, SEG_NT, 0, c->run>>>(a);
+    else k_seg_k2<LEFT, false><<<nb, SEG_NT, 0, c->run>>>(a);
+    LAUNCHCHK(c);
+    return 0;
+}
+
 template <int CH>
 static int launch_lk2(fdga_ctx* c) {
     if (c->d.nonlocal) {
@@ -749,25 +857,13 @@ static int launch_lk2(fdga_ctx* c) {
         return sym_fill(c, c->FL[CH].K2, sym_k2(c, CH).ncls ? c->sg[CH == PCH ? SG_PP2 : SG_PH2].repop : nullptr,
                         c->n2 * c->NP);
     }
-    const SymCls sym = sym_k2(c, CH);
-    const size_t nw = nclass(sym, c->n2 * c->NP);
-    k_gemv_lk2<CH><<<cdiv(nw * WAVE, 256), 256, 0, c->run>>>(c->FL[CH].K2, c->FL[ACH].K2, pi_of(c, CH, true), vtx_F(c),
-                                                            c->d.nK2b, c->d.nK2f, c->d.nK1, c->nVP, c->NP,
-                                                            c->d.T * kSign[CH], box_bound(c), sym);
-    LAUNCHCHK(c);
-    return 0;
+    return launch_seg_k2<true>(c, 1 << CH);
 }
 
-// BSE_L_K2! of the p and a channels: one launch for the local solver
-static int launch_lk2_pa(fdga_ctx* c) {
-    if (c->d.nonlocal) return launch_lk2<PCH>(c) || launch_lk2<ACH>(c);
-    const SymCls sp = sym_k2(c, PCH), sa = sym_k2(c, ACH);
-    const size_t np = nclass(sp, c->n2 * c->NP), na = nclass(sa, c->n2 * c->NP);
-    k_gemv_lk2_pa<<<cdiv((np + na) * WAVE, 256), 256, 0, c->run>>>(
-        c->FL[PCH].K2, pi_of(c, PCH, true), sp, c->d.T * kSign[PCH], c->FL[ACH].K2, pi_of(c, ACH, true), sa,
-        c->d.T * kSign[ACH], vtx_F(c), c->d.nK2b, c->d.nK2f, c->d.nK1, c->nVP, c->NP, box_bound(c), (int)np);
-    LAUNCHCHK(c);
-    return 0;
+// BSE_L_K2! of the three channels: one launch for the local solver
+static int launch_lk2_all(fdga_ctx* c) {
+    if (c->d.nonlocal) return launch_lk2<PCH>(c) || launch_lk2<ACH>(c) || launch_lk2<TCH>(c);
+    return launch_seg_k2<true>(c, 7);
 }
 
 // the arrays of channel ch's weight: W on the band and its far sums from Π and Π0 and their tails
@@ -813,16 +909,15 @@ static int launch_k1(fdga_ctx* c) {
     return 0;
 }
 
-// BSE_K1! of the p and a channels in one launch (t separately: its post-processing reads the
-// finished a channel)
-static int launch_k1_pa(fdga_ctx* c) {
-    if (!c->w_fresh && (launch_w<PCH>(c) || launch_w<ACH>(c))) return -3;
+// BSE_K1! of the three channels in one launch; for the local solver with the weight totals of BSE_K2!
+static int launch_k1_all(fdga_ctx* c) {
+    if (!c->w_fresh && (launch_w<PCH>(c) || launch_w<ACH>(c) || launch_w<TCH>(c))) return -3;
     const SymCls sym = symcls(c, SG_K1);
     const int nw = (int)nclass(sym, c->n1 * c->NP);
-    k_gemv_k1_pa<<<(unsigned)(2 * nw), 256, 0, c->run>>>(c->Fb[PCH].K1, c->Wc[PCH], wtail(c, PCH), c->d.T * kSign[PCH],
-                                                          c->Fb[ACH].K1, c->Wc[ACH], wtail(c, ACH), c->d.T * kSign[ACH],
-                                                          vtx_F(c), c->d.nK1, c->d.nK1, c->nVP, c->wb, c->NP,
-                                                          box_bound(c), sym, nw);
+    const unsigned nt = c->d.nonlocal ? 0 : cdiv((size_t)3 * c->NW2 * WAVE, 256);
+    k_k1_all<<<(unsigned)(2 * nw) + nt, 256, 0, c->run>>>(
+        c->Fb[PCH].K1, c->Fb[ACH].K1, c->Fb[TCH].K1, c->Wc[PCH], c->Wc[ACH], c->Wc[TCH], wtail(c, PCH), wtail(c, ACH),
+        wtail(c, TCH), vtx_F(c), c->d.nK1, c->d.nK1, c->nVP, c->wb, c->NP, c->d.T, box_bound(c), sym, nw, seg_tot_args(c));
     LAUNCHCHK(c);
     return 0;
 }
@@ -872,42 +967,14 @@ template <int CH>
 static int launch_k2(fdga_ctx* c) {
     if (c->d.nonlocal) return launch_k2_nl<CH>(c);
     if (!c->w_fresh && launch_w<CH>(c)) return -3;
-    const SymCls sym = sym_k2(c, CH);
-    const size_t nw = nclass(sym, c->n2 * c->NP);
-    k_gemv_k2<CH><<<cdiv(nw * WAVE, 256), 256, 0, c->run>>>(c->Fb[CH].K2, c->Fb[ACH].K2, c->Wc[CH], wtail(c, CH), vtx_F(c),
-                                                           chanF(c, c->FL[CH]),
-                                                           chanF(c, c->FL[ACH]), c->d.nK2b, c->d.nK2f, c->d.nK1, c->nVP,
-                                                           c->wb, c->NP, c->d.T * kSign[CH], box_bound(c), sym);
-    LAUNCHCHK(c);
-    return 0;
-}
-
-// BSE_K2! of the a and t channels in one kernel (t needs the finished a channel)
-static int launch_k2_at(fdga_ctx* c) {
-    if (c->d.nonlocal) return launch_k2_nl<ACH>(c) || launch_k2_nl<TCH>(c);
-    if (!c->w_fresh && (launch_w<ACH>(c) || launch_w<TCH>(c))) return -3;
-    const SymCls sym = symcls(c, SG_PH2);   // a and t share SGph[2]
-    const size_t nw = nclass(sym, c->n2 * c->NP);
-    k_gemv_k2_at<<<cdiv(nw * WAVE, 256), 256, 0, c->run>>>(c->Fb[ACH].K2, c->Fb[TCH].K2, c->Wc[ACH], c->Wc[TCH],
-                                                          wtail(c, ACH), wtail(c, TCH), vtx_F(c),
-                                                          chanF(c, c->FL[ACH]), chanF(c, c->FL[TCH]), c->d.nK2b, c->d.nK2f,
-                                                          c->d.nK1, c->nVP, c->wb, c->NP, c->d.T, box_bound(c), sym);
-    LAUNCHCHK(c);
-    return 0;
+    return launch_seg_k2<false>(c, 1 << CH);
 }
 
 // BSE_K2! of the three channels: one launch for the local solver
 static int launch_k2_all(fdga_ctx* c) {
-    if (c->d.nonlocal) return launch_k2<PCH>(c) || launch_k2_at(c);
+    if (c->d.nonlocal) return launch_k2<PCH>(c) || launch_k2<ACH>(c) || launch_k2<TCH>(c);
     if (!c->w_fresh && (launch_w<PCH>(c) || launch_w<ACH>(c) || launch_w<TCH>(c))) return -3;
-    const SymCls sp = sym_k2(c, PCH), sat = symcls(c, SG_PH2);
-    const size_t np = nclass(sp, c->n2 * c->NP), nat = nclass(sat, c->n2 * c->NP);
-    k_gemv_k2_all<<<cdiv((np + nat) * WAVE, 256), 256, 0, c->run>>>(
-        c->Fb[PCH].K2, c->Wc[PCH], wtail(c, PCH), chanF(c, c->FL[PCH]), sp, (int)np, c->Fb[ACH].K2, c->Fb[TCH].K2,
-        c->Wc[ACH], c->Wc[TCH], wtail(c, ACH), wtail(c, TCH), vtx_F(c), chanF(c, c->FL[ACH]), chanF(c, c->FL[TCH]),
-        c->d.nK2b, c->d.nK2f, c->d.nK1, c->nVP, c->wb, c->NP, c->d.T, box_bound(c), sat);
-    LAUNCHCHK(c);
-    return 0;
+    return launch_seg_k2<false>(c, 7);
 }
 
 // classes of the channel's K3 (BSE_K3!: SGpp[3] / SGph[3]; BSE_L_K3!: SGppL[3] / SGphL[3]),
@@ -1513,6 +1580,14 @@ int fdga_create(fdga_ctx** out, const fdga_dims* dims) {
         rc |= dalloc(c, &c->k2y, (size_t)c->NV2 * c->NW2 * c->NP);
         rc |= dalloc(c, &c->lk2x, (size_t)c->NV2 * c->NV2 * c->NW2);
     }
+    if (!d.nonlocal) {
+        const size_t ns = (size_t)2 * d.nK2f * (2 * (d.nK2b + d.nK2f) - 2), nr = (size_t)2 * d.r_nK2f * (2 * (d.r_nK2b + d.r_nK2f) - 2);
+        for (int r = 0; r < 3; ++r) {
+            rc |= dalloc(c, &c->seg[r], ns);
+            if (d.ref_kind == 1) rc |= dalloc(c, &c->seg[3 + r], nr);
+        }
+        rc |= dalloc(c, &c->wtot, (size_t)3 * c->NW2);
+    }
     rc |= dalloc(c, &c->sde0, c->nGel);
     rc |= dalloc(c, &c->u2C, (size_t)(4 * d.nG - 1) * c->NkG);
     size_t ntab = (size_t)(2 * d.tab_nb - 1) * (2 * d.tab_nf) * (2 * d.tab_nf);
@@ -1563,6 +1638,8 @@ int fdga_destroy(fdga_ctx* c) {
                        c->k2x, c->k2xf, c->k2y, c->lk2x, c->pchunk[0], c->pchunk[1]})
         if (p) (void)hipFree(p);
     for (auto* t : c->tab) if (t) (void)hipFree(t);
+    for (auto* p : c->seg) if (p) (void)hipFree(p);
+    if (c->wtot) (void)hipFree(c->wtot);
     for (auto* p : c->cache) if (p) (void)hipFree(p);
     for (int r = 0; r < 3; ++r) {
         if (c->R[r]) (void)hipFree(c->R[r]);
@@ -1750,6 +1827,25 @@ int fdga_init(fdga_ctx* c) {
 }  // extern "C"
 
 namespace {
+// the local solver's K2 classes in the order of their representatives' Ω, then ν (the order in which the
+// segment kernels' waves share lines); the lattice solver's as they are
+fdga_sym::Classes by_omega(fdga_sym::Classes cl, const fdga_ctx* c) {
+    if (c->d.nonlocal) return cl;
+    std::vector<int> ord(cl.ncls());
+    std::iota(ord.begin(), ord.end(), 0);
+    auto key = [&](int k) {
+        const int rep = cl.mem[cl.off[k]] >> 2;
+        return std::pair<int, int>(rep % c->NW2, rep / c->NW2);
+    };
+    std::sort(ord.begin(), ord.end(), [&](int a, int b) { return key(a) < key(b); });
+    fdga_sym::Classes r;
+    r.off.push_back(0);
+    for (int k : ord) {
+        r.mem.insert(r.mem.end(), cl.mem.begin() + cl.off[k], cl.mem.begin() + cl.off[k + 1]);
+        r.off.push_back((int)r.mem.size());
+    }
+    return r;
+}
 // uploads a group's classes; with `n` > 0 also the per-element table (representative << 2) | op
 // over the n elements of the output
 int upload_sym(fdga_ctx* c, int id, const fdga_sym::Classes& cl, size_t n = 0) {
@@ -1813,8 +1909,8 @@ int fdga_init_sym_grp(fdga_ctx* c) {
         const int64_t iW = r % NW, iv = (r / NW) % NV, rest = r / (NW * NV), ivp = rest % NV, p = rest / NV;
         return iv + NV * (ivp + NV * (iW + NW * p));
     };
-    const Classes pp2 = build(m2, gens({G21, G2pp}));
-    const Classes ph2 = build(m2, gens({G21, G2ph}));
+    const Classes pp2 = by_omega(build(m2, gens({G21, G2pp})), c);
+    const Classes ph2 = by_omega(build(m2, gens({G21, G2ph})), c);
     // the lattice solver evaluates Σ, K2, L_K2 and the SDE L-vertices at every element and fills the
     // class members afterwards (per-element tables); K1 and the local gathers evaluate by class
     const size_t nS = nl ? c->nGel : 0, n2 = nl ? c->n2 * c->NP : 0;
@@ -2091,12 +2187,16 @@ static int iterate_two_chains(fdga_ctx* c, int32_t strategy, int32_t update_sigm
     int rc = 0;
     // chain B on st2
     c->run = c->st2;
-    if (strategy == FDGA_FDPA) rc = launch_lk2_pa(c) || fdga_bse_l_k2(c, TCH);
+    if (strategy == FDGA_FDPA) {
+        rc = launch_lk2_all(c);
+        c->seg_fresh = 1;
+    }
     rc = rc ? rc : launch_w_all(c);
     c->w_fresh = 1;
-    rc = rc ? rc : (launch_k1_pa(c) || fdga_bse_k1(c, TCH, 0));
+    rc = rc ? rc : launch_k1_all(c);
+    c->tot_fresh = 1;
     rc = rc ? rc : launch_k2_all(c);
-    c->w_fresh = 0;
+    c->w_fresh = c->seg_fresh = c->tot_fresh = 0;
     c->run = c->st;
     if (rc) return -3;
     // chain A on st
@@ -2210,7 +2310,7 @@ static int iterate_eager(fdga_ctx* c, int32_t strategy, int32_t update_sigma, in
     const bool fused = strategy == FDGA_FDPA && bse3_fused(c);   // both K3 equations in stage 6
     if (strategy == FDGA_FDPA) {
         stage_begin(c);
-        if (launch_lk2_pa(c) || fdga_bse_l_k2(c, TCH)) return -3;
+        if (launch_lk2_all(c)) return -3;
         stage_end(c, 2);
         stage_begin(c);
         const int all[3] = {PCH, ACH, TCH};
@@ -2221,11 +2321,12 @@ static int iterate_eager(fdga_ctx* c, int32_t strategy, int32_t update_sigma, in
     // the K1/K2 weights depend on Π, Π0, FL and F0 only: computed once for both stages
     if (launch_w_all(c)) return -3;
     c->w_fresh = 1;
-    int rc = launch_k1_pa(c) || fdga_bse_k1(c, TCH, 0);
+    int rc = launch_k1_all(c);
+    c->tot_fresh = 1;
     stage_end(c, 4);
     stage_begin(c);
     rc = rc ? rc : launch_k2_all(c);
-    c->w_fresh = 0;
+    c->w_fresh = c->tot_fresh = 0;
     if (rc) return -3;
     stage_end(c, 5);
     stage_begin(c);
@@ -2840,9 +2941,7 @@ int group_iterate_eager(fdga_group* g, int strategy, int update_sigma) {
     for (fdga_ctx* c : g->m) {
         if (update_sigma && (fdga_dyson(c) || fdga_bubbles(c))) return member_err(g, c);
         if (fdga_build_k3_cache(c)) return member_err(g, c);
-        if (fd)
-            for (int ch : {PCH, ACH, TCH})
-                if (fdga_bse_l_k2(c, ch)) return member_err(g, c);
+        if (fd && launch_lk2_all(c)) return member_err(g, c);
     }
     if (fd && gemms) {
         if (group_join(g) || group_gemm(g, 0, true) || group_fork(g)) return -3;
@@ -2853,10 +2952,11 @@ int group_iterate_eager(fdga_group* g, int strategy, int update_sigma) {
         fdga_ctx* c = g->m[j];
         if (launch_w_all(c)) return member_err(g, c);
         c->w_fresh = 1;
-        int rc = 0;
-        for (int ch : {PCH, ACH, TCH}) rc = rc ? rc : fdga_bse_k1(c, ch, 0);
+        c->seg_fresh = fd;
+        int rc = launch_k1_all(c);
+        c->tot_fresh = 1;
         rc = rc ? rc : launch_k2_all(c);
-        c->w_fresh = 0;
+        c->w_fresh = c->seg_fresh = c->tot_fresh = 0;
         if (rc) return member_err(g, c);
         if (fused[j]) {
             if (!g->timing && group_bse3(g, c)) return -3;

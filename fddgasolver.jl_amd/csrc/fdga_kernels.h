@@ -7,9 +7,10 @@
 //   s-wave averages        k_pavg_multi
 //   build_K3_cache!        k_cache               gather: Γ_irr / F0 / F-base caches
 //   BSE_L_K3!, BSE_K3!     zgemm_tiles<...>      batched complex GEMM on v_mfma_f64_16x16x4f64
-//   BSE_K1!, BSE_K2!,      k_bse_w + k_gemv_*    gather-GEMV over the bubble mesh
-//   BSE_L_K2!              (k_bse_w and k_tail_sums keep W and the far sums on the band the gathers read)
-//   SDE!                   k_sde_L, k_sde_sigma_local, k_u2_*, k_occupation
+//   BSE_K1!                k_bse_w + k_gemv_k1   gather-GEMV over the bubble mesh (k_bse_w and k_tail_sums keep W
+//                          and the far sums on the band the gathers read)
+//   BSE_K2!, BSE_L_K2!     local solver fdga_local.h; lattice k_k2nl_*, k_lk2nl_table and GEMMs
+//   SDE!                   k_seg_sde (fdga_local.h), k_sde_L_nl, k_sde_L, k_sde_sigma_*, k_u2_*, k_occupation
 #pragma once
 #include <type_traits>
 
@@ -2371,14 +2372,6 @@ __global__ __launch_bounds__(256) void k_gemv_k1(double2* __restrict__ K1, const
                                                  int n1, int nWP, int nVP, int wb, int NP, double scale, int NK, SymCls sym) {
     gemv_k1_block<CH>(blockIdx.x, K1, K1a, W, Wtail, F, n1, nWP, nVP, wb, NP, scale, NK, sym);
 }
-// the p and a channels in one launch (blocks [0, nb) p, the rest a); t needs the finished a channel
-__global__ __launch_bounds__(256) void k_gemv_k1_pa(double2* __restrict__ K1p, const double2* __restrict__ Wp,
-                                                    WTail Wtp, double scalep, double2* __restrict__ K1a_,
-                                                    const double2* __restrict__ Wa, WTail Wta, double scalea, VtxV F, int n1, int nWP, int nVP, int wb, int NP, int NK,
-                                                    SymCls sym, int nb) {
-    if ((int)blockIdx.x < nb) gemv_k1_block<PCH>(blockIdx.x, K1p, nullptr, Wp, Wtp, F, n1, nWP, nVP, wb, NP, scalep, NK, sym);
-    else gemv_k1_block<ACH>(blockIdx.x - nb, K1a_, nullptr, Wa, Wta, F, n1, nWP, nVP, wb, NP, scalea, NK, sym);
-}
 
 // BSE_K2!: K2(Ω, ν, P) = T s Σ_ω [F(Ω,ν,ω) - F(Ω,∞,ω)] W(ω) + FL.K2 (t: 2 FLt - FLa).
 // In the difference the channel's own K1(Ω) and K2(Ω, ω) cancel (the νInf evaluation keeps
@@ -2398,217 +2391,10 @@ __device__ __forceinline__ double2 k2x_psp(const VtxV& F, int m, int v, int w) {
     return x;
 }
 template <int CH>
-__device__ __forceinline__ double2 k2d_psp(const VtxV& F, int m, int v, int w, int p) {
-    double2 x = k2x_psp<CH>(F, m, v, w);
-    const ChanV& g = F.g[CH];
-    if (in_b(m, g.n3b) && in_f(v, g.n3f) && in_f(w, g.n3f)) x = cadd(x, g.k3(m, v, w, p));
-    return x;
-}
-// the ω-dependent summand in the channel's spin component (t: density, 2 F(t) - F(a))
-template <int CH>
-__device__ __forceinline__ double2 k2d_term(const VtxV& F, int m, int v, int w, int p) {
-    if (CH == TCH) return csub(cscale(k2d_psp<TCH>(F, m, v, w, p), 2.0), k2d_psp<ACH>(F, m, v, w, p));
-    return k2d_psp<CH>(F, m, v, w, p);
-}
-template <int CH>
 __device__ __forceinline__ double2 k2d_rank1(const VtxV& F, int m, int v, int p) {
     if (CH == TCH) return csub(cscale(F.g[TCH].k2(m, v, p), 2.0), F.g[ACH].k2(m, v, p));
     return F.g[CH].k2(m, v, p);
 }
-template <int CH>
-__device__ __forceinline__ void gemv_k2_wave(int wid, int lane, double2* __restrict__ K2, const double2* __restrict__ K2a,
-                                             const double2* __restrict__ W, const WTail& Wtail,
-                                             const VtxV& F, const ChanV& Lr, const ChanV& La, int n2b, int n2f, int nWP,
-                                             int nVP, int wb, int NP, double scale, int NK, const SymCls& sym) {
-    const int NW2 = 2 * n2b - 1, NV2 = 2 * n2f;
-    if (wid >= sym.count(NW2 * NV2 * NP)) return;
-    const int o0 = sym.rep(wid);
-    const int iW = o0 % NW2, iv = (o0 / NW2) % NV2, p = o0 / (NW2 * NV2);
-    const int m = iW - (n2b - 1), v = iv - n2f;
-    const int Wc = window(NK, m, v);
-    const size_t row = (size_t)(m + nWP - 1) + (size_t)(2 * nWP - 1) * p;
-    const double2* Wr = W + (size_t)(2 * wb) * row + wb;   // Wr[ω], |ω| within the band
-    // only the window is iterated for the summand; the far weights come from the tail sums
-    const int lo = max(0, nVP - Wc), hi = min(2 * nVP - 1, nVP + Wc);
-    double sr = 0.0, si = 0.0, mr = 0.0, mi = 0.0;
-    for (int iw = lo + lane; iw <= hi; iw += WAVE) {
-        const double2 wv = Wr[iw - nVP];
-        double2 x = cmul(k2d_term<CH>(F, m, v, iw - nVP, p), wv);
-        sr += x.x; si += x.y;
-        mr += wv.x; mi += wv.y;
-    }
-    double2 tl, tr;
-    far_pair(k2d_term<CH>(F, m, v, lane == 0 ? -Wc - 1 : Wc + 1, p), tl, tr);
-    sr = wave_sum(sr); si = wave_sum(si);
-    mr = wave_sum(mr); mi = wave_sum(mi);
-    const double2 wl = lo > 0 ? Wtail.left(row, nVP, wb, lo) : czero();
-    const double2 wr = hi < 2 * nVP - 1 ? Wtail.right(row, nVP, wb, hi) : czero();
-    double2 acc = cadd(cadd(cmk(sr, si), cmul(tl, wl)), cmul(tr, wr));
-    acc = cadd(acc, cmul(k2d_rank1<CH>(F, m, v, p), cadd(cmk(mr, mi), cadd(wl, wr))));
-    const double2 raw = cscale(acc, scale);
-    int b, e;
-    sym.range(wid, b, e);
-    for (int k = b + lane; k < e; k += WAVE) {
-        const int code = sym.member(wid, k), o = code >> 2;
-        double2 val = sym_apply(code & 3, raw);
-        if (CH == TCH) {
-            val = cadd(val, cscale(Lr.K2[o], 2.0));
-            val = cadd(val, cscale(La.K2[o], -1.0));
-            val = cscale(cadd(val, K2a[o]), 0.5);
-        } else {
-            val = cadd(val, Lr.K2[o]);
-        }
-        K2[o] = val;
-    }
-}
-template <int CH>
-__global__ __launch_bounds__(256) void k_gemv_k2(double2* __restrict__ K2, const double2* __restrict__ K2a,
-                                                 const double2* __restrict__ W, WTail Wtail, VtxV F,
-                                                 ChanV Lr, ChanV La, int n2b, int n2f, int nWP, int nVP, int wb, int NP,
-                                                 double scale, int NK, SymCls sym) {
-    gemv_k2_wave<CH>((blockIdx.x * blockDim.x + threadIdx.x) / WAVE, threadIdx.x & (WAVE - 1), K2, K2a, W, Wtail, F, Lr, La,
-                     n2b, n2f, nWP, nVP, wb, NP, scale, NK, sym);
-}
-
-// BSE_K2! of the a and t channels in one pass.  The t channel runs in the density component,
-// F(t, dSp) = 2 F(t, pSp) + F(t, xSp) = 2 F(t, pSp) - F(a, pSp) (src/vertex.jl:288-336), so the
-// a-channel evaluation is shared:  K2a = T Σ fa Wa + FL.a.K2,
-// K2t = (T (-1) Σ (2 ft - fa) Wt + 2 FL.t.K2 - FL.a.K2 + K2a) / 2   (src/BSE_templates.jl:95-110)
-__device__ __forceinline__ void gemv_k2_at_wave(int wid, int lane, double2* __restrict__ K2a, double2* __restrict__ K2t,
-                                                const double2* __restrict__ Wa, const double2* __restrict__ Wt,
-                                                const WTail& Wat, const WTail& Wtt,
-                                                const VtxV& F, const ChanV& La, const ChanV& Lt, int n2b, int n2f, int nWP,
-                                                int nVP, int wb, int NP, double T, int NK, const SymCls& sym) {
-    const int NW2 = 2 * n2b - 1, NV2 = 2 * n2f;
-    if (wid >= sym.count(NW2 * NV2 * NP)) return;
-    const int o0 = sym.rep(wid);
-    const int iW = o0 % NW2, iv = (o0 / NW2) % NV2, p = o0 / (NW2 * NV2);
-    const int m = iW - (n2b - 1), v = iv - n2f;
-    const int Wc = window(NK, m, v);
-    const size_t row = (size_t)(m + nWP - 1) + (size_t)(2 * nWP - 1) * p;
-    const size_t roff = (size_t)(2 * wb) * row + wb;   // band rows, indexed by ω
-    const double2* wa = Wa + roff;
-    const double2* wt = Wt + roff;
-    const int lo = max(0, nVP - Wc), hi = min(2 * nVP - 1, nVP + Wc);
-    double ar = 0.0, ai = 0.0, tr = 0.0, ti = 0.0;
-    double amr = 0.0, ami = 0.0, tmr = 0.0, tmi = 0.0;
-    for (int iw = lo + lane; iw <= hi; iw += WAVE) {
-        const int w = iw - nVP;
-        const double2 fa = k2d_psp<ACH>(F, m, v, w, p);
-        const double2 ft = k2d_psp<TCH>(F, m, v, w, p);
-        const double2 wav = wa[w], wtv = wt[w];
-        const double2 xa = cmul(fa, wav);
-        const double2 xt = cmul(csub(cscale(ft, 2.0), fa), wtv);
-        ar += xa.x; ai += xa.y; tr += xt.x; ti += xt.y;
-        amr += wav.x; ami += wav.y; tmr += wtv.x; tmi += wtv.y;
-    }
-    // far summands: lane 0 at ω = -Wc-1, lane 1 at ω = Wc+1
-    const int wf = lane == 0 ? -Wc - 1 : Wc + 1;
-    const double2 fa = k2d_psp<ACH>(F, m, v, wf, p);
-    const double2 ft = k2d_psp<TCH>(F, m, v, wf, p);
-    double2 fal, far_, fdl, fdr;
-    far_pair(fa, fal, far_);
-    far_pair(csub(cscale(ft, 2.0), fa), fdl, fdr);
-    ar = wave_sum(ar); ai = wave_sum(ai); tr = wave_sum(tr); ti = wave_sum(ti);
-    amr = wave_sum(amr); ami = wave_sum(ami); tmr = wave_sum(tmr); tmi = wave_sum(tmi);
-    const bool hl = lo > 0, hr = hi < 2 * nVP - 1;
-    const double2 awl = hl ? Wat.left(row, nVP, wb, lo) : czero();
-    const double2 awr = hr ? Wat.right(row, nVP, wb, hi) : czero();
-    const double2 twl = hl ? Wtt.left(row, nVP, wb, lo) : czero();
-    const double2 twr = hr ? Wtt.right(row, nVP, wb, hi) : czero();
-    double2 A = cadd(cadd(cmk(ar, ai), cmul(fal, awl)), cmul(far_, awr));
-    double2 D = cadd(cadd(cmk(tr, ti), cmul(fdl, twl)), cmul(fdr, twr));
-    A = cadd(A, cmul(k2d_rank1<ACH>(F, m, v, p), cadd(cmk(amr, ami), cadd(awl, awr))));
-    D = cadd(D, cmul(k2d_rank1<TCH>(F, m, v, p), cadd(cmk(tmr, tmi), cadd(twl, twr))));
-    const double2 rawa = cscale(A, T), rawt = cscale(D, -T);
-    int b, e;
-    sym.range(wid, b, e);
-    for (int k = b + lane; k < e; k += WAVE) {
-        const int code = sym.member(wid, k), o = code >> 2;
-        const double2 ka = cadd(sym_apply(code & 3, rawa), La.K2[o]);
-        double2 kt = sym_apply(code & 3, rawt);
-        kt = cadd(kt, cscale(Lt.K2[o], 2.0));
-        kt = cadd(kt, cscale(La.K2[o], -1.0));
-        K2a[o] = ka;
-        K2t[o] = cscale(cadd(kt, ka), 0.5);
-    }
-}
-// BSE_K2! of all three channels in one launch: waves [0, wp) the p classes (SGpp[2]), then the a and
-// t classes (SGph[2], t finished from a in the same wave)
-__global__ __launch_bounds__(256, 4) void k_gemv_k2_all(double2* __restrict__ K2p, const double2* __restrict__ Wp,
-                                                     WTail Wtp, ChanV Lp, SymCls symp, int wp,
-                                                     double2* __restrict__ K2a, double2* __restrict__ K2t,
-                                                     const double2* __restrict__ Wa, const double2* __restrict__ Wt,
-                                                     WTail Wat, WTail Wtt,
-                                                     VtxV F, ChanV La, ChanV Lt, int n2b, int n2f, int nWP, int nVP, int wb,
-                                                     int NP, double T, int NK, SymCls symat) {
-    const int wid = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
-    if (wid < wp)
-        gemv_k2_wave<PCH>(wid, lane, K2p, nullptr, Wp, Wtp, F, Lp, La, n2b, n2f, nWP, nVP, wb, NP, T, NK, symp);
-    else
-        gemv_k2_at_wave(wid - wp, lane, K2a, K2t, Wa, Wt, Wat, Wtt, F, La, Lt, n2b, n2f, nWP, nVP, wb, NP, T, NK, symat);
-}
-__global__ __launch_bounds__(256, 4) void k_gemv_k2_at(double2* __restrict__ K2a, double2* __restrict__ K2t,
-                                                    const double2* __restrict__ Wa, const double2* __restrict__ Wt,
-                                                    WTail Wat, WTail Wtt,
-                                                    VtxV F, ChanV La, ChanV Lt, int n2b, int n2f, int nWP, int nVP,
-                                                    int wb, int NP, double T, int NK, SymCls sym) {
-    gemv_k2_at_wave((blockIdx.x * blockDim.x + threadIdx.x) / WAVE, threadIdx.x & (WAVE - 1), K2a, K2t, Wa, Wt, Wat, Wtt, F,
-                    La, Lt, n2b, n2f, nWP, nVP, wb, NP, T, NK, sym);
-}
-
-// BSE_L_K2! of the local solver (src/BSEa/BSEa_K2.jl:1-40): Σ over the bubble mesh of
-//   Γ(Ω, ν, ω) Π0(ω) F0(Ω, ω~, ∞).  Γ excludes F0 and the own channel, so it vanishes outside
-//   the frequency window.  (The lattice solver's form is k_lk2nl_table + GEMM.)
-template <int CH>
-__device__ __forceinline__ void gemv_lk2_wave(int wid, int lane, double2* __restrict__ out, const double2* __restrict__ outa,
-                                              const double2* __restrict__ Pi0, const VtxV& F, int n2b, int n2f, int nWP,
-                                              int nVP, int NP, double scale, int NK, const SymCls& sym) {
-    constexpr int SP = ChSpin<CH>::SP;
-    constexpr int FLG = FL_ALL & ~FL_F0 & ~(FL_GP << CH);
-    const int NW2 = 2 * n2b - 1, NV2 = 2 * n2f;
-    if (wid >= sym.count(NW2 * NV2 * NP)) return;
-    const int o0 = sym.rep(wid);
-    const int iW = o0 % NW2, iv = (o0 / NW2) % NV2, p = o0 / (NW2 * NV2);
-    const int m = iW - (n2b - 1), v = iv - n2f;
-    const double2* P0 = Pi0 + (size_t)(2 * nVP) * ((size_t)(m + nWP - 1) + (size_t)(2 * nWP - 1) * p);
-    double sr = 0.0, si = 0.0;
-    const int Wc = window(NK, m, v);
-    const int lo = max(0, nVP - Wc), hi = min(2 * nVP - 1, nVP + Wc);
-    for (int q = lo + lane; q <= hi; q += WAVE) {
-        const int w = q - nVP;
-        double2 x = cmul(cmul(F.eval(m, v, w, p, CH, SP, FLG), P0[q]), F.f0.eval(m, crossing(m, w, CH), FDGA_INF, CH, SP));
-        sr += x.x; si += x.y;
-    }
-    sr = wave_sum(sr);
-    si = wave_sum(si);
-    const double2 raw = cscale(cmk(sr, si), scale);
-    int b, e;
-    sym.range(wid, b, e);
-    for (int k = b + lane; k < e; k += WAVE) {
-        const int code = sym.member(wid, k), o = code >> 2;
-        double2 val = sym_apply(code & 3, raw);
-        if (CH == TCH) val = cscale(cadd(val, outa[o]), 0.5);
-        out[o] = val;
-    }
-}
-template <int CH>
-__global__ __launch_bounds__(256) void k_gemv_lk2(double2* __restrict__ out, const double2* __restrict__ outa,
-                                                  const double2* __restrict__ Pi0, VtxV F, int n2b, int n2f, int nWP,
-                                                  int nVP, int NP, double scale, int NK, SymCls sym) {
-    gemv_lk2_wave<CH>((blockIdx.x * blockDim.x + threadIdx.x) / WAVE, threadIdx.x & (WAVE - 1), out, outa, Pi0, F, n2b, n2f,
-                      nWP, nVP, NP, scale, NK, sym);
-}
-// the p and a channels in one launch (waves [0, wp) p, the rest a); t needs the finished a channel
-__global__ __launch_bounds__(256) void k_gemv_lk2_pa(double2* __restrict__ outp, const double2* __restrict__ Pi0p,
-                                                     SymCls symp, double scalep, double2* __restrict__ outa_,
-                                                     const double2* __restrict__ Pi0a, SymCls syma, double scalea, VtxV F,
-                                                     int n2b, int n2f, int nWP, int nVP, int NP, int NK, int wp) {
-    const int wid = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
-    if (wid < wp) gemv_lk2_wave<PCH>(wid, lane, outp, nullptr, Pi0p, F, n2b, n2f, nWP, nVP, NP, scalep, NK, symp);
-    else gemv_lk2_wave<ACH>(wid - wp, lane, outa_, nullptr, Pi0a, F, n2b, n2f, nWP, nVP, NP, scalea, NK, syma);
-}
-
 // ---------------------------------------------------------------------------------------
 // BSE_K2! and BSE_L_K2! of the s-wave lattice solver as tables and GEMMs.  In the s-wave vertex
 // the cross channels are P-averaged and F0 is local, so the ω-dependent part of the BSE_K2!
@@ -2776,20 +2562,14 @@ __global__ void k_k2nl_symfinish(double2* __restrict__ K2, const double2* __rest
 }
 
 // ---------------------------------------------------------------------------------------
-// SDE_channel_L_pp! / _ph! (src/SDE.jl:79-217; NL src/nonlocal/SDE.jl:3-142).
-// kind 0: Vertex channels g (momentum p if NP > 1); kind 1: RefVertex tables.
+// SDE_channel_L_pp! / _ph! (src/SDE.jl:79-217; NL src/nonlocal/SDE.jl:3-142) at the RefVertex level (its
+// tables; the Vertex levels: k_seg_sde, k_sde_L_nl).
 template <bool DP, bool DH>
-__device__ __forceinline__ void sde_terms(const ChanV& gp, const ChanV& gt, const ChanV& ga, const RefV& ref, int kind,
-                                 int m, int v, int w, int pc, double2& xp, double2& xh) {
+__device__ __forceinline__ void sde_terms(const RefV& ref, int m, int v, int w, double2& xp, double2& xh) {
     xp = czero();
     xh = czero();
-    if (kind == 0) {
-        if (DP) xp = gp.eval(m, bmf(m, w), v, pc);
-        if (DH) xh = cadd(ga.eval(m, v, w, pc), gt.eval(m, v, w, pc));
-    } else {
-        if (DP) xp = csub(ref.eval(m, bmf(m, w), v, PCH, PSP), ref.bare(PSP));
-        if (DH) xh = csub(csub(cadd(ref.eval(m, v, w, ACH, PSP), ref.eval(m, v, w, TCH, PSP)), ref.bare(PSP)), ref.bare(PSP));
-    }
+    if (DP) xp = csub(ref.eval(m, bmf(m, w), v, PCH, PSP), ref.bare(PSP));
+    if (DH) xh = csub(csub(cadd(ref.eval(m, v, w, ACH, PSP), ref.eval(m, v, w, TCH, PSP)), ref.bare(PSP)), ref.bare(PSP));
 }
 // WHICH: bit 0 computes Lpp, bit 1 Lph.  Under a symmetry group the two outputs have their own
 // classes (SGpp2, SGph2): one wave per class of either (k_sde_L_pair).
@@ -2797,8 +2577,7 @@ template <int WHICH>
 __device__ __forceinline__ void sde_L_wave(int wid, int lane, double2* __restrict__ Lpp, double2* __restrict__ Lph,
                                            const double2* __restrict__ Pipp, const double2* __restrict__ Piph,
                                            const double2* __restrict__ Tpp, const double2* __restrict__ Tph,
-                                           const ChanV& gp, const ChanV& gt, const ChanV& ga, const RefV& ref, int kind,
-                                           int n2b, int n2f, int nWP, int nVP, int wb, int NP, int chanNP, double2 TU,
+                                           const RefV& ref, int n2b, int n2f, int nWP, int nVP, int wb, int NP, double2 TU,
                                            int NK, const SymCls& sym) {
     constexpr bool DP = WHICH & 1, DH = WHICH & 2;
     const int NW2 = 2 * n2b - 1, NV2 = 2 * n2f;
@@ -2806,7 +2585,6 @@ __device__ __forceinline__ void sde_L_wave(int wid, int lane, double2* __restric
     const int o0 = sym.rep(wid);
     const int iW = o0 % NW2, iv = (o0 / NW2) % NV2, p = o0 / (NW2 * NV2);
     const int m = iW - (n2b - 1), v = iv - n2f;
-    const int pc = chanNP > 1 ? p : 0;
     const int Wc = window(NK, m, v);
     const int lo = max(0, nVP - Wc), hi = min(2 * nVP - 1, nVP + Wc);
     const size_t row = (size_t)(m + nWP - 1) + (size_t)(2 * nWP - 1) * p;
@@ -2814,12 +2592,12 @@ __device__ __forceinline__ void sde_L_wave(int wid, int lane, double2* __restric
     double ar = 0.0, ai = 0.0, br = 0.0, bi = 0.0;
     for (int iw = lo + lane; iw <= hi; iw += WAVE) {
         double2 xp, xh;
-        sde_terms<DP, DH>(gp, gt, ga, ref, kind, m, v, iw - nVP, pc, xp, xh);
+        sde_terms<DP, DH>(ref, m, v, iw - nVP, xp, xh);
         if (DP) { double2 a = cmul(Pipp[base + iw], xp); ar += a.x; ai += a.y; }
         if (DH) { double2 b = cmul(Piph[base + iw], xh); br += b.x; bi += b.y; }
     }
     double2 fxp, fxh, xpl, xpr, xhl, xhr;
-    sde_terms<DP, DH>(gp, gt, ga, ref, kind, m, v, lane == 0 ? -Wc - 1 : Wc + 1, pc, fxp, fxh);
+    sde_terms<DP, DH>(ref, m, v, lane == 0 ? -Wc - 1 : Wc + 1, fxp, fxh);
     far_pair(fxp, xpl, xpr);
     far_pair(fxh, xhl, xhr);
     ar = wave_sum(ar); ai = wave_sum(ai); br = wave_sum(br); bi = wave_sum(bi);
@@ -2844,26 +2622,21 @@ __device__ __forceinline__ void sde_L_wave(int wid, int lane, double2* __restric
 // both outputs per element (no symmetry groups)
 __global__ __launch_bounds__(256) void k_sde_L(double2* __restrict__ Lpp, double2* __restrict__ Lph, const double2* __restrict__ Pipp,
                         const double2* __restrict__ Piph, const double2* __restrict__ Tpp, const double2* __restrict__ Tph,
-                        ChanV gp, ChanV gt, ChanV ga, RefV ref, int kind,
-                        int n2b, int n2f, int nWP, int nVP, int wb, int NP, int chanNP, double2 TU, int NK, SymCls sym) {
+                        RefV ref, int n2b, int n2f, int nWP, int nVP, int wb, int NP, double2 TU, int NK, SymCls sym) {
     const int wid = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
-    sde_L_wave<3>(wid, lane, Lpp, Lph, Pipp, Piph, Tpp, Tph, gp, gt, ga, ref, kind, n2b, n2f, nWP, nVP, wb, NP, chanNP, TU,
-                  NK, sym);
+    sde_L_wave<3>(wid, lane, Lpp, Lph, Pipp, Piph, Tpp, Tph, ref, n2b, n2f, nWP, nVP, wb, NP, TU, NK, sym);
 }
 // the classes of SGpp2 (waves [0, ncls_pp)) and of SGph2 (the waves after them) in one launch
 __global__ __launch_bounds__(256) void k_sde_L_pair(double2* __restrict__ Lpp, double2* __restrict__ Lph,
                         const double2* __restrict__ Pipp, const double2* __restrict__ Piph, const double2* __restrict__ Tpp,
-                        const double2* __restrict__ Tph, ChanV gp, ChanV gt, ChanV ga, RefV ref, int kind,
-                        int n2b, int n2f, int nWP, int nVP, int wb, int NP, int chanNP, double2 TU, int NK, SymCls spp,
-                        SymCls sph) {
+                        const double2* __restrict__ Tph, RefV ref, int n2b, int n2f, int nWP, int nVP, int wb, int NP,
+                        double2 TU, int NK, SymCls spp, SymCls sph) {
     const int wid = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
     const int npp = spp.count((2 * n2b - 1) * (2 * n2f) * NP);
     if (wid < npp)
-        sde_L_wave<1>(wid, lane, Lpp, Lph, Pipp, Piph, Tpp, Tph, gp, gt, ga, ref, kind, n2b, n2f, nWP, nVP, wb, NP, chanNP,
-                      TU, NK, spp);
+        sde_L_wave<1>(wid, lane, Lpp, Lph, Pipp, Piph, Tpp, Tph, ref, n2b, n2f, nWP, nVP, wb, NP, TU, NK, spp);
     else
-        sde_L_wave<2>(wid - npp, lane, Lpp, Lph, Pipp, Piph, Tpp, Tph, gp, gt, ga, ref, kind, n2b, n2f, nWP, nVP, wb, NP,
-                      chanNP, TU, NK, sph);
+        sde_L_wave<2>(wid - npp, lane, Lpp, Lph, Pipp, Piph, Tpp, Tph, ref, n2b, n2f, nWP, nVP, wb, NP, TU, NK, sph);
 }
 
 // SDE L-vertices of the s-wave lattice solver at a Vertex level (kind 0), one wave per (Ω, P).
