@@ -611,31 +611,16 @@ int sde_level_L(fdga_ctx* c, const Level& lv, const double2* Pp, const double2* 
     const int NK = sde_box_bound(c);
     const double2* Tpp = pi_tail(c, Pp);
     const double2* Tph = pi_tail(c, Ph);
-    if (d.nonlocal && lv.kind == 0) {   // lattice solver, Vertex level: one wave per (Ω, P)
-        const unsigned nb = (unsigned)cdiv((size_t)c->NW2 * c->NP * WAVE, 256);
-        const SdeLevelNL l0{lv.g[0], lv.g[1], lv.g[2], lv.chanNP};
+    if (d.nonlocal && lv.kind == 0) {   // lattice solver, Vertex level: one block per (Ω, P)
+        const unsigned nb = (unsigned)(c->NW2 * c->NP);
+        const SdeLevelNL l0{lv.g[0], lv.g[1], lv.g[2], lv.chanNP, 1};
         if (lv2) {
-            const SdeLevelNL l1{lv2->g[0], lv2->g[1], lv2->g[2], lv2->chanNP};
             // a momentum-independent second level (the local reference vertex): its K3 terms as GEMMs
             // over the momenta after the pass
             const bool refgemm = lv2->chanNP == 1 && c->NP > 1;
-            // (the target level's K3 form fixed at compile time: one load form in the loops)
-            // (with it fixed, the target level's a/t K3 sum runs in k_sde_h3 after the pass)
-            if (refgemm && l0.gp.k3f && l0.ga.k3f && l0.gt.k3f) {
-                k_sde_L_nl<2, true, 1><<<nb, 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, l0, l1, d.nK2b, d.nK2f,
-                                                               d.nK1, c->nVP, c->wb, c->NP, TU);
-                k_sde_h3<true><<<nb, 256, 0, c->run>>>(c->Lph, Ph, l0.ga, l0.gt, d.nK2b, d.nK2f, d.nK1, c->nVP, c->NP, TU);
-            } else if (refgemm && !l0.gp.k3f && !l0.ga.k3f && !l0.gt.k3f) {
-                k_sde_L_nl<2, true, 0><<<nb, 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, l0, l1, d.nK2b, d.nK2f,
-                                                               d.nK1, c->nVP, c->wb, c->NP, TU);
-                k_sde_h3<false><<<nb, 256, 0, c->run>>>(c->Lph, Ph, l0.ga, l0.gt, d.nK2b, d.nK2f, d.nK1, c->nVP, c->NP, TU);
-            } else if (refgemm) {   // (the reference level's K3 terms still in the GEMMs below)
-                k_sde_L_nl<2, true><<<nb, 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, l0, l1, d.nK2b, d.nK2f,
-                                                            d.nK1, c->nVP, c->wb, c->NP, TU);
-            } else {
-                k_sde_L_nl<2><<<nb, 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, l0, l1, d.nK2b, d.nK2f, d.nK1,
-                                                      c->nVP, c->wb, c->NP, TU);
-            }
+            const SdeLevelNL l1{lv2->g[0], lv2->g[1], lv2->g[2], lv2->chanNP, !refgemm};
+            k_sde_L_nl<2><<<nb, 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, l0, l1, d.nK2b, d.nK2f, d.nK1, c->nVP,
+                                                  c->wb, c->NP, TU);
             LAUNCHCHK(c);
             if (refgemm) {
                 const ChanV& gp = lv2->g[PCH];

@@ -2652,61 +2652,14 @@ struct ChanBox {
     int pc;
     __device__ double2 k1(int m) const { return in_b(m, g.n1) ? g.k1(m, pc) : czero(); }
     __device__ double2 k2(int m, int n) const { return in_b(m, g.n2b) && in_f(n, g.n2f) ? g.k2(m, n, pc) : czero(); }
-    __device__ double2 k3(int m, int n, int np) const {
-        return in_b(m, g.n3b) && in_f(n, g.n3f) && in_f(np, g.n3f) ? g.k3(m, n, np, pc) : czero();
-    }
-    template <bool K32>
-    __device__ double2 k3p(int m, int n, int np) const {   // (pc >= 0)
-        return in_b(m, g.n3b) && in_f(n, g.n3f) && in_f(np, g.n3f) ? g.template k3p<K32>(m, n, np, pc) : czero();
-    }
 };
 // the channels of one Vertex level of the lattice SDE: at momentum P (chanNP > 1) or the local
 // vertex (chanNP = 1)
 struct SdeLevelNL {
     ChanV gp, gt, ga;
     int chanNP;
+    int k3;   // with its K3 terms
 };
-__device__ __forceinline__ double2 shfl_xor2(double2 v, int mask) {
-    return cmk(__shfl_xor(v.x, mask, WAVE), __shfl_xor(v.y, mask, WAVE));
-}
-// The p-channel K3 sum of the lattice SDE for every ν of the level's K3 box (2 n3f <= 64):
-//   S(ν) = Σ_n K3p(Ω, n, ν) Πpp(Ω - n - 1)   (n in the box, Ω - n - 1 on the bubble mesh)
-// with the lanes over n, so that each load reads a contiguous column of K3 (its first index), and the
-// products of four ν at a time reduced across the wave by recursive halving (lanes exchange half
-// their partial sums at distances 32 and 16, then sum at 8, 4, 2 and 1).  Returns S(ν) at the lane
-// iv = ν + n2f (ν = iv - n2f outside the box: zero).
-template <bool K32>
-__device__ __forceinline__ double2 sde_p3_lanes(const ChanV& g, int pc, int m, const double2* pp, int nVP, int n2f,
-                                                int lane) {
-    const int n3 = g.n3f, NV = 2 * n3;
-    const int n = lane - n3, wp = m - n - 1;
-    const bool ln = lane < NV && wp >= -nVP && wp < nVP;
-    const double2 w = ln ? pp[wp] : czero();
-    const bool h5 = lane & 32, h4 = lane & 16;
-    const int vme = lane - n2f + n3;   // this lane's ν, as an index into the box
-    double2 mine = czero();
-    for (int c0 = 0; c0 < NV; c0 += 4) {
-        double2 x[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            x[j] = (ln && c0 + j < NV) ? cmul(g.template k3p<K32>(m, n, c0 + j - n3, pc), w) : czero();
-        double2 y[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) y[k] = cadd(h5 ? x[2 + k] : x[k], shfl_xor2(h5 ? x[k] : x[2 + k], 32));
-        double2 u = cadd(h4 ? y[1] : y[0], shfl_xor2(h4 ? y[0] : y[1], 16));
-        u = cadd(u, shfl_xor2(u, 8));
-        u = cadd(u, shfl_xor2(u, 4));
-        u = cadd(u, shfl_xor2(u, 2));
-        u = cadd(u, shfl_xor2(u, 1));
-        // u is S(ν) of box index c0 + ((lane >> 5) & 1) * 2 + ((lane >> 4) & 1)
-        const int jv = (vme - c0) & 3;
-        const int src = ((jv >> 1) & 1) << 5 | (jv & 1) << 4;
-        const double2 s = cmk(__shfl(u.x, src, WAVE), __shfl(u.y, src, WAVE));
-        if (vme >= c0 && vme < c0 + 4) mine = s;
-    }
-    return mine;
-}
-
 // The K3 terms of a momentum-independent Vertex level (the local reference vertex) in the lattice SDE
 // L-vertices, as FP64 GEMMs per Ω of its K3 box over all momenta at once (n, ν in that box, the Π
 // rows of (Ω, P)):
@@ -2753,75 +2706,139 @@ struct SdeRefE {   // L(Ω, ν, P) += T U C(ν, P) inside the L box
     }
 };
 
-// NLEV Vertex levels summed into one pair of L-vertices (the target vertex and the local reference
-// vertex of the fdPA iteration share ΣΠ, the bubble rows and the launch).  SKIP1: the second level's
-// K3 terms are left out (added by the momentum GEMMs SdeRef*, when that level is momentum-independent).
-// F0: the first level's K3 form fixed at compile time (0 FP64, 1 FP32; -1: read from the level); with
-// a fixed form the first level's a/t K3 sum is left to k_sde_h3 (a lean kernel of its own)
-template <int NLEV, bool SKIP1 = false, int F0 = -1>
+// K3 elements of one 16-byte load: one FP64 value or two FP32 neighbours along ν
+template <bool K32>
+struct SdePack {
+    static constexpr int n = K32 ? 2 : 1;
+    double2 x[n];
+    __device__ __forceinline__ SdePack(const double2* p) {
+        if constexpr (K32) {
+            const float4 v = *reinterpret_cast<const float4*>(p);
+            x[0] = cmk(v.x, v.y);
+            x[1] = cmk(v.z, v.w);
+        } else {
+            x[0] = *p;
+        }
+    }
+};
+// one lattice (Ω, P) slab of K3, in units of 16 bytes (an even number of FP32 values a column)
+template <bool K32>
+__device__ __forceinline__ const double2* sde_slab(const ChanV& g, int m, int pc) {
+    const size_t N = 2 * (size_t)g.n3f, o = N * N * ((size_t)(m + g.n3b - 1) + (size_t)(2 * g.n3b - 1) * pc);
+    return g.K3 + (K32 ? o / 2 : o);
+}
+constexpr int SDE_W = 512;   // weights staged at a time
+// add(ν index, Σ_n K3p(n, ν) w(n)) for every ν of the box, by 8 lanes a column: a load reads 128 contiguous bytes
+template <bool K32, class W, class ADD>
+__device__ __forceinline__ void sde_k3_cols(const double2* K, int N, double2* wsm, int tid, W&& w, ADD&& add) {
+    constexpr int E = SdePack<K32>::n;
+    const int G = N / E, s = tid & 7;
+    for (int n0 = 0; n0 < N; n0 += SDE_W) {
+        const int nc = min(SDE_W, N - n0);
+        __syncthreads();
+        for (int n = tid; n < nc; n += 256) wsm[n] = w(n0 + n);
+        __syncthreads();
+        for (int j = tid >> 3; j < N; j += 32) {
+            const double2* col = K + (size_t)G * j + n0 / E;
+            double2 a = czero();
+#pragma unroll 4
+            for (int r = s; r < nc / E; r += 8) {
+                const SdePack<K32> v(col + r);
+#pragma unroll
+                for (int q = 0; q < E; ++q) a = cadd(a, cmul(v.x[q], wsm[E * r + q]));
+            }
+#pragma unroll
+            for (int d = 4; d; d >>= 1) a = cadd(a, cmk(__shfl_xor(a.x, d, 8), __shfl_xor(a.y, d, 8)));
+            if (s == 0) add(j, a);
+        }
+    }
+}
+// add(ν index, Σ_n [A + B](ν, n) w(n)) for every ν of the box: threads over the packs of a column and over
+// columns, so that a load of the block reads contiguous memory; the column groups' sums meet in LDS
+template <bool K32, class W, class ADD>
+__device__ __forceinline__ void sde_k3_rows(const double2* A, const double2* B, int N, double2* wsm, double2* red, int tid,
+                                            W&& w, ADD&& add) {
+    constexpr int E = SdePack<K32>::n;
+    const int G = N / E, Gc = min(G, 256), ncg = 256 / Gc, r = tid % Gc, cg = tid / Gc;
+    for (int n0 = 0; n0 < N; n0 += SDE_W) {
+        const int nc = min(SDE_W, N - n0);
+        __syncthreads();
+        for (int n = tid; n < nc; n += 256) wsm[n] = w(n0 + n);
+        __syncthreads();
+        for (int r0 = 0; r0 < G; r0 += Gc) {
+            double2 a[E];
+#pragma unroll
+            for (int q = 0; q < E; ++q) a[q] = czero();
+            if (cg < ncg && r0 + r < G) {
+#pragma unroll 4
+                for (int j = cg; j < nc; j += ncg) {
+                    const size_t o = (size_t)G * (n0 + j) + r0 + r;
+                    const SdePack<K32> x(A + o), y(B + o);
+                    const double2 wj = wsm[j];
+#pragma unroll
+                    for (int q = 0; q < E; ++q) a[q] = cadd(a[q], cmul(cadd(x.x[q], y.x[q]), wj));
+                }
+#pragma unroll
+                for (int q = 0; q < E; ++q) red[E * (cg * Gc + r) + q] = a[q];
+            }
+            __syncthreads();
+            for (int i = tid; i < E * Gc; i += 256) {
+                if (E * r0 + i >= N) break;
+                double2 t = red[i];
+                for (int k = 1; k < ncg; ++k) t = cadd(t, red[E * Gc * k + i]);
+                add(E * r0 + i, t);
+            }
+            __syncthreads();
+        }
+    }
+}
+// NLEV Vertex levels summed into one pair of L-vertices (the target vertex and the local reference vertex of
+// the fdPA iteration share ΣΠ and the launch); a level's K3 terms with k3 set (a momentum-independent level's
+// are the GEMMs SdeRef*).  One block per (Ω, P), momentum fastest (blocks in flight share the slab of a
+// momentum-independent level): the terms without K3 first, then each K3 block read once, in 16-byte loads, its
+// sums added.  Bound by reading K3: K3 boxes (16, 32), 256 momenta, FP64 422 us (3.7 TB/s; one wave per (Ω, P)
+// with a second kernel for the a and t sums 473), FP32 275 us (405); boxes of 72, 576 momenta, FP32, one level
+// 839 us (one wave per (Ω, P), whose lanes took ν in two passes there, 2348).
+template <int NLEV>
 __global__ __launch_bounds__(256) void k_sde_L_nl(double2* __restrict__ Lpp, double2* __restrict__ Lph,
                                                   const double2* __restrict__ Pipp, const double2* __restrict__ Piph,
                                                   const double2* __restrict__ Tpp, const double2* __restrict__ Tph,
                                                   SdeLevelNL lv0, SdeLevelNL lv1, int n2b, int n2f, int nWP, int nVP,
                                                   int wb, int NP, double2 TU) {
-    const int wid = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
+    __shared__ double2 wsm[SDE_W], red[2 * 256], k2s[2][NLEV];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid / WAVE;
     const int NW2 = 2 * n2b - 1, NV2 = 2 * n2f;
-    if (wid >= NW2 * NP) return;
-    // momentum fastest: the waves in flight share Ω, so the local reference vertex's K3(Ω) slab (the
-    // same at every momentum) stays in L2 while they read it
-    const int p = wid % NP, iW = wid / NP;
-    const int m = iW - (n2b - 1);
+    const int p = (int)blockIdx.x % NP, iW = (int)blockIdx.x / NP, m = iW - (n2b - 1);
     const size_t row = (size_t)(m + nWP - 1) + (size_t)(2 * nWP - 1) * p;
     const double2* pp = Pipp + (size_t)(2 * nVP) * row + nVP;   // pp[ω], ω in [-nVP, nVP)
     const double2* ph = Piph + (size_t)(2 * nVP) * row + nVP;
-    auto inmesh = [&](int w) { return w >= -nVP && w < nVP; };
-    // totals over the bubble mesh (band + tails)
-    double a0 = 0, a1 = 0, b0 = 0, b1 = 0;
-    for (int w = -wb + lane; w < wb; w += WAVE) {
-        const double2 x = pp[w], y = ph[w];
-        a0 += x.x; a1 += x.y; b0 += y.x; b1 += y.y;
-    }
-    a0 = wave_sum(a0); a1 = wave_sum(a1); b0 = wave_sum(b0); b1 = wave_sum(b1);
-    const double2* tp = Tpp + (size_t)(2 * (wb + 1)) * row;
-    const double2* th = Tph + (size_t)(2 * (wb + 1)) * row;
-    const double2 spp = cadd(cmk(a0, a1), cadd(tp[0], tp[2 * wb + 1]));
-    const double2 sph = cadd(cmk(b0, b1), cadd(th[0], th[2 * wb + 1]));
-    // per level: the ν-independent K2 sums and K1
-    double2 k2p[NLEV], k2h[NLEV], k1p[NLEV], k1h[NLEV];
-#pragma unroll
-    for (int l = 0; l < NLEV; ++l) {
+    auto wpp = [&](int n) { return m - n - 1 >= -nVP && m - n - 1 < nVP ? pp[m - n - 1] : czero(); };
+    auto wph = [&](int n) { return n >= -nVP && n < nVP ? ph[n] : czero(); };
+    // ΣΠ over the bubble mesh from the tail sums on both sides of ω = 0
+    const double2* tp = Tpp + (size_t)(2 * (wb + 1)) * row + wb;
+    const double2* th = Tph + (size_t)(2 * (wb + 1)) * row + wb;
+    const double2 spp = cadd(tp[0], tp[1]), sph = cadd(th[0], th[1]);
+    // the ν-independent K2 sums: wave 2 l + 0 the p channel's of level l, wave 2 l + 1 those of a and t
+    if (wv < 2 * NLEV) {
+        const int l = wv >> 1;
         const SdeLevelNL& L = l == 0 ? lv0 : lv1;
         const int pc = L.chanNP > 1 ? p : 0;
-        const ChanBox P{L.gp, pc}, A{L.ga, pc}, T{L.gt, pc};
-        double c0 = 0, c1 = 0, d0 = 0, d1 = 0;
-        for (int n = -L.gp.n2f + lane; n < L.gp.n2f; n += WAVE) {
-            const int wp = m - n - 1;   // Lpp: K2p(Ω, n) at n = Ω - ω - 1
-            if (inmesh(wp)) { const double2 x = cmul(P.k2(m, n), pp[wp]); c0 += x.x; c1 += x.y; }
+        double2 s = czero();
+        if (wv & 1) {
+            const ChanBox A{L.ga, pc}, T{L.gt, pc};
+            const int nf = max(L.ga.n2f, L.gt.n2f);
+            for (int n = -nf + lane; n < nf; n += WAVE) s = cadd(s, cmul(cadd(A.k2(m, n), T.k2(m, n)), wph(n)));
+        } else {
+            const ChanBox P{L.gp, pc};
+            for (int n = -L.gp.n2f + lane; n < L.gp.n2f; n += WAVE) s = cadd(s, cmul(P.k2(m, n), wpp(n)));
         }
-        for (int n = -max(L.ga.n2f, L.gt.n2f) + lane; n < max(L.ga.n2f, L.gt.n2f); n += WAVE) {
-            if (inmesh(n)) { const double2 y = cmul(cadd(A.k2(m, n), T.k2(m, n)), ph[n]); d0 += y.x; d1 += y.y; }
-        }
-        k2p[l] = cmk(wave_sum(c0), wave_sum(c1));
-        k2h[l] = cmk(wave_sum(d0), wave_sum(d1));
-        k1p[l] = P.k1(m);
-        k1h[l] = cadd(A.k1(m), T.k1(m));
+        s = cmk(wave_sum(s.x), wave_sum(s.y));
+        if (lane == 0) k2s[wv & 1][l] = s;
     }
-    // the p-channel K3 sums with the lanes over the summation index (one pass over ν: 2 n2f <= 64)
-    double2 p3[NLEV];
-    bool p3l[NLEV];
-#pragma unroll
-    for (int l = 0; l < NLEV; ++l) {
-        const SdeLevelNL& L = l == 0 ? lv0 : lv1;
-        p3l[l] = NV2 <= WAVE && 2 * L.gp.n3f <= WAVE;
-        p3[l] = czero();
-        if (p3l[l] && in_b(m, L.gp.n3b) && !(l == 1 && SKIP1)) {
-            const int pc = L.chanNP > 1 ? p : 0;
-            const bool f32 = (l == 0 && F0 >= 0) ? F0 == 1 : L.gp.k3f != 0;
-            p3[l] = f32 ? sde_p3_lanes<true>(L.gp, pc, m, pp, nVP, n2f, lane)
-                             : sde_p3_lanes<false>(L.gp, pc, m, pp, nVP, n2f, lane);
-        }
-    }
-    for (int iv = lane; iv < NV2; iv += WAVE) {
+    __syncthreads();
+    double2* Lp = Lpp + iW + (size_t)NW2 * NV2 * p;
+    double2* Lh = Lph + iW + (size_t)NW2 * NV2 * p;
+    for (int iv = tid; iv < NV2; iv += 256) {
         const int v = iv - n2f;
         double2 xp = czero(), xh = czero();
 #pragma unroll
@@ -2829,74 +2846,35 @@ __global__ __launch_bounds__(256) void k_sde_L_nl(double2* __restrict__ Lpp, dou
             const SdeLevelNL& L = l == 0 ? lv0 : lv1;
             const int pc = L.chanNP > 1 ? p : 0;
             const ChanBox P{L.gp, pc}, A{L.ga, pc}, T{L.gt, pc};
-            xp = cadd(xp, cadd(cmul(cadd(k1p[l], P.k2(m, v)), spp), k2p[l]));
-            xh = cadd(xh, cadd(cmul(cadd(k1h[l], cadd(A.k2(m, v), T.k2(m, v))), sph), k2h[l]));
-            const int n3p = L.gp.n3f, n3h = max(L.ga.n3f, L.gt.n3f);
-            if (l == 1 && SKIP1) continue;
-            // the K3 form is the level's (one vertex): the loops branch on it once
-            if (p3l[l]) {
-                if (in_b(m, L.gp.n3b) && in_f(v, n3p)) xp = cadd(xp, p3[l]);
-            } else if (in_b(m, L.gp.n3b) && in_f(v, n3p)) {
-                auto psum = [&](auto form) {   // (wide boxes)
-                    constexpr bool K32 = decltype(form)::value;
-                    double2 sp = czero();
-                    for (int n = -n3p; n < n3p; ++n) {
-                        const int wp = m - n - 1;
-                        if (inmesh(wp)) sp = cadd(sp, cmul(P.template k3p<K32>(m, n, v), pp[wp]));
-                    }
-                    return sp;
-                };
-                const bool f32 = (l == 0 && F0 >= 0) ? F0 == 1 : L.gp.k3f != 0;
-                xp = cadd(xp, f32 ? psum(std::true_type{}) : psum(std::false_type{}));
-            }
-            if (!(l == 0 && F0 >= 0) && (in_b(m, L.ga.n3b) || in_b(m, L.gt.n3b)) && in_f(v, n3h)) {
-                auto hsum = [&](auto form) {
-                    constexpr bool K32 = decltype(form)::value;
-                    double2 sh = czero();
-#pragma unroll 8
-                    for (int n = -n3h; n < n3h; ++n)
-                        if (inmesh(n))
-                            sh = cadd(sh, cmul(cadd(A.template k3p<K32>(m, v, n), T.template k3p<K32>(m, v, n)), ph[n]));
-                    return sh;
-                };
-                const bool f32 = (l == 0 && F0 >= 0) ? F0 == 1 : L.ga.k3f != 0;
-                xh = cadd(xh, f32 ? hsum(std::true_type{}) : hsum(std::false_type{}));
-            }
+            xp = cadd(xp, cadd(cmul(cadd(P.k1(m), P.k2(m, v)), spp), k2s[0][l]));
+            xh = cadd(xh, cadd(cmul(cadd(cadd(A.k1(m), T.k1(m)), cadd(A.k2(m, v), T.k2(m, v))), sph), k2s[1][l]));
         }
-        const size_t o = (size_t)iW + (size_t)NW2 * ((size_t)iv + (size_t)NV2 * p);
-        Lpp[o] = cmul(xp, TU);
-        Lph[o] = cmul(xh, TU);
+        Lp[(size_t)NW2 * iv] = cmul(xp, TU);
+        Lh[(size_t)NW2 * iv] = cmul(xh, TU);
+    }
+#pragma unroll
+    for (int l = 0; l < NLEV; ++l) {
+        const SdeLevelNL& L = l == 0 ? lv0 : lv1;
+        const int pc = L.chanNP > 1 ? p : 0, n3 = L.gp.n3f, N = 2 * n3;
+        if (!L.k3 || !in_b(m, L.gp.n3b)) continue;
+        __syncthreads();   // L as written so far is read back below, by other threads
+        auto to = [&](double2* X) {
+            return [=](int i, double2 s) {
+                const int v = i - n3;
+                if (!in_f(v, n2f)) return;
+                double2& x = X[(size_t)NW2 * (v + n2f)];
+                x = cadd(x, cmul(s, TU));
+            };
+        };
+        auto wp = [&](int i) { return wpp(i - n3); };
+        auto wh = [&](int i) { return wph(i - n3); };
+        if (L.gp.k3f) sde_k3_cols<true>(sde_slab<true>(L.gp, m, pc), N, wsm, tid, wp, to(Lp));
+        else sde_k3_cols<false>(sde_slab<false>(L.gp, m, pc), N, wsm, tid, wp, to(Lp));
+        if (L.ga.k3f) sde_k3_rows<true>(sde_slab<true>(L.ga, m, pc), sde_slab<true>(L.gt, m, pc), N, wsm, red, tid, wh, to(Lh));
+        else sde_k3_rows<false>(sde_slab<false>(L.ga, m, pc), sde_slab<false>(L.gt, m, pc), N, wsm, red, tid, wh, to(Lh));
     }
 }
 
-// The a/t K3 sum of a lattice Vertex level at momentum P, added to Lph (the part k_sde_L_nl<.., F0>
-// leaves out): Lph(Ω, ν, P) += T U Σ_n [K3a + K3t](Ω, ν, n, P) Πph(Ω, n, P), the sum in k_sde_L_nl's
-// order.  One wave per (Ω, P), momentum fastest, lanes over ν; few registers, so many waves in flight.
-template <bool K32>
-__global__ __launch_bounds__(256) void k_sde_h3(double2* __restrict__ Lph, const double2* __restrict__ Piph, ChanV ga,
-                                                ChanV gt, int n2b, int n2f, int nWP, int nVP, int NP, double2 TU) {
-    const int wid = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
-    const int NW2 = 2 * n2b - 1, NV2 = 2 * n2f;
-    if (wid >= NW2 * NP) return;
-    const int p = wid % NP, iW = wid / NP;
-    const int m = iW - (n2b - 1);
-    if (!in_b(m, ga.n3b) && !in_b(m, gt.n3b)) return;
-    const size_t row = (size_t)(m + nWP - 1) + (size_t)(2 * nWP - 1) * p;
-    const double2* ph = Piph + (size_t)(2 * nVP) * row + nVP;
-    const ChanBox A{ga, p}, T{gt, p};
-    const int n3h = max(ga.n3f, gt.n3f);
-    for (int iv = lane; iv < NV2; iv += WAVE) {
-        const int v = iv - n2f;
-        if (!in_f(v, n3h)) continue;
-        double2 sh = czero();
-#pragma unroll 8
-        for (int n = -n3h; n < n3h; ++n)
-            if (n >= -nVP && n < nVP)
-                sh = cadd(sh, cmul(cadd(A.template k3p<K32>(m, v, n), T.template k3p<K32>(m, v, n)), ph[n]));
-        const size_t o = (size_t)iW + (size_t)NW2 * ((size_t)iv + (size_t)NV2 * p);
-        Lph[o] = cadd(Lph[o], cmul(sh, TU));
-    }
-}
 
 // Σ(ν) += scale T Σ_Ω [G(Ω-ν) Lpp(Ω,ν) + G(Ω+ν) Lph(Ω,ν)]  (src/SDE.jl:242-263); one wave per ν
 __device__ __forceinline__ void sde_sigma_local_wave(int wid, int lane, double2* __restrict__ S, const double2* __restrict__ G,
