@@ -97,6 +97,7 @@ struct fdga_ctx {
     double2* Ptail[4] = {nullptr, nullptr, nullptr, nullptr};      // tail sums of Π0pp, Π0ph, Πpp, Πph
     size_t ntail = 0;                                               // elements of one tail-sum array
     double2* pchunk[2] = {nullptr, nullptr};   // lattice bubble: chunk sums of the last Πpp / Πph [P, chunk, Ω]
+    double2* pfar = nullptr;                   // and the sums beyond its inner chunks [side, Ω, Πpp / Πph]
     int w_fresh = 0;                                                // Wc valid for the current iteration
     double2* seg[6] = {};                                           // local solver: K2 of F (p, t, a) and F0 along diagonals
     double2* wtot = nullptr;                                        // local solver: Σ_ω W per (Ω, channel)
@@ -394,11 +395,12 @@ std::vector<BubbleFold> bubble_folds(int L, int LG) {
 
 // band tail sums of one array on the bubble mesh (rows of 2 nVP entries)
 // ω entries per block of the lattice bubble (k_bubble_nl): 16 at L = 16 (16 x 256 complex in LDS);
-// 6 at L = 24 (6 x 576 complex + 24 twiddles, 55.7 KB); otherwise as many L x L tiles as fit 64 KB
+// 6 at L = 24 (6 x 576 complex + 24 twiddles, 55.7 KB); otherwise up to 8 (a whole line of Π per store, and
+// several blocks a CU on small lattices), as many L x L tiles twice as fit 64 KB
 int bubble_nb(int L) {
     if (L == 16) return 16;
     if (L == 24) return 6;
-    return std::max(1, std::min(16, (65536 / (int)sizeof(double2) - L) / (L * L)));
+    return std::max(1, std::min(8, (65536 / (int)sizeof(double2) - L) / (2 * L * L)));
 }
 
 int tail_sums(fdga_ctx* c, const double2* X, double2* T) {
@@ -439,27 +441,33 @@ int bubbles_into(fdga_ctx* c, double2* pp, double2* ph, const double2* Gsrc, boo
     if (dft2(c, c->tmpG1, c->NG, d.LG, -1, 1.0 / ((double)d.LG * d.LG), Gsrc)) return -3;
     // the Π_R products and the backward DFT over R' (src/nonlocal/bubble.jl:110-155) in one pass
     const int L = d.L, NB = bubble_nb(L);
-    const dim3 grid(cdiv(c->NVP, NB), c->NWP);
+    const int nchunk = (int)cdiv(c->NVP, NB);
     double2 *cpp = c->pchunk[0], *cph = c->pchunk[1];
     // the chunks [wlo, whi) that k_tail_sums_chunked reads entry by entry: those that meet the band
     const int wlo = band ? (c->nVP - c->wb) / NB : 0;
-    const int whi = band ? (c->nVP + c->wb + NB - 1) / NB : (int)grid.x;
+    const int whi = band ? (c->nVP + c->wb + NB - 1) / NB : nchunk;
+    // the inner chunks: those and the ones that meet G's mesh
+    const int ilo = std::min(wlo, std::max(0, c->nVP - d.nG) / NB);
+    const int ihi = std::max(whi, std::min(nchunk, (c->nVP + d.nG + NB - 1) / NB));
+    const int nin = ihi - ilo;
+    double2* fout = nin < nchunk ? c->pfar : nullptr;
+    const dim3 grid(nin + (fout ? 1 : 0), c->NWP);
     kernel_begin(c);
     if (L == 16 && d.precision == FDGA_FP32) {
         // the FP32 form: G(R) rounded to FP32 (into tmpG2), the products and the transform in FP32
         float2* GR32 = reinterpret_cast<float2*>(c->tmpG2);
         k_narrow32<<<cdiv(c->nGel, 256), 256, 0, c->run>>>(GR32, c->tmpG1, c->nGel);
         k_bubble_nl<16, 16, 512, float2><<<grid, 512, (size_t)NB * 256 * sizeof(float2), c->run>>>(
-            pp, ph, GR32, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi);
+            pp, ph, GR32, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, fout);
     } else if (L == 16) {
         k_bubble_nl<16, 16, 512><<<grid, 512, (size_t)NB * 256 * sizeof(double2), c->run>>>(
-            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi);
+            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, fout);
     } else if (L == 24) {
         k_bubble_nl<24, 6><<<grid, 256, (size_t)(NB * 576 + 24) * sizeof(double2), c->run>>>(
-            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi);
+            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, fout);
     } else {
-        k_bubble_nl<0, 0><<<grid, 256, (size_t)(NB * L * L + L) * sizeof(double2), c->run>>>(
-            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi);
+        k_bubble_nl<0, 0><<<grid, 256, (size_t)(2 * NB * L * L + L) * sizeof(double2), c->run>>>(
+            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, fout);
     }
     if (pp == c->Pipp) {
         c->pi_band = band ? 3 : 0;
@@ -469,8 +477,8 @@ int bubbles_into(fdga_ctx* c, double2* pp, double2* ph, const double2* Gsrc, boo
     LAUNCHCHK(c);
     // tail sums from the bubble's chunk sums
     const unsigned nblk = (unsigned)c->NWP * (unsigned)cdiv(c->NP, TAIL_NPB);
-    k_tail_sums_chunked<<<2 * nblk, 256, 0, c->run>>>(pp, cpp, pi_tail(c, pp), ph, cph, pi_tail(c, ph), nblk, c->nVP, c->wb,
-                                                      NB, (int)grid.x, c->NWP, c->NP);
+    k_tail_sums_chunked<<<2 * nblk, 256, 0, c->run>>>(pp, cpp, pi_tail(c, pp), ph, cph, pi_tail(c, ph), fout, nblk, c->nVP,
+                                                      c->wb, NB, ilo, nin, c->NWP, c->NP);
     LAUNCHCHK(c);
     return 0;
 }
@@ -1560,6 +1568,7 @@ int fdga_create(fdga_ctx** out, const fdga_dims* dims) {
         const size_t nch = (size_t)c->NP * cdiv(c->NVP, bubble_nb(d.L)) * c->NWP;
         rc |= dalloc(c, &c->pchunk[0], nch);
         rc |= dalloc(c, &c->pchunk[1], nch);
+        rc |= dalloc(c, &c->pfar, (size_t)4 * c->NWP);
         rc |= dalloc(c, &c->k2x, (size_t)c->NV2 * (2 * (size_t)c->wb) * c->NW2);
         rc |= dalloc(c, &c->k2xf, (size_t)c->NV2 * 2 * c->NW2);
         rc |= dalloc(c, &c->k2y, (size_t)c->NV2 * c->NW2 * c->NP);
@@ -1620,7 +1629,7 @@ int fdga_destroy(fdga_ctx* c) {
     for (double2* p : {c->Gbare, c->G0, c->Sig0, c->G, c->Sig, c->tmpG1, c->tmpG2, c->tmpG3, c->Pi0pp, c->Pi0ph,
                        c->Pipp, c->Piph, c->Wc[0], c->Wc[1], c->Wc[2], c->Lpp, c->Lph, c->tmpL1, c->tmpL2, c->sde0, c->u2C,
                        c->stage, c->Wfar[0], c->Wfar[1], c->Wfar[2], c->Ptail[0], c->Ptail[1], c->Ptail[2], c->Ptail[3],
-                       c->k2x, c->k2xf, c->k2y, c->lk2x, c->pchunk[0], c->pchunk[1]})
+                       c->k2x, c->k2xf, c->k2y, c->lk2x, c->pchunk[0], c->pchunk[1], c->pfar})
         if (p) (void)hipFree(p);
     for (auto* t : c->tab) if (t) (void)hipFree(t);
     for (auto* p : c->seg) if (p) (void)hipFree(p);

@@ -190,21 +190,7 @@ __global__ void k_dft2_rows(double2* data, const double2* src, size_t nrows, int
 // LDS, and written once as Π(ω, Ω, q), q = q1 + L q2.  Πpp and Πph use the LDS plane in turn.
 // LDS plane: s[R' * NB + ω - ω0] (the NB frequencies of one R' are contiguous).
 template <int L>
-struct BubbleDft {
-    // y = Σ_j x[j] e^{+2πi jk/L} over j < L, twiddles tw[k] = e^{+2πi k/L}
-    __device__ static void run(double2* x, const double2* tw, int Lr) {
-        double2 y[L];
-#pragma unroll
-        for (int k = 0; k < L; ++k) {
-            double2 acc = czero();
-#pragma unroll
-            for (int j = 0; j < L; ++j) acc = cadd(acc, cmul(x[j], tw[(j * k) % L]));
-            y[k] = acc;
-        }
-#pragma unroll
-        for (int k = 0; k < L; ++k) x[k] = y[k];
-    }
-};
+struct BubbleDft;
 // length 16: radix-4 in two stages, j = 4 j1 + j2, k = k1 + 4 k2:
 //   X[k1 + 4 k2] = Σ_j2 e^{2πi j2 k2/4} [e^{2πi j2 k1/16} Σ_j1 x[4 j1 + j2] e^{2πi j1 k1/4}]
 template <class CT>
@@ -342,13 +328,18 @@ __device__ __forceinline__ CT bubble_R(const CT* __restrict__ GR, const BubbleFo
     return acc;
 }
 
-// Blocks (16 ω chunks) with blockIdx.x in [wlo, whi) store their Π values; every block stores its chunk
-// sums.  The iteration passes the chunks that hold the band ω ∈ [-wb, wb) (every Π entry a later
-// stage reads outside the band enters only through the chunk sums); [0, gridDim.x) stores all of Π.
-// LT: L fixed at compile time (16: radix-4 FFT; 24: unrolled direct DFT), or 0 for a run-time
-// L <= 32 (direct DFT through private arrays, for small test lattices).  Block: NT threads (512 at
-// L = 16, held to 128 VGPRs: two blocks per CU, twice the waves on the same LDS tiles, to hide the
-// latency of the G(R) gathers).
+// Blocks take the NB-ω chunks ilo + blockIdx.x of the inner range [ilo, ilo + nin); those in [wlo, whi) store
+// their Π values, and all store their chunk sums.  The iteration passes for [wlo, whi) the chunks that hold the
+// band ω ∈ [-wb, wb) (every Π entry a later stage reads outside the band enters only through the chunk sums) and
+// for the inner range those and the ones that meet G's mesh: beyond it every product vanishes except the
+// origin's, which is the same at every momentum, and one block per Ω (blockIdx.x = nin) sums it over all ω of
+// either side (`fout`).  [0, chunks) for both stores all of Π.
+// L = 16, G's mesh of 512 in a bubble mesh of 4096, nΩ = 64: 270 us in FP64 (all chunks stored and summed one by
+// one: 712), 176 in FP32 (546).  L = 10, LG = 20, 120 of 296: 49 us (317, with the transform in private arrays);
+// L = 8, 128 of 512: 30 us (275).
+// LT: L fixed at compile time (16: radix-4 FFT, 24: 3 x 8), or 0 for a run-time L <= 32: a direct DFT from one
+// LDS plane to a second, four outputs per thread.  Block: NT threads (512 at L = 16, held to 128 VGPRs: two
+// blocks per CU, twice the waves on the same LDS tiles, to hide the latency of the G(R) gathers).
 // CT: double2, or float2 for the FP32 form (G(R), the products, the transform and the LDS tiles in
 // FP32; Π stored and the chunk sums accumulated in FP64): 32 KB of LDS per block and at most 80 VGPRs,
 // three blocks per CU.
@@ -357,15 +348,36 @@ __global__ __launch_bounds__(NT, NT >= 512 ? (sizeof(CT) == 8 ? 6 : 4) : 1) void
                                                    const CT* __restrict__ GR, const BubbleFold* __restrict__ folds,
                                                    int nG, int Lr, int nW, int nV, double T, int NBr,
                                                    double2* __restrict__ cpp, double2* __restrict__ cph, int wlo,
-                                                   int whi) {
-    extern __shared__ double2 sm[];   // NB * L * L (+ L twiddles unless L = 16) of CT
+                                                   int whi, int ilo, int nin, double2* __restrict__ fout) {
+    extern __shared__ double2 sm[];   // NB * L * L (twice for a run-time L; + L twiddles unless L = 16) of CT
     const int L = LT ? LT : Lr, LL = L * L, NB = NBT ? NBT : NBr;
     CT* s = reinterpret_cast<CT*>(sm);
-    CT* tw = s + NB * LL;
+    CT* s2 = s + NB * LL;
+    CT* tw = s + (LT ? 1 : 2) * NB * LL;
     const int tid = threadIdx.x;
-    const int iw0 = blockIdx.x * NB, iW = blockIdx.y;
+    const int chunk = ilo + (int)blockIdx.x, iw0 = chunk * NB, iW = blockIdx.y;
     const int m = iW - (nW - 1);
     const int nb = min(NB, 2 * nV - iw0);
+    if ((int)blockIdx.x == nin) {   // fout[side + 2 (iΩ + NΩ which)]
+        for (int q = 0; q < 4; ++q) {
+            const int which = q >> 1, lo = q & 1 ? (ilo + nin) * NB : 0, hi = q & 1 ? 2 * nV : ilo * NB;
+            double2 a = czero();
+            for (int k = lo + tid; k < hi; k += NT) {
+                const CT v = bubble_R(GR, folds[0], nG, T, m, k - nV, which);
+                a = cadd(a, cmk(v.x, v.y));
+            }
+            a = cmk(wave_sum(a.x), wave_sum(a.y));
+            if ((tid & (WAVE - 1)) == 0) sm[tid / WAVE] = a;
+            __syncthreads();
+            if (tid == 0) {
+                a = sm[0];
+                for (int k = 1; k < NT / WAVE; ++k) a = cadd(a, sm[k]);
+                fout[(q & 1) + 2 * (iW + (2 * nW - 1) * which)] = a;
+            }
+            __syncthreads();
+        }
+        return;
+    }
     if (LT != 16)
         for (int k = tid; k < L; k += blockDim.x) {
             double sn, cs;
@@ -376,20 +388,19 @@ __global__ __launch_bounds__(NT, NT >= 512 ? (sizeof(CT) == 8 ? 6 : 4) : 1) void
         // Far from ω = 0 one of each product's two frequencies lies outside G's mesh for every ω of
         // the block: then every product vanishes except the origin's (R = 0, the asymptotic G on both
         // sides), which folds onto R' = 0 alone, and the transform of that delta is the constant
-        // Π_R(ω, R' = 0) at every momentum (exactly: the radix-4 steps add zeros and multiply zeros).
+        // Π_R(ω, R' = 0) at every momentum (exactly: the transforms add zeros and multiply zeros).
         // Such blocks store that constant and its chunk sums without the products and transforms:
-        // the same values (up to the sign of zeros).  (L = 16, the radix-4 form.)
-        bool far = LT == 16;
-        if (LT == 16)
-            for (int wl = 0; wl < nb; ++wl) {
-                const int n = iw0 + wl - nV, n2nd = which == 0 ? bmf(m, n) : bpf(m, n);
-                far = far && (!in_f(n, nG) || !in_f(n2nd, nG));
-            }
+        // the same values (up to the sign of zeros).
+        bool far = true;
+        for (int wl = 0; wl < nb; ++wl) {
+            const int n = iw0 + wl - nV, n2nd = which == 0 ? bmf(m, n) : bpf(m, n);
+            far = far && (!in_f(n, nG) || !in_f(n2nd, nG));
+        }
         if (far) {
             if (tid < NB)
                 s[tid] = tid < nb ? bubble_R(GR, folds[0], nG, T, m, iw0 + tid - nV, which) : cmk_as<CT>(0.0, 0.0);
             __syncthreads();
-            if ((int)blockIdx.x >= wlo && (int)blockIdx.x < whi) {
+            if (chunk >= wlo && chunk < whi) {
                 double2* out = which == 0 ? pp : ph;
                 const size_t qs = (size_t)(2 * nV) * (size_t)(2 * nW - 1);
                 for (int e = tid; e < NB * LL; e += blockDim.x) {
@@ -405,7 +416,7 @@ __global__ __launch_bounds__(NT, NT >= 512 ? (sizeof(CT) == 8 ? 6 : 4) : 1) void
                         const int wl = (j + P) % NB;
                         if (wl < nb) { const CT v = s[wl]; sr += v.x; si += v.y; }
                     }
-                    cs[(size_t)P + (size_t)LL * (blockIdx.x + (size_t)gridDim.x * iW)] = cmk(sr, si);
+                    cs[(size_t)P + (size_t)LL * (blockIdx.x + (size_t)nin * iW)] = cmk(sr, si);
                 }
             __syncthreads();   // s is reused by the next products
             continue;
@@ -431,32 +442,60 @@ __global__ __launch_bounds__(NT, NT >= 512 ? (sizeof(CT) == 8 ? 6 : 4) : 1) void
         __syncthreads();
         // along R1' (thread: ω, R2'), then along R2' (thread: ω, q1) with the write-out
         for (int pass = 0; pass < 2; ++pass) {
-            for (int e = tid; e < NB * L; e += blockDim.x) {
-                const int wl = e % NB, r = e / NB;
-                const int base = pass == 0 ? L * r : r, step = pass == 0 ? 1 : L;
-                CT x[LT ? LT : 32];
-                for (int j = 0; j < L; ++j) x[j] = s[(base + step * j) * NB + wl];
-                if (LT) BubbleDft<LT ? LT : 1>::run(x, tw, L);
-                else {
-                    CT y[32];
-                    for (int k = 0; k < L; ++k) {
-                        CT acc = cmk_as<CT>(0.0, 0.0);
-                        for (int j = 0; j < L; ++j) acc = cadd(acc, cmul(x[j], tw[(j * k) % L]));
-                        y[k] = acc;
+            if constexpr (LT != 0) {
+                for (int e = tid; e < NB * L; e += blockDim.x) {
+                    const int wl = e % NB, r = e / NB;
+                    const int base = pass == 0 ? L * r : r, step = pass == 0 ? 1 : L;
+                    CT x[LT ? LT : 1];
+                    for (int j = 0; j < L; ++j) x[j] = s[(base + step * j) * NB + wl];
+                    BubbleDft<LT>::run(x, tw, L);
+                    if (pass == 0) {
+                        for (int k = 0; k < L; ++k) s[(base + k) * NB + wl] = x[k];
+                    } else {
+                        // back into the thread's own column, for the chunk sums below
+                        for (int k = 0; k < L; ++k) s[(r + L * k) * NB + wl] = x[k];
+                        if (wl < nb && chunk >= wlo && chunk < whi) {
+                            double2* out = which == 0 ? pp : ph;
+                            const size_t o = (size_t)(iw0 + wl) + (size_t)(2 * nV) * (size_t)iW;
+                            const size_t qs = (size_t)(2 * nV) * (size_t)(2 * nW - 1);
+                            for (int k = 0; k < L; ++k) out[o + qs * (size_t)(r + L * k)] = cmk(x[k].x, x[k].y);
+                        }
                     }
-                    for (int k = 0; k < L; ++k) x[k] = y[k];
                 }
-                if (pass == 0) {
-                    for (int k = 0; k < L; ++k) s[(base + k) * NB + wl] = x[k];
-                } else {
-                    // back into the thread's own column, for the chunk sums below
-                    for (int k = 0; k < L; ++k) s[(r + L * k) * NB + wl] = x[k];
-                    if (wl < nb && (int)blockIdx.x >= wlo && (int)blockIdx.x < whi) {
-                        double2* out = which == 0 ? pp : ph;
-                        const size_t o = (size_t)(iw0 + wl) + (size_t)(2 * nV) * (size_t)iW;
-                        const size_t qs = (size_t)(2 * nV) * (size_t)(2 * nW - 1);
-                        for (int k = 0; k < L; ++k) out[o + qs * (size_t)(r + L * k)] = cmk(x[k].x, x[k].y);
+            } else {   // s -> s2, s2 -> s
+                const CT* src = pass == 0 ? s : s2;
+                CT* dst = pass == 0 ? s2 : s;
+                double2* out = (which == 0 ? pp : ph) + (size_t)iw0 + (size_t)(2 * nV) * (size_t)iW;
+                const size_t qs = (size_t)(2 * nV) * (size_t)(2 * nW - 1);
+                const bool st = chunk >= wlo && chunk < whi;
+                const int NK = (L + 3) / 4;
+                for (int e = tid; e < NB * L * NK; e += blockDim.x) {
+                    const int wl = e % NB, r = (e / NB) % L, k0 = e / (NB * L) * 4;
+                    const int base = pass == 0 ? L * r : r, step = pass == 0 ? 1 : L;
+                    CT acc[4];
+                    int ti[4], dt[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        acc[q] = cmk_as<CT>(0.0, 0.0);
+                        ti[q] = 0;
+                        dt[q] = min(k0 + q, L - 1);
                     }
+                    for (int j = 0; j < L; ++j) {
+                        const CT x = src[(base + step * j) * NB + wl];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            acc[q] = cadd(acc[q], cmul(x, tw[ti[q]]));
+                            ti[q] += dt[q];   // j k mod L
+                            if (ti[q] >= L) ti[q] -= L;
+                        }
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (k0 + q < L) {
+                            dst[(base + step * (k0 + q)) * NB + wl] = acc[q];
+                            if (pass == 1 && wl < nb && st)
+                                out[wl + qs * (size_t)(r + L * (k0 + q))] = cmk(acc[q].x, acc[q].y);
+                        }
                 }
             }
             __syncthreads();
@@ -472,7 +511,7 @@ __global__ __launch_bounds__(NT, NT >= 512 ? (sizeof(CT) == 8 ? 6 : 4) : 1) void
                     const int wl = (j + P) % NB;
                     if (wl < nb) { const CT v = s[P * NB + wl]; sr += v.x; si += v.y; }
                 }
-                cs[(size_t)P + (size_t)LL * (blockIdx.x + (size_t)gridDim.x * iW)] = cmk(sr, si);
+                cs[(size_t)P + (size_t)LL * (blockIdx.x + (size_t)nin * iW)] = cmk(sr, si);
             }
             __syncthreads();   // s is reused by the next products
         }
@@ -2205,10 +2244,11 @@ __global__ __launch_bounds__(256) void k_tail_sums2(const double2* __restrict__ 
     else tail_sums_row(X1, T1, nVP, wb, nrows, blockIdx.x - nrows);
 }
 
-// k_tail_sums for an array whose chunk sums C[P + NP (chunk + NC iΩ)] over NB consecutive ω
-// were written by the lattice bubble: the parts outside the band are the sums of the chunks that
-// lie wholly outside it plus the few entries of the chunks it cuts; the band as in k_tail_sums.
-// Reads NC + 2 wb + O(NB) entries per row instead of 2 nVP.  A block takes the rows of 8
+// k_tail_sums for an array whose chunk sums C[P + NP (chunk - ilo + NC iΩ)] over NB consecutive ω
+// were written by the lattice bubble for its NC inner chunks [ilo, ilo + NC), and the sums beyond them
+// (F[side + 2 iΩ], the same at every momentum; null: nothing beyond): the parts outside the band are those,
+// the sums of the inner chunks that lie wholly outside it and the few entries of the chunks it cuts; the band
+// as in k_tail_sums.  Reads NC + 2 wb + O(NB) entries per row instead of 2 nVP.  A block takes the rows of 8
 // consecutive momenta at one Ω: its chunk-sum reads cover whole 128-byte lines (8 momenta per
 // line), the 32 thread groups' partial sums are added in a fixed order, and each wave then scans
 // the band of two rows.
@@ -2217,8 +2257,8 @@ constexpr int TAIL_NPB = 8;
 __global__ __launch_bounds__(256) void k_tail_sums_chunked(const double2* __restrict__ X0, const double2* __restrict__ C0,
                                                            double2* __restrict__ T0, const double2* __restrict__ X1,
                                                            const double2* __restrict__ C1, double2* __restrict__ T1,
-                                                           unsigned nblk, int nVP, int wb, int NB, int NC, int NWP,
-                                                           int NP) {
+                                                           const double2* __restrict__ F, unsigned nblk, int nVP, int wb,
+                                                           int NB, int ilo, int NC, int NWP, int NP) {
     __shared__ double2 red[2][32][TAIL_NPB + 1];
     __shared__ double2 far[2][TAIL_NPB];
     const bool second = blockIdx.x >= nblk;
@@ -2236,8 +2276,8 @@ __global__ __launch_bounds__(256) void k_tail_sums_chunked(const double2* __rest
         double lr = 0.0, li = 0.0, rr = 0.0, ri = 0.0;
         if (p < NP) {
             const double2* cp = C + (size_t)p + (size_t)NP * (size_t)NC * iW;
-            for (int c = cg; c < cl; c += 32) { const double2 v = cp[(size_t)NP * c]; lr += v.x; li += v.y; }
-            for (int c = cr + cg; c < NC; c += 32) { const double2 v = cp[(size_t)NP * c]; rr += v.x; ri += v.y; }
+            for (int c = cg; c < cl - ilo; c += 32) { const double2 v = cp[(size_t)NP * c]; lr += v.x; li += v.y; }
+            for (int c = cr - ilo + cg; c < NC; c += 32) { const double2 v = cp[(size_t)NP * c]; rr += v.x; ri += v.y; }
         }
         red[0][cg][pl] = cmk(lr, li);
         red[1][cg][pl] = cmk(rr, ri);
@@ -2247,6 +2287,7 @@ __global__ __launch_bounds__(256) void k_tail_sums_chunked(const double2* __rest
         const int side = tid / TAIL_NPB, pl = tid % TAIL_NPB;
         double sr = 0.0, si = 0.0;
         for (int g = 0; g < 32; ++g) { sr += red[side][g][pl].x; si += red[side][g][pl].y; }
+        if (F) { const double2 f = F[side + 2 * (iW + (second ? NWP : 0))]; sr += f.x; si += f.y; }
         far[side][pl] = cmk(sr, si);
     }
     __syncthreads();
