@@ -92,16 +92,14 @@ struct fdga_ctx {
     double2 *Gbare = nullptr, *G0 = nullptr, *Sig0 = nullptr, *G = nullptr, *Sig = nullptr;
     double2 *Pi0pp = nullptr, *Pi0ph = nullptr, *Pipp = nullptr, *Piph = nullptr;
     double2 *Lpp = nullptr, *Lph = nullptr;
-    double2* Wc[3] = {nullptr, nullptr, nullptr};                  // BSE_K1!/BSE_K2! weights per channel
-    double2* Wfar[3] = {nullptr, nullptr, nullptr};                // their far factors per row (WTail)
-    double2* Ptail[4] = {nullptr, nullptr, nullptr, nullptr};      // tail sums of Π0pp, Π0ph, Πpp, Πph
+    double2* Wc[3] = {nullptr, nullptr, nullptr};                  // BSE_K2! weights per channel
+    double2* Ptail[4] = {nullptr, nullptr, nullptr, nullptr};      // sums (k_tail_sums) of Π0pp, Π0ph, Πpp, Πph
     size_t ntail = 0;                                               // elements of one tail-sum array
     double2* pchunk[2] = {nullptr, nullptr};   // lattice bubble: chunk sums of the last Πpp / Πph [P, chunk, Ω]
     double2* pfar = nullptr;                   // and the sums beyond its inner chunks [side, Ω, Πpp / Πph]
-    int w_fresh = 0;                                                // Wc valid for the current iteration
+    int w_fresh = 0;                                                // Wc and wsum valid for the current iteration
     double2* seg[6] = {};                                           // local solver: K2 of F (p, t, a) and F0 along diagonals
-    double2* wtot = nullptr;                                        // local solver: Σ_ω W per (Ω, channel)
-    int tot_fresh = 0;                                              // wtot valid for the current iteration
+    double2* wsum = nullptr;                                        // sums of W over the bubble mesh (K1Args)
     int seg_fresh = 0;                                              // seg valid for the current iteration
     // lattice BSE_K2! / BSE_L_K2! tables and GEMM result (s-wave solver only)
     double2 *k2x = nullptr, *k2xf = nullptr, *k2y = nullptr, *lk2x = nullptr;
@@ -628,7 +626,7 @@ int sde_level_L(fdga_ctx* c, const Level& lv, const double2* Pp, const double2* 
             const bool refgemm = lv2->chanNP == 1 && c->NP > 1;
             const SdeLevelNL l1{lv2->g[0], lv2->g[1], lv2->g[2], lv2->chanNP, !refgemm};
             k_sde_L_nl<2><<<nb, 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, l0, l1, d.nK2b, d.nK2f, d.nK1, c->nVP,
-                                                  c->wb, c->NP, TU);
+                                                  c->NP, TU);
             LAUNCHCHK(c);
             if (refgemm) {
                 const ChanV& gp = lv2->g[PCH];
@@ -646,7 +644,7 @@ int sde_level_L(fdga_ctx* c, const Level& lv, const double2* Pp, const double2* 
             }
         } else {
             k_sde_L_nl<1><<<nb, 256, 0, c->run>>>(c->Lpp, c->Lph, Pp, Ph, Tpp, Tph, l0, l0, d.nK2b, d.nK2f, d.nK1, c->nVP,
-                                                  c->wb, c->NP, TU);
+                                                  c->NP, TU);
         }
         LAUNCHCHK(c);
         // SGpp2 / SGph2 (SG0pp2 / SG0ph2 for the reference system): members from representatives
@@ -662,7 +660,7 @@ int sde_level_L(fdga_ctx* c, const Level& lv, const double2* Pp, const double2* 
         a.Pp = Pp; a.Ph = Ph; a.Tp = Tpp; a.Th = Tph;
         a.Lpp = c->Lpp; a.Lph = c->Lph;
         a.TU = TU;
-        a.n2b = d.nK2b; a.n2f = d.nK2f; a.nWP = d.nK1; a.nVP = c->nVP; a.wb = c->wb;
+        a.n2b = d.nK2b; a.n2f = d.nK2f; a.nWP = d.nK1; a.nVP = c->nVP;
         a.sp = spp; a.sh = sph;
         a.npp = (int)nclass(spp, nout);
         a.nph = (int)nclass(sph, nout);
@@ -744,17 +742,6 @@ int idx_fbase(int ch) { return ch == PCH ? 7 : ch == ACH ? 8 : 9; }
 // classes of the channel's K2 (SGpp[2] = SGppL[2] for p, SGph[2] = SGphL[2] for a and t)
 static SymCls sym_k2(const fdga_ctx* c, int ch) { return symcls(c, ch == PCH ? SG_PP2 : SG_PH2); }
 
-static WTail wtail(fdga_ctx* c, int ch);
-static SegTot seg_tot_args(fdga_ctx* c) {
-    SegTot a{};
-    for (int ch = 0; ch < 3; ++ch) {
-        a.W[ch] = c->Wc[ch];
-        a.T[ch] = wtail(c, ch);
-    }
-    a.out = c->wtot;
-    a.n2b = c->d.nK2b; a.nWP = c->d.nK1; a.wb = c->wb;
-    return a;
-}
 // the local solver's K2 copies along diagonals (F, and F0 when it is a Vertex; once per iteration), and for the
 // channels in `left` (bit ch) the weights of BSE_L_K2! into Wc, in one launch
 static int launch_seg_prep(fdga_ctx* c, int left) {
@@ -774,7 +761,7 @@ static int launch_seg_prep(fdga_ctx* c, int left) {
                 blk += cdiv((size_t)2 * g.n2f * g.rows(), 256);
             }
     a.wblk = blk;
-    a.wper = cdiv((size_t)2 * c->wb * c->NWP, 256);
+    a.wper = cdiv((size_t)2 * c->wb * c->NW2, 256);
     int nw = 0;
     for (int ch = 0; ch < 3; ++ch)
         if (left >> ch & 1) {
@@ -783,7 +770,7 @@ static int launch_seg_prep(fdga_ctx* c, int left) {
             a.wch[nw++] = ch;
         }
     a.f0 = f0;
-    a.nWP = d.nK1; a.nVP = c->nVP; a.wb = c->wb;
+    a.n2b = d.nK2b; a.nWP = d.nK1; a.nVP = c->nVP; a.wb = c->wb;
     blk += nw * a.wper;
     if (blk) k_seg_prep<<<blk, 256, 0, c->run>>>(a);
     LAUNCHCHK(c);
@@ -808,16 +795,12 @@ static int launch_seg_k2(fdga_ctx* c, int chs) {
     a.ref = f0.ref;
     a.Wp = c->Wc[PCH]; a.Wt = c->Wc[TCH]; a.Wa = c->Wc[ACH];
     if (!LEFT) {
-        if (!c->tot_fresh) {
-            k_seg_tot<<<cdiv((size_t)3 * c->NW2 * WAVE, 256), 256, 0, c->run>>>(seg_tot_args(c));
-            LAUNCHCHK(c);
-        }
-        a.tot = c->wtot;
+        a.ws = c->wsum;
         a.Lp = c->FL[PCH].K2; a.Lt = c->FL[TCH].K2; a.La = c->FL[ACH].K2;
     }
     DevChan* out = LEFT ? c->FL : c->Fb;
     a.Kp = out[PCH].K2; a.Kt = out[TCH].K2; a.Ka = out[ACH].K2;
-    a.n2b = d.nK2b; a.n2f = d.nK2f; a.nWP = d.nK1; a.nVP = c->nVP; a.wb = c->wb;
+    a.n2b = d.nK2b; a.n2f = d.nK2f; a.wb = c->wb;
     a.T = d.T;
     a.sp = symcls(c, SG_PP2);
     a.sat = symcls(c, SG_PH2);
@@ -859,72 +842,56 @@ static int launch_lk2_all(fdga_ctx* c) {
     return launch_seg_k2<true>(c, 7);
 }
 
-// the arrays of channel ch's weight: W on the band and its far sums from Π and Π0 and their tails
-static WArgs w_args(fdga_ctx* c, int ch) {
-    double2* P = pi_of(c, ch, false);
-    double2* P0 = pi_of(c, ch, true);
-    return WArgs{c->Wc[ch], c->Wfar[ch], P, P0};
-}
-// the tail sums of channel ch's weight, formed from those of Π and Π0 and the far factors
-static WTail wtail(fdga_ctx* c, int ch) {
-    return WTail{pi_tail(c, pi_of(c, ch, false)), pi_tail(c, pi_of(c, ch, true)), c->Wfar[ch]};
-}
-// K1/K2 weights of channel CH on the band into Wc[CH], their far factors into Wfar[CH]
-template <int CH>
-static int launch_w(fdga_ctx* c) {
-    const size_t nrows = (size_t)c->NWP * c->NP;
-    k_bse_w<CH><<<cdiv(nrows * (2 * c->wb), 256), 256, 0, c->run>>>(w_args(c, CH), vtx_FL(c), f0_view(c), c->d.nK1,
-                                                                       c->nVP, c->wb, box_bound(c), nrows);
+// the K2 weights of the channels in `mask` (bit ch) on the band into Wc
+static int launch_w(fdga_ctx* c, int mask) {
+    WArgs a{};
+    for (int r = 0; r < 3; ++r) {
+        a.W[r] = c->Wc[r];
+        a.L[r] = chanF(c, c->FL[r]);
+    }
+    a.Ppp = c->Pipp; a.Ppp0 = c->Pi0pp; a.Pph = c->Piph; a.Pph0 = c->Pi0ph;
+    a.f0 = f0_view(c);
+    a.n2b = c->d.nK2b; a.nWP = c->d.nK1; a.nVP = c->nVP; a.wb = c->wb; a.NP = c->NP; a.mask = mask;
+    // the momenta of a thread: as many as leave some 512 blocks, at most W_PCH
+    const size_t n = (size_t)2 * c->wb * c->NW2;
+    a.pch = (int)std::max<size_t>(1, std::min<size_t>(W_PCH, n * c->NP / (512 * 256)));
+    k_bse_w<<<dim3(cdiv(2 * c->wb, 32), cdiv(c->NW2, 8), cdiv(c->NP, a.pch)), 256, 0, c->run>>>(a);
     LAUNCHCHK(c);
     return 0;
 }
-// the weights of the three channels in one launch
-static int launch_w_all(fdga_ctx* c) {
-    const size_t nrows = (size_t)c->NWP * c->NP;
-    // lattice solver: one thread per chunk of W_PCH momenta (the P-independent reference factor once)
-    const int pchunk = c->NP >= 2 * W_PCH;
-    const size_t nth = pchunk ? (size_t)c->NWP * cdiv(c->NP, W_PCH) * (2 * c->wb) : nrows * (2 * c->wb);
-    const unsigned nb = cdiv(nth, 256);
-    k_bse_w3<<<3 * nb, 256, 0, c->run>>>(w_args(c, PCH), w_args(c, TCH), w_args(c, ACH), vtx_FL(c), f0_view(c), c->d.nK1,
-                                         c->nVP, c->wb, box_bound(c), nrows, nb, pchunk, c->NP);
+// BSE_K1! of the channels in `mask` and the sums of their weights for BSE_K2!; k1 = false: the sums alone
+static int launch_k1(fdga_ctx* c, int mask, bool k1 = true) {
+    K1Args a{};
+    a.F = vtx_F(c);
+    for (int r = 0; r < 3; ++r) a.L[r] = chanF(c, c->FL[r]);
+    a.Ppp = c->Pipp; a.Ppp0 = c->Pi0pp; a.Pph = c->Piph; a.Pph0 = c->Pi0ph;
+    a.Spp = pi_tail(c, c->Pipp); a.Spp0 = pi_tail(c, c->Pi0pp); a.Sph = pi_tail(c, c->Piph); a.Sph0 = pi_tail(c, c->Pi0ph);
+    a.Kp = c->Fb[PCH].K1; a.Kt = c->Fb[TCH].K1; a.Ka = c->Fb[ACH].K1;
+    a.ws = c->wsum;
+    a.n1 = c->d.nK1; a.n2b = c->d.nK2b; a.nWP = c->d.nK1; a.nVP = c->nVP; a.NP = c->NP; a.mask = mask;
+    a.T = c->d.T;
+    a.sym = symcls(c, SG_K1);
+    a.nk = k1 ? (int)nclass(a.sym, c->n1 * c->NP) : 0;
+    a.ntot = !k1 || a.sym.ncls ? c->NW2 * c->NP : 0;
+    k_k1<<<8 * cdiv((size_t)2 * (a.nk + a.ntot) * WAVE, 8 * 256), 256, 0, c->run>>>(a);
     LAUNCHCHK(c);
     return 0;
 }
-
-template <int CH>
-static int launch_k1(fdga_ctx* c) {
-    if (!c->w_fresh && launch_w<CH>(c)) return -3;
-    const SymCls sym = symcls(c, SG_K1);
-    const size_t nw = nclass(sym, c->n1 * c->NP);
-    k_gemv_k1<CH><<<(unsigned)nw, 256, 0, c->run>>>(c->Fb[CH].K1, c->Fb[ACH].K1, c->Wc[CH], wtail(c, CH), vtx_F(c), c->d.nK1,
-                                                           c->d.nK1, c->nVP, c->wb, c->NP, c->d.T * kSign[CH], box_bound(c), sym);
-    LAUNCHCHK(c);
-    return 0;
-}
-
-// BSE_K1! of the three channels in one launch; for the local solver with the weight totals of BSE_K2!
-static int launch_k1_all(fdga_ctx* c) {
-    if (!c->w_fresh && (launch_w<PCH>(c) || launch_w<ACH>(c) || launch_w<TCH>(c))) return -3;
-    const SymCls sym = symcls(c, SG_K1);
-    const int nw = (int)nclass(sym, c->n1 * c->NP);
-    const unsigned nt = c->d.nonlocal ? 0 : cdiv((size_t)3 * c->NW2 * WAVE, 256);
-    k_k1_all<<<(unsigned)(2 * nw) + nt, 256, 0, c->run>>>(
-        c->Fb[PCH].K1, c->Fb[ACH].K1, c->Fb[TCH].K1, c->Wc[PCH], c->Wc[ACH], c->Wc[TCH], wtail(c, PCH), wtail(c, ACH),
-        wtail(c, TCH), vtx_F(c), c->d.nK1, c->d.nK1, c->nVP, c->wb, c->NP, c->d.T, box_bound(c), sym, nw, seg_tot_args(c));
-    LAUNCHCHK(c);
-    return 0;
+// what BSE_K2! of the channels in `mask` reads: their weights and the sums of these, unless they are there already
+static int k2_inputs(fdga_ctx* c, int mask) {
+    return c->w_fresh ? 0 : launch_w(c, mask) || launch_k1(c, mask, false) ? -3 : 0;
 }
 
 // lattice BSE_K2!: X table, GEMM X W per Ω over the band, finish per (Ω, P)
 template <int CH>
 static int launch_k2_nl(fdga_ctx* c) {
-    if (!c->w_fresh && launch_w<CH>(c)) return -3;
+    if (k2_inputs(c, 1 << CH)) return -3;
     const int NV2 = c->NV2, NW2 = c->NW2, K = 2 * c->wb;
     const size_t nx = (size_t)NV2 * K * NW2 + (size_t)NV2 * 2 * NW2;
     k_k2nl_table<CH><<<cdiv(nx, 256), 256, 0, c->run>>>(c->k2x, c->k2xf, vtx_F(c), c->d.nK2b, c->d.nK2f, c->wb);
     LAUNCHCHK(c);
     const K2nl_A a{c->k2x, NV2, K};
-    const K2nl_B b{c->Wc[CH], K, 0, c->d.nK1 - c->d.nK2b, c->NWP};
+    const K2nl_B b{c->Wc[CH], K, 0, 0, NW2};
     const K2nl_E e{c->k2y, NV2, NW2};
     if (zgemm_launch(0, NW2, c->run, NV2, c->NP, K, cdiv(NV2, GBM), cdiv(c->NP, GBN), nullptr, 0, a, b, e) != hipSuccess)
         return fail(c, "BSE_K2 GEMM launch failed", -3);
@@ -934,8 +901,8 @@ static int launch_k2_nl(fdga_ctx* c) {
     const size_t n2 = c->n2 * c->NP;
     double2* raw = rp ? c->k2raw + (CH == PCH ? 0 : n2) : nullptr;
     k_k2nl_finish<CH><<<cdiv((size_t)NW2 * c->NP * WAVE, 256), 256, 0, c->run>>>(
-        c->Fb[CH].K2, c->Fb[ACH].K2, c->k2y, c->k2xf, c->Wc[CH], wtail(c, CH), vtx_F(c), chanF(c, c->FL[CH]),
-        chanF(c, c->FL[ACH]), c->d.nK2b, c->d.nK2f, c->d.nK1, c->wb, c->NP, c->d.T * kSign[CH], raw);
+        c->Fb[CH].K2, c->Fb[ACH].K2, c->k2y, c->k2xf, c->wsum + (size_t)3 * CH * NW2 * c->NP, vtx_F(c),
+        chanF(c, c->FL[CH]), chanF(c, c->FL[ACH]), c->d.nK2b, c->d.nK2f, c->NP, c->d.T * kSign[CH], raw);
     LAUNCHCHK(c);
     {   // the own-K3 product term (T s Σ_ω K3 W; halved for a finished t, whose post-processing halves)
         const VtxV F = vtx_F(c);
@@ -943,9 +910,9 @@ static int launch_k2_nl(fdga_ctx* c) {
         const double f = c->d.T * kSign[CH] * ((CH == TCH && !raw) ? 0.5 : 1.0);
         const unsigned nb = (unsigned)cdiv((size_t)NW2 * c->NP * WAVE, 256);
         if (F.g[CH].k3f)
-            k_k2nl_k3<CH, true><<<nb, 256, 0, c->run>>>(out, c->Wc[CH], F, c->d.nK2b, c->d.nK2f, c->d.nK1, c->wb, c->NP, f);
+            k_k2nl_k3<CH, true><<<nb, 256, 0, c->run>>>(out, c->Wc[CH], F, c->d.nK2b, c->d.nK2f, c->wb, c->NP, f);
         else
-            k_k2nl_k3<CH, false><<<nb, 256, 0, c->run>>>(out, c->Wc[CH], F, c->d.nK2b, c->d.nK2f, c->d.nK1, c->wb, c->NP, f);
+            k_k2nl_k3<CH, false><<<nb, 256, 0, c->run>>>(out, c->Wc[CH], F, c->d.nK2b, c->d.nK2f, c->wb, c->NP, f);
         LAUNCHCHK(c);
     }
     if (rp) {
@@ -959,14 +926,14 @@ static int launch_k2_nl(fdga_ctx* c) {
 template <int CH>
 static int launch_k2(fdga_ctx* c) {
     if (c->d.nonlocal) return launch_k2_nl<CH>(c);
-    if (!c->w_fresh && launch_w<CH>(c)) return -3;
+    if (k2_inputs(c, 1 << CH)) return -3;
     return launch_seg_k2<false>(c, 1 << CH);
 }
 
 // BSE_K2! of the three channels: one launch for the local solver
 static int launch_k2_all(fdga_ctx* c) {
     if (c->d.nonlocal) return launch_k2<PCH>(c) || launch_k2<ACH>(c) || launch_k2<TCH>(c);
-    if (!c->w_fresh && (launch_w<PCH>(c) || launch_w<ACH>(c) || launch_w<TCH>(c))) return -3;
+    if (k2_inputs(c, 7)) return -3;
     return launch_seg_k2<false>(c, 7);
 }
 
@@ -1559,10 +1526,10 @@ int fdga_create(fdga_ctx** out, const fdga_dims* dims) {
     for (double2** p : {&c->Gbare, &c->G0, &c->Sig0, &c->G, &c->Sig, &c->tmpG1, &c->tmpG2, &c->tmpG3})
         rc |= dalloc(c, p, c->nGel);
     for (double2** p : {&c->Pi0pp, &c->Pi0ph, &c->Pipp, &c->Piph}) rc |= dalloc(c, p, c->nPiel);
-    for (double2** p : {&c->Wc[0], &c->Wc[1], &c->Wc[2]}) rc |= dalloc(c, p, (size_t)c->NWP * c->NP * (2 * (size_t)c->wb));
-    c->ntail = (size_t)c->NWP * c->NP * (2 * (size_t)c->wb + 2);
+    for (double2** p : {&c->Wc[0], &c->Wc[1], &c->Wc[2]}) rc |= dalloc(c, p, (size_t)c->NW2 * c->NP * (2 * (size_t)c->wb));
+    rc |= dalloc(c, &c->wsum, (size_t)9 * c->NW2 * c->NP);
+    c->ntail = (size_t)3 * c->NWP * c->NP;
     for (double2** p : {&c->Ptail[0], &c->Ptail[1], &c->Ptail[2], &c->Ptail[3]}) rc |= dalloc(c, p, c->ntail);
-    for (double2** p : {&c->Wfar[0], &c->Wfar[1], &c->Wfar[2]}) rc |= dalloc(c, p, (size_t)4 * c->NWP * c->NP);
     for (double2** p : {&c->Lpp, &c->Lph, &c->tmpL1, &c->tmpL2}) rc |= dalloc(c, p, c->nL);
     if (d.nonlocal) {
         const size_t nch = (size_t)c->NP * cdiv(c->NVP, bubble_nb(d.L)) * c->NWP;
@@ -1580,7 +1547,6 @@ int fdga_create(fdga_ctx** out, const fdga_dims* dims) {
             rc |= dalloc(c, &c->seg[r], ns);
             if (d.ref_kind == 1) rc |= dalloc(c, &c->seg[3 + r], nr);
         }
-        rc |= dalloc(c, &c->wtot, (size_t)3 * c->NW2);
     }
     rc |= dalloc(c, &c->sde0, c->nGel);
     rc |= dalloc(c, &c->u2C, (size_t)(4 * d.nG - 1) * c->NkG);
@@ -1628,12 +1594,12 @@ int fdga_destroy(fdga_ctx* c) {
     if (c->st) (void)hipStreamSynchronize(c->st);
     for (double2* p : {c->Gbare, c->G0, c->Sig0, c->G, c->Sig, c->tmpG1, c->tmpG2, c->tmpG3, c->Pi0pp, c->Pi0ph,
                        c->Pipp, c->Piph, c->Wc[0], c->Wc[1], c->Wc[2], c->Lpp, c->Lph, c->tmpL1, c->tmpL2, c->sde0, c->u2C,
-                       c->stage, c->Wfar[0], c->Wfar[1], c->Wfar[2], c->Ptail[0], c->Ptail[1], c->Ptail[2], c->Ptail[3],
+                       c->stage, c->Ptail[0], c->Ptail[1], c->Ptail[2], c->Ptail[3],
                        c->k2x, c->k2xf, c->k2y, c->lk2x, c->pchunk[0], c->pchunk[1], c->pfar})
         if (p) (void)hipFree(p);
     for (auto* t : c->tab) if (t) (void)hipFree(t);
     for (auto* p : c->seg) if (p) (void)hipFree(p);
-    if (c->wtot) (void)hipFree(c->wtot);
+    if (c->wsum) (void)hipFree(c->wsum);
     for (auto* p : c->cache) if (p) (void)hipFree(p);
     for (int r = 0; r < 3; ++r) {
         if (c->R[r]) (void)hipFree(c->R[r]);
@@ -2073,9 +2039,7 @@ int fdga_bse_l_k3(fdga_ctx* c, int32_t ch) {
 
 int fdga_bse_k1(fdga_ctx* c, int32_t ch, int32_t is_mfrg) {
     if (is_mfrg) return launch_form_ch<FORM_K1_MFRG>(c, ch, 1);
-    if (ch == PCH) return launch_k1<PCH>(c);
-    if (ch == TCH) return launch_k1<TCH>(c);
-    if (ch == ACH) return launch_k1<ACH>(c);
+    if (ch >= PCH && ch <= ACH) return launch_k1(c, 1 << ch);
     return fail(c, "bad channel");
 }
 
@@ -2185,12 +2149,11 @@ static int iterate_two_chains(fdga_ctx* c, int32_t strategy, int32_t update_sigm
         rc = launch_lk2_all(c);
         c->seg_fresh = 1;
     }
-    rc = rc ? rc : launch_w_all(c);
+    rc = rc ? rc : launch_w(c, 7);
     c->w_fresh = 1;
-    rc = rc ? rc : launch_k1_all(c);
-    c->tot_fresh = 1;
+    rc = rc ? rc : launch_k1(c, 7);
     rc = rc ? rc : launch_k2_all(c);
-    c->w_fresh = c->seg_fresh = c->tot_fresh = 0;
+    c->w_fresh = c->seg_fresh = 0;
     c->run = c->st;
     if (rc) return -3;
     // chain A on st
@@ -2313,14 +2276,13 @@ static int iterate_eager(fdga_ctx* c, int32_t strategy, int32_t update_sigma, in
     }
     stage_begin(c);
     // the K1/K2 weights depend on Π, Π0, FL and F0 only: computed once for both stages
-    if (launch_w_all(c)) return -3;
+    if (launch_w(c, 7)) return -3;
     c->w_fresh = 1;
-    int rc = launch_k1_all(c);
-    c->tot_fresh = 1;
+    int rc = launch_k1(c, 7);
     stage_end(c, 4);
     stage_begin(c);
     rc = rc ? rc : launch_k2_all(c);
-    c->w_fresh = c->tot_fresh = 0;
+    c->w_fresh = 0;
     if (rc) return -3;
     stage_end(c, 5);
     stage_begin(c);
@@ -2944,13 +2906,12 @@ int group_iterate_eager(fdga_group* g, int strategy, int update_sigma) {
     }
     for (size_t j = 0; j < fused.size(); ++j) {
         fdga_ctx* c = g->m[j];
-        if (launch_w_all(c)) return member_err(g, c);
+        if (launch_w(c, 7)) return member_err(g, c);
         c->w_fresh = 1;
         c->seg_fresh = fd;
-        int rc = launch_k1_all(c);
-        c->tot_fresh = 1;
-        rc = rc ? rc : launch_k2_all(c);
-        c->w_fresh = c->seg_fresh = c->tot_fresh = 0;
+        int rc = launch_k1(c, 7);
+            rc = rc ? rc : launch_k2_all(c);
+        c->w_fresh = c->seg_fresh = 0;
         if (rc) return member_err(g, c);
         if (fused[j]) {
             if (!g->timing && group_bse3(g, c)) return -3;

@@ -10,7 +10,7 @@
 // |ω| <= Wc = NK + |Ω| + |ν| + 2 (NK bounds every box of F, F0 and its tables) X and Y are summed
 // point by point; beyond it neither depends on ω any more (every converted or crossed argument lies
 // outside every box, so only bare vertices and K1/K2 classes at the fixed arguments remain), and the
-// far sums are X_far Σ_far Π + Y_far Σ_far Π0 with the tail sums of Π and Π0 (k_tail_sums layout).
+// far sums are X_far Σ_far Π + Y_far Σ_far Π0 with the sums of Π and Π0 outside the window (tail_left, tail_right).
 #pragma once
 #include "fdga_kernels.h"
 
@@ -24,7 +24,7 @@ struct FormArgs {
     F0V f0;                    // reference vertex
     const double2* Pi;         // Π of the channel [ω, Ω, P]
     const double2* Pi0;        // Π0 of the channel
-    const double2* Pt;         // their tail sums on the band
+    const double2* Pt;         // their sums outside the band (k_tail_sums)
     const double2* P0t;
     double2* out;              // Fbuff.γr.K1 or K2
     const double2* outa;       // Fbuff.γa (the t channel's post-processing reads the finished a channel)
@@ -108,9 +108,11 @@ __device__ __forceinline__ void form_wave(int wid, int lane, const FormArgs& a) 
     si = wave_sum(si);
     double2 acc = cmk(sr, si);
     if (lo > 0)
-        acc = cadd(acc, cadd(cmul(xl, tail_left(a.Pt, row, nVP, a.wb, lo)), cmul(yl, tail_left(a.P0t, row, nVP, a.wb, lo))));
+        acc = cadd(acc, cadd(cmul(xl, tail_left(a.Pt, pi, row, nVP, a.wb, lo, lane)),
+                             cmul(yl, tail_left(a.P0t, pi0, row, nVP, a.wb, lo, lane))));
     if (hi < 2 * nVP - 1)
-        acc = cadd(acc, cadd(cmul(xr, tail_right(a.Pt, row, nVP, a.wb, hi)), cmul(yr, tail_right(a.P0t, row, nVP, a.wb, hi))));
+        acc = cadd(acc, cadd(cmul(xr, tail_right(a.Pt, pi, row, nVP, a.wb, hi, lane)),
+                             cmul(yr, tail_right(a.P0t, pi0, row, nVP, a.wb, hi, lane))));
     const double2 raw = cscale(acc, a.scale);
     int b, e;
     a.sym.range(wid, b, e);

@@ -7,8 +7,7 @@
 //   s-wave averages        k_pavg_multi
 //   build_K3_cache!        k_cache               gather: Γ_irr / F0 / F-base caches
 //   BSE_L_K3!, BSE_K3!     zgemm_tiles<...>      batched complex GEMM on v_mfma_f64_16x16x4f64
-//   BSE_K1!                k_bse_w + k_gemv_k1   gather-GEMV over the bubble mesh (k_bse_w and k_tail_sums keep W
-//                          and the far sums on the band the gathers read)
+//   BSE_K1!                k_k1                  sums over the K2 boxes, the rest from the sums of Π
 //   BSE_K2!, BSE_L_K2!     local solver fdga_local.h; lattice k_k2nl_*, k_lk2nl_table and GEMMs
 //   SDE!                   k_seg_sde (fdga_local.h), k_sde_L_nl, k_sde_L, k_sde_sigma_*, k_u2_*, k_occupation
 #pragma once
@@ -30,6 +29,7 @@ __device__ __forceinline__ double wave_sum(double v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
     return v;
 }
+__device__ __forceinline__ double2 wave_sum2(double2 v) { return cmk(wave_sum(v.x), wave_sum(v.y)); }
 
 // ---------------------------------------------------------------------------------------
 // Symmetry classes of an output array (SymmetryGroup of init_sym_grp!, src/ParquetSolver.jl:203-231).
@@ -2057,139 +2057,85 @@ struct Dense_C {
 // ---------------------------------------------------------------------------------------
 // BSE weight on the bubble mesh for K1/K2 (src/BSEa/BSEa_K1.jl:38-43, BSEa_K2.jl:77-85):
 //   W(ω, Ω, P) = (Π - Π0) F0(Ω, ω~, ∞, Ch, Sp) + Π FL(Ω, ω~, ∞, P, Ch, Sp),  ω~ = crossing(Ω, ω)
-// W is stored on the band of 2 wb frequencies around ω = 0 that the gathers read (iw in
-// [nVP - wb, nVP + wb), row stride 2 wb), and its far sums (the tail layout of k_tail_sums) are
-// formed from the tail sums of Π and Π0: for |ω| > NK + |Ω| + 2 the factors F0(Ω, ω~, ∞) and
-// FL(Ω, ω~, ∞) no longer depend on ω (|ω~| lies beyond every box, so only the bare vertex and the
-// channel's K1(Ω) remain), so Σ_far W = F0_far Σ_far (Π - Π0) + FL_far Σ_far Π.  That holds for the
-// tails the gathers use (lo <= nVP - NK - |Ω| - 2); entries nearer ω = 0 are not used.
-// One thread per band entry and per tail entry of a row (2 wb + 2 per row, rows (Ω, P) in order).
-struct WArgs {   // the arrays of one channel's weight
-    double2* W;      // W on the band [2 wb, rows]
-    double2* far;    // per row: F0 and FL at the left far point, then at the right one [4, rows]
-    const double2* Pi; const double2* Pi0;
-};
-// The tail sums of W are not stored: at row r and tail entry k (the layout of k_tail_sums) they are
-// (Πt - Π0t)·F0_far + Πt·FL_far with the tail sums Πt, Π0t of Π and Π0 and the row's far factors of
-// that side (WTail::at).  One thread per band entry; the row's first also evaluates the far factors.
+// With one argument at infinity only the channel's own classes are left (src/vertex.jl:209-284), K1 and, inside
+// its box, K2 (t: the density component 2 γt - γa): F0(Ω, ω~, ∞) = c0 + K2_0(Ω, ω~) with c0 = U + K1_0(Ω), and
+// FL(Ω, ω~, ∞, P) = kL + K2_L(Ω, ω~, P) with kL = K1_L(Ω, P).
+__device__ __forceinline__ double2 box_k1(const ChanV& g, int m, int p) { return in_b(m, g.n1) ? g.k1(m, p) : czero(); }
+__device__ __forceinline__ double2 box_k2(const ChanV& g, int m, int n, int p) {
+    return in_b(m, g.n2b) && in_f(n, g.n2f) ? g.k2(m, n, p) : czero();
+}
+// the channel's own K1 and K2 in the component its BSE sums (t: 2 γt - γa)
 template <int CH>
-__device__ __forceinline__ void bse_w_elem(size_t e, const WArgs& a, const VtxV& FL, const F0V& f0, int nWP, int nVP,
-                                           int wb, int NK, size_t nrows) {
-    constexpr int ch = CH, sp = ChSpin<CH>::SP;
-    double2* __restrict__ W = a.W;
-    const double2* __restrict__ Pi = a.Pi;
-    const double2* __restrict__ Pi0 = a.Pi0;
-    const int per = 2 * wb;
-    const size_t row = e / per;
-    if (row >= nrows) return;
-    const int t = (int)(e - row * per);
-    const int iW = (int)(row % (size_t)(2 * nWP - 1)), p = (int)(row / (size_t)(2 * nWP - 1));
-    const int m = iW - (nWP - 1);
-    {
-        const int iw = nVP - wb + t, w = iw - nVP;
-        const size_t o = (size_t)iw + (size_t)(2 * nVP) * row;
-        const int wc = crossing(m, w, ch);
-        const double2 f0r = f0.eval(m, wc, FDGA_INF, ch, sp);
-        const double2 flr = FL.eval(m, wc, FDGA_INF, p, ch, sp, FL_ALL);
-        const double2 pi = Pi[o];
-        W[(size_t)t + (size_t)(2 * wb) * row] = cadd(cmul(csub(pi, Pi0[o]), f0r), cmul(pi, flr));
-    }
-    for (int side = t; side < 2; side += per) {   // the row's far factors, one side per thread
-        const int wf = side ? NK + abs(m) + 3 : -(NK + abs(m) + 3);
-        const int wc = crossing(m, wf, ch);
-        a.far[4 * row + 2 * side] = f0.eval(m, wc, FDGA_INF, ch, sp);
-        a.far[4 * row + 2 * side + 1] = FL.eval(m, wc, FDGA_INF, p, ch, sp, FL_ALL);
-    }
+__device__ __forceinline__ double2 own_k1(const ChanV* g, int m, int p) {
+    if (CH == TCH) return csub(cscale(box_k1(g[TCH], m, p), 2.0), box_k1(g[ACH], m, p));
+    return box_k1(g[CH], m, p);
 }
 template <int CH>
-__global__ __launch_bounds__(256) void k_bse_w(WArgs a, VtxV FL, F0V f0, int nWP, int nVP, int wb, int NK, size_t nrows) {
-    bse_w_elem<CH>(blockIdx.x * (size_t)blockDim.x + threadIdx.x, a, FL, f0, nWP, nVP, wb, NK, nrows);
+__device__ __forceinline__ double2 own_k2(const ChanV* g, int m, int n, int p) {
+    if (CH == TCH) return csub(cscale(box_k2(g[TCH], m, n, p), 2.0), box_k2(g[ACH], m, n, p));
+    return box_k2(g[CH], m, n, p);
 }
-// The same weights with one thread per (band entry, Ω) and a chunk of W_PCH momenta: the local
-// reference vertex's factor F0(Ω, ω~, ∞) does not depend on P and is evaluated once for the chunk
-// (the lattice solver; identical values to bse_w_elem).
-constexpr int W_PCH = 8;
 template <int CH>
-__device__ __forceinline__ void bse_w_pchunk(size_t e, const WArgs& a, const VtxV& FL, const F0V& f0, int nWP, int nVP,
-                                             int wb, int NK, int NP) {
-    constexpr int ch = CH, sp = ChSpin<CH>::SP;
-    double2* __restrict__ W = a.W;
-    const double2* __restrict__ Pi = a.Pi;
-    const double2* __restrict__ Pi0 = a.Pi0;
-    const int per = 2 * wb, NWP = 2 * nWP - 1, npc = (NP + W_PCH - 1) / W_PCH;
-    const size_t col = e / per;
-    if (col >= (size_t)NWP * npc) return;
-    const int t = (int)(e - col * per);
-    const int iW = (int)(col % NWP), pc = (int)(col / NWP);
-    const int m = iW - (nWP - 1);
-    const int iw = nVP - wb + t, w = iw - nVP;
-    const int wc = crossing(m, w, ch);
-    const double2 f0r = f0.eval(m, wc, FDGA_INF, ch, sp);
-    const int p0 = pc * W_PCH, p1 = min(p0 + W_PCH, NP);
-#pragma unroll 4
-    for (int p = p0; p < p1; ++p) {
-        const size_t row = (size_t)iW + (size_t)NWP * p;
-        const size_t o = (size_t)iw + (size_t)(2 * nVP) * row;
-        const double2 flr = FL.eval(m, wc, FDGA_INF, p, ch, sp, FL_ALL);
-        const double2 pi = Pi[o];
-        W[(size_t)t + (size_t)(2 * wb) * row] = cadd(cmul(csub(pi, Pi0[o]), f0r), cmul(pi, flr));
-    }
-    // the rows' far factors (F0 and FL at the first ω beyond every box, on each side): one (side,
-    // momentum) pair per thread of the column, so that no thread evaluates them in a chain
-    for (int j = t; j < 2 * W_PCH; j += per) {
-        const int side = j / W_PCH, p = p0 + j % W_PCH;
-        if (p >= p1) continue;
-        const int wf = side ? NK + abs(m) + 3 : -(NK + abs(m) + 3);
-        const int wcf = crossing(m, wf, ch);
-        const size_t row = (size_t)iW + (size_t)NWP * p;
-        a.far[4 * row + 2 * side] = f0.eval(m, wcf, FDGA_INF, ch, sp);
-        a.far[4 * row + 2 * side + 1] = FL.eval(m, wcf, FDGA_INF, p, ch, sp, FL_ALL);
-    }
+__device__ __forceinline__ double2 f0_const(const F0V& f0, int m) {
+    return f0.kind == 1 ? cadd(f0.ref.U, own_k1<CH>(f0.g, m, 0)) : f0.ref.U;
 }
-// the three channels' weights in one launch (nb blocks each, in the order p, t, a); pchunk: one
-// thread per (band entry, Ω, chunk of W_PCH momenta)
-__global__ __launch_bounds__(256) void k_bse_w3(WArgs ap, WArgs at, WArgs aa, VtxV FL, F0V f0, int nWP, int nVP, int wb,
-                                                int NK, size_t nrows, unsigned nb, int pchunk, int NP) {
-    const unsigned ch = blockIdx.x / nb;
-    const size_t e = (blockIdx.x - ch * nb) * (size_t)blockDim.x + threadIdx.x;
-    if (pchunk) {
-        if (ch == 0) bse_w_pchunk<PCH>(e, ap, FL, f0, nWP, nVP, wb, NK, NP);
-        else if (ch == 1) bse_w_pchunk<TCH>(e, at, FL, f0, nWP, nVP, wb, NK, NP);
-        else bse_w_pchunk<ACH>(e, aa, FL, f0, nWP, nVP, wb, NK, NP);
-        return;
-    }
-    if (ch == 0) bse_w_elem<PCH>(e, ap, FL, f0, nWP, nVP, wb, NK, nrows);
-    else if (ch == 1) bse_w_elem<TCH>(e, at, FL, f0, nWP, nVP, wb, NK, nrows);
-    else bse_w_elem<ACH>(e, aa, FL, f0, nWP, nVP, wb, NK, nrows);
+template <int CH>
+__device__ __forceinline__ double2 f0_k2(const F0V& f0, int m, int n) {
+    return f0.kind == 1 ? own_k2<CH>(f0.g, m, n, 0) : czero();
 }
 
-// Tail sums of rows on the bubble ν-mesh (2 nVP entries, ω index iw = ω + nVP), kept on the band
-// of half-width wb around ω = 0 that the gathers can ask for: per row r,
-//   left[i]  = Σ_{k < nVP - wb + i} X[k]    (i = 0 .. wb)
-//   right[j] = Σ_{k >= nVP + j} X[k]        (j = 0 .. wb)
-// stored as T[r * 2 (wb + 1) + i] and T[r * 2 (wb + 1) + wb + 1 + j].
-__device__ __forceinline__ void wave_incl_scan(double& r, double& i, int lane) {
-#pragma unroll
-    for (int o = 1; o < WAVE; o <<= 1) {
-        const double yr = __shfl_up(r, o, WAVE), yi = __shfl_up(i, o, WAVE);
-        if (lane >= o) { r += yr; i += yi; }
+// W of the channels in `mask` (bit ch) on the band |ω| < wb and the rows of the K2 mesh, the only ones that a
+// kernel reads: W[ω + wb + 2 wb (iΩ + Nω2 P)].  One thread per (ω, Ω, chunk of `pch` momenta): F0's part once per
+// chunk, a and t from one load of Πph and Π0ph.  A block takes 32 ω of 8 Ω: Π and W in runs of 512 bytes, and the
+// K2 lines, which hold neighbours in Ω, are shared in the block.  Bound by its reads and writes: L = 16, K2 (32, 32),
+// wb = 131: 141 us (all rows of the mesh and a and t apart: 274), L = 24 (36, 36) 173 us (386).
+struct WArgs {
+    double2* W[3];
+    const double2 *Ppp, *Ppp0, *Pph, *Pph0;
+    ChanV L[3];
+    F0V f0;
+    int n2b, nWP, nVP, wb, NP, mask, pch;
+};
+constexpr int W_PCH = 8;
+__global__ __launch_bounds__(256) void k_bse_w(WArgs a) {
+    const int per = 2 * a.wb, NW2 = 2 * a.n2b - 1, NWP = 2 * a.nWP - 1;
+    const int t = (int)(blockIdx.x * 32 + threadIdx.x % 32), iW = (int)(blockIdx.y * 8 + threadIdx.x / 32);
+    const int p0 = (int)blockIdx.z * a.pch;
+    if (t >= per || iW >= NW2) return;
+    const int m = iW - (a.n2b - 1), w = t - a.wb, wc = crossing(m, w, PCH);
+    const bool dp = a.mask >> PCH & 1, dt = a.mask >> TCH & 1, da = a.mask >> ACH & 1;
+    double2 fp = czero(), ft = czero(), fa = czero();
+    if (dp) fp = cadd(f0_const<PCH>(a.f0, m), f0_k2<PCH>(a.f0, m, wc));
+    if (dt) ft = cadd(f0_const<TCH>(a.f0, m), f0_k2<TCH>(a.f0, m, w));
+    if (da) fa = cadd(f0_const<ACH>(a.f0, m), f0_k2<ACH>(a.f0, m, w));
+    const int p1 = min(p0 + a.pch, a.NP);
+#pragma unroll 2
+    for (int p = p0; p < p1; ++p) {
+        const size_t pi = (size_t)(w + a.nVP) + (size_t)(2 * a.nVP) * ((size_t)(m + a.nWP - 1) + (size_t)NWP * p);
+        const size_t o = (size_t)t + (size_t)per * ((size_t)iW + (size_t)NW2 * p);
+        if (dp) {
+            const double2 P = a.Ppp[pi], d = csub(P, a.Ppp0[pi]);
+            a.W[PCH][o] = cadd(cmul(d, fp), cmul(P, cadd(own_k1<PCH>(a.L, m, p), own_k2<PCH>(a.L, m, wc, p))));
+        }
+        if (dt || da) {
+            const double2 P = a.Pph[pi], d = csub(P, a.Pph0[pi]);
+            if (dt) a.W[TCH][o] = cadd(cmul(d, ft), cmul(P, cadd(own_k1<TCH>(a.L, m, p), own_k2<TCH>(a.L, m, w, p))));
+            if (da) a.W[ACH][o] = cadd(cmul(d, fa), cmul(P, cadd(own_k1<ACH>(a.L, m, p), own_k2<ACH>(a.L, m, w, p))));
+        }
     }
 }
-// One 256-thread block per row.  The parts outside the band are summed with a strided
-// (coalesced) loop and a block reduction; the band is scanned in chunks of 256 entries (wave
-// scans, then the preceding waves' totals), the left side from its outer end inwards and the
-// right side from ω = wb - 1 down to 0.
-__device__ __forceinline__ void tail_sums_row(const double2* __restrict__ X, double2* __restrict__ T, int nVP, int wb,
+
+// Sums of one row (Ω, P) of Π over the bubble mesh: S[3 row + 0, 1, 2] left of the band |ω| < wb, right of it,
+// and over the whole mesh.
+__device__ __forceinline__ void tail_sums_row(const double2* __restrict__ X, double2* __restrict__ S, int nVP, int wb,
                                               size_t nrows, size_t row) {
     constexpr int NWV = 256 / WAVE;
-    __shared__ double sh[4][NWV];
+    __shared__ double2 sh[3][NWV];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid / WAVE;
     if (row >= nrows) return;
     const double2* x = X + row * (size_t)(2 * nVP);
-    double2* tl = T + row * (size_t)(2 * (wb + 1));
-    double2* tr = tl + (wb + 1);
     const int nout = nVP - wb;   // entries of each side outside the band
-    double lr = 0.0, li = 0.0, rr = 0.0, ri = 0.0;
+    double2 l = czero(), r = czero(), c = czero();
     int q = tid;
     for (; q + 3 * 256 < nout; q += 4 * 256) {   // four loads of each side in flight
         double2 a[4], b[4];
@@ -2199,59 +2145,38 @@ __device__ __forceinline__ void tail_sums_row(const double2* __restrict__ X, dou
             b[u] = x[2 * nVP - 1 - q - 256 * u];
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) { lr += a[u].x; li += a[u].y; rr += b[u].x; ri += b[u].y; }
+        for (int u = 0; u < 4; ++u) { l = cadd(l, a[u]); r = cadd(r, b[u]); }
     }
-    for (; q < nout; q += 256) {
-        const double2 a = x[q], b = x[2 * nVP - 1 - q];
-        lr += a.x; li += a.y; rr += b.x; ri += b.y;
-    }
-    lr = wave_sum(lr); li = wave_sum(li); rr = wave_sum(rr); ri = wave_sum(ri);
-    if (lane == 0) { sh[0][wv] = lr; sh[1][wv] = li; sh[2][wv] = rr; sh[3][wv] = ri; }
+    for (; q < nout; q += 256) { l = cadd(l, x[q]); r = cadd(r, x[2 * nVP - 1 - q]); }
+    for (q = nout + tid; q < nVP + wb; q += 256) c = cadd(c, x[q]);
+    l = wave_sum2(l); r = wave_sum2(r); c = wave_sum2(c);
+    if (lane == 0) { sh[0][wv] = l; sh[1][wv] = r; sh[2][wv] = c; }
     __syncthreads();
-    double cl_r = 0.0, cl_i = 0.0, cr_r = 0.0, cr_i = 0.0;   // running sums carried across chunks
-#pragma unroll
-    for (int k = 0; k < NWV; ++k) { cl_r += sh[0][k]; cl_i += sh[1][k]; cr_r += sh[2][k]; cr_i += sh[3][k]; }
-    if (tid == 0) { tl[0] = cmk(cl_r, cl_i); tr[wb] = cmk(cr_r, cr_i); }
-    for (int c0 = 0; c0 < wb; c0 += 256) {
-        __syncthreads();   // sh is reused
-        const int i = c0 + tid;
-        const double2 a = i < wb ? x[nout + i] : czero();
-        const double2 b = i < wb ? x[nVP + wb - 1 - i] : czero();
-        double ar = a.x, ai = a.y, br = b.x, bi = b.y;
-        wave_incl_scan(ar, ai, lane);
-        wave_incl_scan(br, bi, lane);
-        if (lane == WAVE - 1) { sh[0][wv] = ar; sh[1][wv] = ai; sh[2][wv] = br; sh[3][wv] = bi; }
-        __syncthreads();
-        double pl_r = cl_r, pl_i = cl_i, pr_r = cr_r, pr_i = cr_i;
-        for (int k = 0; k < wv; ++k) { pl_r += sh[0][k]; pl_i += sh[1][k]; pr_r += sh[2][k]; pr_i += sh[3][k]; }
-        if (i < wb) {
-            tl[i + 1] = cmk(pl_r + ar, pl_i + ai);
-            tr[wb - 1 - i] = cmk(pr_r + br, pr_i + bi);
-        }
-#pragma unroll
-        for (int k = 0; k < NWV; ++k) { cl_r += sh[0][k]; cl_i += sh[1][k]; cr_r += sh[2][k]; cr_i += sh[3][k]; }
+    if (tid == 0) {
+        for (int k = 1; k < NWV; ++k) { l = cadd(l, sh[0][k]); r = cadd(r, sh[1][k]); c = cadd(c, sh[2][k]); }
+        S[3 * row] = l;
+        S[3 * row + 1] = r;
+        S[3 * row + 2] = cadd(c, cadd(l, r));
     }
 }
-__global__ __launch_bounds__(256) void k_tail_sums(const double2* __restrict__ X, double2* __restrict__ T, int nVP, int wb,
+__global__ __launch_bounds__(256) void k_tail_sums(const double2* __restrict__ X, double2* __restrict__ S, int nVP, int wb,
                                                    size_t nrows) {
-    tail_sums_row(X, T, nVP, wb, nrows, blockIdx.x);
+    tail_sums_row(X, S, nVP, wb, nrows, blockIdx.x);
 }
 // two arrays in one launch (blocks [0, nrows) the first)
-__global__ __launch_bounds__(256) void k_tail_sums2(const double2* __restrict__ X0, double2* __restrict__ T0,
-                                                    const double2* __restrict__ X1, double2* __restrict__ T1, int nVP, int wb,
+__global__ __launch_bounds__(256) void k_tail_sums2(const double2* __restrict__ X0, double2* __restrict__ S0,
+                                                    const double2* __restrict__ X1, double2* __restrict__ S1, int nVP, int wb,
                                                     size_t nrows) {
-    if (blockIdx.x < nrows) tail_sums_row(X0, T0, nVP, wb, nrows, blockIdx.x);
-    else tail_sums_row(X1, T1, nVP, wb, nrows, blockIdx.x - nrows);
+    if (blockIdx.x < nrows) tail_sums_row(X0, S0, nVP, wb, nrows, blockIdx.x);
+    else tail_sums_row(X1, S1, nVP, wb, nrows, blockIdx.x - nrows);
 }
 
 // k_tail_sums for an array whose chunk sums C[P + NP (chunk - ilo + NC iΩ)] over NB consecutive ω
 // were written by the lattice bubble for its NC inner chunks [ilo, ilo + NC), and the sums beyond them
-// (F[side + 2 iΩ], the same at every momentum; null: nothing beyond): the parts outside the band are those,
-// the sums of the inner chunks that lie wholly outside it and the few entries of the chunks it cuts; the band
-// as in k_tail_sums.  Reads NC + 2 wb + O(NB) entries per row instead of 2 nVP.  A block takes the rows of 8
-// consecutive momenta at one Ω: its chunk-sum reads cover whole 128-byte lines (8 momenta per
-// line), the 32 thread groups' partial sums are added in a fixed order, and each wave then scans
-// the band of two rows.
+// (F[side + 2 iΩ], the same at every momentum; null: nothing beyond): of Π itself only the few entries of the
+// chunks that the band cuts are read.  A block takes the rows of 8 consecutive momenta at one Ω: its chunk-sum
+// reads cover whole 128-byte lines (8 momenta per line), and the 32 thread groups' partial sums are added in a
+// fixed order.  L = 16: 48 us (with sums at every ω of the band for windows of all sizes, read from Π: 164).
 constexpr int TAIL_NPB = 8;
 // Both arrays of a bubble (Πpp, Πph) in one launch: blocks [0, nblk) the first, the rest the second.
 __global__ __launch_bounds__(256) void k_tail_sums_chunked(const double2* __restrict__ X0, const double2* __restrict__ C0,
@@ -2259,8 +2184,8 @@ __global__ __launch_bounds__(256) void k_tail_sums_chunked(const double2* __rest
                                                            const double2* __restrict__ C1, double2* __restrict__ T1,
                                                            const double2* __restrict__ F, unsigned nblk, int nVP, int wb,
                                                            int NB, int ilo, int NC, int NWP, int NP) {
-    __shared__ double2 red[2][32][TAIL_NPB + 1];
-    __shared__ double2 far[2][TAIL_NPB];
+    __shared__ double2 red[3][32][TAIL_NPB + 1];
+    __shared__ double2 far[3][TAIL_NPB];
     const bool second = blockIdx.x >= nblk;
     const double2* __restrict__ X = second ? X1 : X0;
     const double2* __restrict__ C = second ? C1 : C0;
@@ -2270,25 +2195,30 @@ __global__ __launch_bounds__(256) void k_tail_sums_chunked(const double2* __rest
     const int iW = (int)(bid % NWP), p0 = (int)(bid / NWP) * TAIL_NPB;
     const int nout = nVP - wb;                 // far left: ω index < nout; far right: >= nVP + wb
     const int cl = nout / NB;                  // chunks [0, cl) lie wholly left of the band
-    const int cr = (nVP + wb + NB - 1) / NB;   // chunks [cr, NC) lie wholly right of it
+    const int cr = (nVP + wb + NB - 1) / NB;   // chunks from cr on lie wholly right of it
     {
         const int pl = tid % TAIL_NPB, cg = tid / TAIL_NPB, p = p0 + pl;
-        double lr = 0.0, li = 0.0, rr = 0.0, ri = 0.0;
+        double2 l = czero(), r = czero(), c = czero();
         if (p < NP) {
             const double2* cp = C + (size_t)p + (size_t)NP * (size_t)NC * iW;
-            for (int c = cg; c < cl - ilo; c += 32) { const double2 v = cp[(size_t)NP * c]; lr += v.x; li += v.y; }
-            for (int c = cr - ilo + cg; c < NC; c += 32) { const double2 v = cp[(size_t)NP * c]; rr += v.x; ri += v.y; }
+            for (int q = cg; q < NC; q += 32) {
+                const double2 v = cp[(size_t)NP * q];
+                if (q < cl - ilo) l = cadd(l, v);
+                else if (q >= cr - ilo) r = cadd(r, v);
+                else c = cadd(c, v);
+            }
         }
-        red[0][cg][pl] = cmk(lr, li);
-        red[1][cg][pl] = cmk(rr, ri);
+        red[0][cg][pl] = l;
+        red[1][cg][pl] = r;
+        red[2][cg][pl] = c;
     }
     __syncthreads();
-    if (tid < 2 * TAIL_NPB) {
-        const int side = tid / TAIL_NPB, pl = tid % TAIL_NPB;
-        double sr = 0.0, si = 0.0;
-        for (int g = 0; g < 32; ++g) { sr += red[side][g][pl].x; si += red[side][g][pl].y; }
-        if (F) { const double2 f = F[side + 2 * (iW + (second ? NWP : 0))]; sr += f.x; si += f.y; }
-        far[side][pl] = cmk(sr, si);
+    if (tid < 3 * TAIL_NPB) {
+        const int part = tid / TAIL_NPB, pl = tid % TAIL_NPB;
+        double2 s = czero();
+        for (int g = 0; g < 32; ++g) s = cadd(s, red[part][g][pl]);
+        if (F && part < 2) s = cadd(s, F[part + 2 * (iW + (second ? NWP : 0))]);
+        far[part][pl] = s;
     }
     __syncthreads();
     for (int pl = wv; pl < TAIL_NPB; pl += 256 / WAVE) {
@@ -2296,56 +2226,31 @@ __global__ __launch_bounds__(256) void k_tail_sums_chunked(const double2* __rest
         if (p >= NP) break;
         const size_t row = (size_t)iW + (size_t)NWP * p;
         const double2* x = X + row * (size_t)(2 * nVP);
-        double2* tl = T + row * (size_t)(2 * (wb + 1));
-        double2* tr = tl + (wb + 1);
         // the entries of the two cut chunks that lie outside the band
-        double lr = 0.0, li = 0.0, rr = 0.0, ri = 0.0;
-        for (int k = cl * NB + lane; k < nout; k += WAVE) { const double2 v = x[k]; lr += v.x; li += v.y; }
-        for (int k = nVP + wb + lane; k < min(cr * NB, 2 * nVP); k += WAVE) { const double2 v = x[k]; rr += v.x; ri += v.y; }
-        double cl_r = far[0][pl].x + wave_sum(lr), cl_i = far[0][pl].y + wave_sum(li);
-        double cr_r = far[1][pl].x + wave_sum(rr), cr_i = far[1][pl].y + wave_sum(ri);
-        if (lane == 0) { tl[0] = cmk(cl_r, cl_i); tr[wb] = cmk(cr_r, cr_i); }
-        // the band: left from its outer end inwards, right from ω = wb - 1 down to 0
-        for (int c0 = 0; c0 < wb; c0 += WAVE) {
-            const int i = c0 + lane;
-            const double2 a = i < wb ? x[nout + i] : czero();
-            const double2 b = i < wb ? x[nVP + wb - 1 - i] : czero();
-            double ar = a.x, ai = a.y, br = b.x, bi = b.y;
-            wave_incl_scan(ar, ai, lane);
-            wave_incl_scan(br, bi, lane);
-            if (i < wb) {
-                tl[i + 1] = cmk(cl_r + ar, cl_i + ai);
-                tr[wb - 1 - i] = cmk(cr_r + br, cr_i + bi);
-            }
-            cl_r += __shfl(ar, WAVE - 1, WAVE); cl_i += __shfl(ai, WAVE - 1, WAVE);
-            cr_r += __shfl(br, WAVE - 1, WAVE); cr_i += __shfl(bi, WAVE - 1, WAVE);
+        double2 l = czero(), r = czero();
+        for (int k = cl * NB + lane; k < nout; k += WAVE) l = cadd(l, x[k]);
+        for (int k = nVP + wb + lane; k < min(cr * NB, 2 * nVP); k += WAVE) r = cadd(r, x[k]);
+        l = wave_sum2(l);
+        r = wave_sum2(r);
+        if (lane == 0) {
+            T[3 * row] = cadd(far[0][pl], l);
+            T[3 * row + 1] = cadd(far[1][pl], r);
+            T[3 * row + 2] = cadd(far[2][pl], cadd(far[0][pl], far[1][pl]));
         }
     }
 }
-// far sums of one row outside the window [lo, hi]: Σ_{k < lo} and Σ_{k > hi}
-// (nVP - wb <= lo <= nVP < hi + 1 <= nVP + wb)
-__device__ __forceinline__ double2 tail_left(const double2* T, size_t row, int nVP, int wb, int lo) {
-    return T[row * (size_t)(2 * (wb + 1)) + (lo - (nVP - wb))];
+// Σ of a row x of Π (one wave) left of the window's first index lo and right of its last one hi, from the sums S
+// outside the band and the band's entries outside the window (nVP - wb <= lo <= nVP < hi + 1 <= nVP + wb)
+__device__ __forceinline__ double2 tail_left(const double2* S, const double2* x, size_t row, int nVP, int wb, int lo, int lane) {
+    double2 s = czero();
+    for (int k = nVP - wb + lane; k < lo; k += WAVE) s = cadd(s, x[k]);
+    return cadd(S[3 * row], wave_sum2(s));
 }
-__device__ __forceinline__ double2 tail_right(const double2* T, size_t row, int nVP, int wb, int hi) {
-    return T[row * (size_t)(2 * (wb + 1)) + (wb + 1) + (hi + 1 - nVP)];
+__device__ __forceinline__ double2 tail_right(const double2* S, const double2* x, size_t row, int nVP, int wb, int hi, int lane) {
+    double2 s = czero();
+    for (int k = hi + 1 + lane; k < nVP + wb; k += WAVE) s = cadd(s, x[k]);
+    return cadd(S[3 * row + 1], wave_sum2(s));
 }
-// tail sums of a BSE weight W = (Π - Π0) F0 + Π FL, formed from the tail sums of Π and Π0 and the
-// row's far factors (k_bse_w): Σ_far W = F0_far Σ_far (Π - Π0) + FL_far Σ_far Π
-struct WTail {
-    const double2* Pt; const double2* P0t; const double2* far;
-    __device__ __forceinline__ double2 at(size_t row, int k, int wb) const {   // entry k of the row's tail layout
-        const size_t o = row * (size_t)(2 * (wb + 1)) + k;
-        const int side = k > wb ? 1 : 0;
-        const double2 pt = Pt[o];
-        return cadd(cmul(csub(pt, P0t[o]), far[4 * row + 2 * side]), cmul(pt, far[4 * row + 2 * side + 1]));
-    }
-    __device__ __forceinline__ double2 left(size_t row, int nVP, int wb, int lo) const { return at(row, lo - (nVP - wb), wb); }
-    __device__ __forceinline__ double2 right(size_t row, int nVP, int wb, int hi) const {
-        return at(row, (wb + 1) + (hi + 1 - nVP), wb);
-    }
-};
-
 // Frequency window of the gather-GEMVs.  Every vertex term that depends on the summed
 // frequency ω is supported on |ω| <= Wc = NK + |m| + |n| + 2, where NK bounds every box of the
 // vertex (K1 boxes reach furthest: their bosonic argument is a sum or difference of Ω, ν, ω).
@@ -2360,58 +2265,129 @@ __device__ __forceinline__ void far_pair(double2 t, double2& left, double2& righ
     right = cmk(__shfl(t.x, 1, WAVE), __shfl(t.y, 1, WAVE));
 }
 
-// BSE_K1!: K1(Ω, P) = T s Σ_ω F(Ω, ∞, ω, P, Ch, Sp) W(ω).  One 256-thread block per output
-// class (the K1 mesh has few outputs; four waves per output shorten each one's chain of gathers).
-template <int CH>
-__device__ __forceinline__ void gemv_k1_block(int wid, double2* __restrict__ K1, const double2* __restrict__ K1a,
-                                              const double2* __restrict__ W, const WTail& Wtail,
-                                              const VtxV& F, int n1, int nWP, int nVP, int wb, int NP, double scale, int NK,
-                                              const SymCls& sym) {
-    constexpr int SP = ChSpin<CH>::SP;
-    constexpr int NT = 256;
-    __shared__ double red[NT / WAVE][2];
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid / WAVE;
-    const int NW1 = 2 * n1 - 1;
-    if (wid >= sym.count(NW1 * NP)) return;
-    const int o0 = sym.rep(wid);
-    const int iW = o0 % NW1, p = o0 / NW1;
-    const int m = iW - (n1 - 1);
-    const int Wc = window(NK, m, 0);
-    const size_t row = (size_t)(m + nWP - 1) + (size_t)(2 * nWP - 1) * p;
-    const double2* Wr = W + (size_t)(2 * wb) * row + wb;   // Wr[ω], |ω| within the band
-    const int lo = max(0, nVP - Wc), hi = min(2 * nVP - 1, nVP + Wc);
-    double sr = 0.0, si = 0.0;
-    for (int iw = lo + tid; iw <= hi; iw += NT) {
-        double2 x = cmul(F.eval(m, FDGA_INF, iw - nVP, p, CH, SP, FL_ALL), Wr[iw - nVP]);
-        sr += x.x; si += x.y;
+// BSE_K1!: K1(Ω, P) = T s Σ_ω F(Ω, ∞, ω, P, Ch, Sp) W(ω), and the sums of W that BSE_K2! takes.  F(Ω, ∞, ω) holds
+// the channel's own classes only (as F0 and FL in W), c0 + K1(Ω, P) + K2_0(Ω, ω) + K2(Ω, ω, P), so that
+//   Σ W = c0 (ΣΠ - ΣΠ0) + kL ΣΠ + Σ_ω x(ω),   x(ω) = (Π - Π0) K2_0(Ω, ω~) + Π K2_L(Ω, ω~, P)
+//   K1  = T s [(c0 + K1(Ω, P)) ΣW + Σ_ω (K2_0(Ω, ω) + K2(Ω, ω, P)) W(ω)]
+// with sums over the K2 boxes alone and ΣΠ from the tail sums; W(ω) is formed in place.  Two waves per class of
+// (Ω, P), one for p and one for a and t (one load of Π and of each K2 for both), lanes over ω; without groups they also store Σ W left and right of the
+// band and in all for the rows of the K2 mesh, ws[iΩ + Nω2 (P + NP (part + 3 ch))], under groups the waves after
+// the nk classes do.  Each XCD takes a range of classes of its own: neighbours in Ω share the lines of K2.
+// Bound by the address rate of the K2 loads (Ω is fastest there, a line per lane).  L = 16, nΩ = 64, K2 (32, 32):
+// 119 us for the three channels (F evaluated at every ω of the window, two launches: 333); L = 24, 72, (36, 36):
+// 235 us (503).  Blocks of 8 neighbours in Ω of one kind measured 286 against 160 us, a and t apart 160 to 119.
+struct K1Args {
+    VtxV F;
+    ChanV L[3];
+    const double2 *Ppp, *Ppp0, *Pph, *Pph0;      // Π, Π0 and their sums
+    const double2 *Spp, *Spp0, *Sph, *Sph0;
+    double2 *Kp, *Kt, *Ka, *ws;
+    int n1, n2b, nWP, nVP, NP, mask;             // mask: channels (bit ch)
+    double T;
+    SymCls sym;
+    int nk, ntot;
+};
+struct K1Row { double2 raw, l, r, tot; };
+// o: p, or a and then t
+template <bool PH>
+__device__ __forceinline__ void k1_row(const K1Args& a, int m, int p, int lane, K1Row& oa, K1Row& ot) {
+    const size_t row = (size_t)(m + a.nWP - 1) + (size_t)(2 * a.nWP - 1) * p;
+    const double2* pi = (PH ? a.Pph : a.Ppp) + (size_t)(2 * a.nVP) * row + a.nVP;
+    const double2* pi0 = (PH ? a.Pph0 : a.Ppp0) + (size_t)(2 * a.nVP) * row + a.nVP;
+    const double2* S = (PH ? a.Sph : a.Spp) + 3 * row;
+    const double2* S0 = (PH ? a.Sph0 : a.Spp0) + 3 * row;
+    const F0V& f0 = a.F.f0;
+    constexpr int C = PH ? ACH : PCH;
+    const double2 c0 = f0_const<C>(f0, m), kL = own_k1<C>(a.L, m, p);
+    double2 c0t = czero(), kLt = czero(), tot = czero(), k = czero(), tott = czero(), kt = czero();
+    if (PH) { c0t = f0_const<TCH>(f0, m); kLt = own_k1<TCH>(a.L, m, p); }
+    int nf = max(a.L[C].n2f, a.F.g[C].n2f), nb = max(a.L[C].n2b, a.F.g[C].n2b);
+    if (f0.kind == 1) { nf = max(nf, f0.g[C].n2f); nb = max(nb, f0.g[C].n2b); }
+    if (in_b(m, nb)) {
+        // ω or ω~ in a box, on the mesh
+        const int lo = max(-a.nVP, PH ? -nf : min(0, m) - nf), hi = min(a.nVP, PH ? nf : max(0, m) + nf);
+        for (int w = lo + lane; w < hi; w += WAVE) {
+            const int wc = PH ? w : crossing(m, w, PCH);
+            const double2 P = pi[w], d = csub(P, pi0[w]);
+            const double2 l = box_k2(a.L[C], m, wc, p), f = box_k2(a.F.g[C], m, w, p);
+            double2 gc = czero(), gw = czero();
+            if (f0.kind == 1) {
+                gc = box_k2(f0.g[C], m, wc, 0);
+                gw = PH ? gc : box_k2(f0.g[C], m, w, 0);
+            }
+            const double2 x = cadd(cmul(d, gc), cmul(P, l));
+            tot = cadd(tot, x);
+            k = cadd(k, cmul(cadd(gw, f), cadd(x, cadd(cmul(d, c0), cmul(P, kL)))));
+            if (PH) {
+                const double2 lt = csub(cscale(box_k2(a.L[TCH], m, w, p), 2.0), l);
+                const double2 ft = csub(cscale(box_k2(a.F.g[TCH], m, w, p), 2.0), f);
+                const double2 gt = f0.kind == 1 ? csub(cscale(box_k2(f0.g[TCH], m, w, 0), 2.0), gc) : czero();
+                const double2 xt = cadd(cmul(d, gt), cmul(P, lt));
+                tott = cadd(tott, xt);
+                kt = cadd(kt, cmul(cadd(gt, ft), cadd(xt, cadd(cmul(d, c0t), cmul(P, kLt)))));
+            }
+        }
     }
-    sr = wave_sum(sr); si = wave_sum(si);
-    if (lane == 0) { red[wv][0] = sr; red[wv][1] = si; }
-    __syncthreads();
-    if (wv != 0) return;
-    const double tsr = red[0][0] + red[1][0] + red[2][0] + red[3][0];
-    const double tsi = red[0][1] + red[1][1] + red[2][1] + red[3][1];
-    double2 tl, tr;
-    far_pair(F.eval(m, FDGA_INF, lane == 0 ? -Wc - 1 : Wc + 1, p, CH, SP, FL_ALL), tl, tr);
-    // every lane of wave 0 holds the same sums; lanes write the class members
-    double2 acc = cmk(tsr, tsi);
-    if (lo > 0) acc = cadd(acc, cmul(tl, Wtail.left(row, nVP, wb, lo)));
-    if (hi < 2 * nVP - 1) acc = cadd(acc, cmul(tr, Wtail.right(row, nVP, wb, hi)));
-    const double2 raw = cscale(acc, scale);
-    int b, e;
-    sym.range(wid, b, e);
-    for (int k = b + lane; k < e; k += WAVE) {
-        const int code = sym.member(wid, k), o = code >> 2;
-        double2 v = sym_apply(code & 3, raw);
-        if (CH == TCH) v = cscale(cadd(v, K1a[o]), 0.5);
-        K1[o] = v;
+    auto finish = [&](K1Row& o, double2 c, double2 kl, double2 sum, double2 kk, double2 k1, double sc) {
+        auto far = [&](int q) { return cadd(cmul(csub(S[q], S0[q]), c), cmul(S[q], kl)); };
+        o.l = far(0);
+        o.r = far(1);
+        o.tot = cadd(wave_sum2(sum), far(2));
+        o.raw = cscale(cadd(cmul(cadd(c, k1), o.tot), wave_sum2(kk)), sc);
+    };
+    finish(oa, c0, kL, tot, k, own_k1<C>(a.F.g, m, p), a.T);
+    if (PH) finish(ot, c0t, kLt, tott, kt, own_k1<TCH>(a.F.g, m, p), -a.T);
+}
+__device__ __forceinline__ void k1_store(const K1Args& a, int ch, int m, int p, const K1Row o, int lane) {
+    const size_t NW2 = 2 * a.n2b - 1, nq = NW2 * a.NP;
+    double2* w = a.ws + (size_t)(m + a.n2b - 1) + NW2 * (size_t)p + nq * (3 * ch);
+    if (lane == 0) {
+        w[0] = o.l;
+        w[nq] = o.r;
+        w[2 * nq] = o.tot;
     }
 }
-template <int CH>
-__global__ __launch_bounds__(256) void k_gemv_k1(double2* __restrict__ K1, const double2* __restrict__ K1a,
-                                                 const double2* __restrict__ W, WTail Wtail, VtxV F,
-                                                 int n1, int nWP, int nVP, int wb, int NP, double scale, int NK, SymCls sym) {
-    gemv_k1_block<CH>(blockIdx.x, K1, K1a, W, Wtail, F, n1, nWP, nVP, wb, NP, scale, NK, sym);
+__global__ __launch_bounds__(256) void k_k1(K1Args a) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int blk = (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8);
+    const int wid = blk * (256 / WAVE) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
+    const bool pw = wid & 1;
+    const int cls = wid >> 1;
+    if (cls >= a.nk + a.ntot) return;
+    if (pw ? !(a.mask >> PCH & 1) : !(a.mask & (1 << ACH | 1 << TCH))) return;
+    int m, p, b = 0, e = 0;
+    const bool sums = cls >= a.nk;   // the sums alone
+    if (sums) {
+        const int NW2 = 2 * a.n2b - 1;
+        m = (cls - a.nk) % NW2 - (a.n2b - 1);
+        p = (cls - a.nk) / NW2;
+    } else {
+        const int NW1 = 2 * a.n1 - 1, o0 = a.sym.rep(cls);
+        m = o0 % NW1 - (a.n1 - 1);
+        p = o0 / NW1;
+        a.sym.range(cls, b, e);
+    }
+    const bool st = sums || (!a.sym.ncls && in_b(m, a.n2b));
+    K1Row ra{}, rt{};
+    if (pw) {
+        k1_row<false>(a, m, p, lane, ra, rt);
+        if (st) k1_store(a, PCH, m, p, ra, lane);
+        for (int k = b + lane; k < e; k += WAVE) {
+            const int code = a.sym.member(cls, k);
+            a.Kp[code >> 2] = sym_apply(code & 3, ra.raw);
+        }
+        return;
+    }
+    k1_row<true>(a, m, p, lane, ra, rt);
+    const bool ma = a.mask >> ACH & 1, mt = a.mask >> TCH & 1;
+    if (st && ma) k1_store(a, ACH, m, p, ra, lane);
+    if (st && mt) k1_store(a, TCH, m, p, rt, lane);
+    for (int k = b + lane; k < e; k += WAVE) {
+        const int code = a.sym.member(cls, k), o = code >> 2;
+        const double2 ka = ma ? sym_apply(code & 3, ra.raw) : a.Ka[o];
+        if (ma) a.Ka[o] = ka;
+        if (mt) a.Kt[o] = cscale(cadd(sym_apply(code & 3, rt.raw), ka), 0.5);   // src/BSE_templates.jl:29-33
+    }
 }
 
 // BSE_K2!: K2(Ω, ν, P) = T s Σ_ω [F(Ω,ν,ω) - F(Ω,∞,ω)] W(ω) + FL.K2 (t: 2 FLt - FLa).
@@ -2533,21 +2509,15 @@ __device__ __forceinline__ double2 k2_add_fl(double2 val, double2 lr, double2 la
 template <int CH>
 __global__ __launch_bounds__(256) void k_k2nl_finish(double2* __restrict__ K2, const double2* __restrict__ K2a,
                                                      const double2* __restrict__ Y, const double2* __restrict__ Xf,
-                                                     const double2* __restrict__ W, WTail Wtail,
-                                                     VtxV F, ChanV Lr, ChanV La, int n2b, int n2f, int nWP, int wb,
-                                                     int NP, double scale, double2* __restrict__ raw) {
+                                                     const double2* __restrict__ ws, VtxV F, ChanV Lr, ChanV La, int n2b,
+                                                     int n2f, int NP, double scale, double2* __restrict__ raw) {
     const int wid = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
     const int NW2 = 2 * n2b - 1, NV2 = 2 * n2f;
     if (wid >= NW2 * NP) return;
     const int iW = wid % NW2, p = wid / NW2;
     const int m = iW - (n2b - 1);
-    const size_t row = (size_t)(m + nWP - 1) + (size_t)(2 * nWP - 1) * p;
-    const double2* Wr = W + (size_t)(2 * wb) * row + wb;   // Wr[ω], ω in [-wb, wb)
-    const double2 wl = Wtail.at(row, 0, wb), wr = Wtail.at(row, (wb + 1) + wb, wb);   // issued first
-    double sr = 0.0, si = 0.0;
-    for (int k = lane; k < 2 * wb; k += WAVE) { const double2 x = Wr[k - wb]; sr += x.x; si += x.y; }
-    sr = wave_sum(sr); si = wave_sum(si);
-    const double2 wtot = cadd(cmk(sr, si), cadd(wl, wr));
+    const size_t q = (size_t)iW + (size_t)NW2 * p, nq = (size_t)NW2 * NP;
+    const double2 wl = ws[q], wr = ws[q + nq], wtot = ws[q + 2 * nq];
     for (int iv = lane; iv < NV2; iv += WAVE) {
         const int v = iv - n2f;
         double2 acc = Y[(size_t)iv + (size_t)NV2 * (iW + (size_t)NW2 * p)];
@@ -2565,7 +2535,7 @@ __global__ __launch_bounds__(256) void k_k2nl_finish(double2* __restrict__ K2, c
 // One wave per (Ω, P) as the finish, lanes over ν; K32: F.K3 held in FP32.
 template <int CH, bool K32>
 __global__ __launch_bounds__(256) void k_k2nl_k3(double2* __restrict__ out, const double2* __restrict__ W, VtxV F,
-                                                 int n2b, int n2f, int nWP, int wb, int NP, double f) {
+                                                 int n2b, int n2f, int wb, int NP, double f) {
     const int wid = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
     const int NW2 = 2 * n2b - 1, NV2 = 2 * n2f;
     if (wid >= NW2 * NP) return;
@@ -2573,8 +2543,7 @@ __global__ __launch_bounds__(256) void k_k2nl_k3(double2* __restrict__ out, cons
     const int m = iW - (n2b - 1);
     const ChanV& g = F.g[CH];
     if (!in_b(m, g.n3b)) return;
-    const size_t row = (size_t)(m + nWP - 1) + (size_t)(2 * nWP - 1) * p;
-    const double2* Wr = W + (size_t)(2 * wb) * row + wb;   // Wr[ω], ω in [-wb, wb)
+    const double2* Wr = W + (size_t)(2 * wb) * wid + wb;   // Wr[ω], ω in [-wb, wb)
     for (int iv = lane; iv < NV2; iv += WAVE) {
         const int v = iv - n2f;
         if (!in_f(v, g.n3f)) continue;
@@ -2644,12 +2613,12 @@ __device__ __forceinline__ void sde_L_wave(int wid, int lane, double2* __restric
     ar = wave_sum(ar); ai = wave_sum(ai); br = wave_sum(br); bi = wave_sum(bi);
     double2 A = cmk(ar, ai), B = cmk(br, bi);
     if (lo > 0) {
-        if (DP) A = cadd(A, cmul(tail_left(Tpp, row, nVP, wb, lo), xpl));
-        if (DH) B = cadd(B, cmul(tail_left(Tph, row, nVP, wb, lo), xhl));
+        if (DP) A = cadd(A, cmul(tail_left(Tpp, Pipp + base, row, nVP, wb, lo, lane), xpl));
+        if (DH) B = cadd(B, cmul(tail_left(Tph, Piph + base, row, nVP, wb, lo, lane), xhl));
     }
     if (hi < 2 * nVP - 1) {
-        if (DP) A = cadd(A, cmul(tail_right(Tpp, row, nVP, wb, hi), xpr));
-        if (DH) B = cadd(B, cmul(tail_right(Tph, row, nVP, wb, hi), xhr));
+        if (DP) A = cadd(A, cmul(tail_right(Tpp, Pipp + base, row, nVP, wb, hi, lane), xpr));
+        if (DH) B = cadd(B, cmul(tail_right(Tph, Piph + base, row, nVP, wb, hi, lane), xhr));
     }
     const double2 rawp = cmul(A, TU), rawh = cmul(B, TU);
     int b, e;
@@ -2845,7 +2814,7 @@ __global__ __launch_bounds__(256) void k_sde_L_nl(double2* __restrict__ Lpp, dou
                                                   const double2* __restrict__ Pipp, const double2* __restrict__ Piph,
                                                   const double2* __restrict__ Tpp, const double2* __restrict__ Tph,
                                                   SdeLevelNL lv0, SdeLevelNL lv1, int n2b, int n2f, int nWP, int nVP,
-                                                  int wb, int NP, double2 TU) {
+                                                  int NP, double2 TU) {
     __shared__ double2 wsm[SDE_W], red[2 * 256], k2s[2][NLEV];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid / WAVE;
     const int NW2 = 2 * n2b - 1, NV2 = 2 * n2f;
@@ -2855,10 +2824,7 @@ __global__ __launch_bounds__(256) void k_sde_L_nl(double2* __restrict__ Lpp, dou
     const double2* ph = Piph + (size_t)(2 * nVP) * row + nVP;
     auto wpp = [&](int n) { return m - n - 1 >= -nVP && m - n - 1 < nVP ? pp[m - n - 1] : czero(); };
     auto wph = [&](int n) { return n >= -nVP && n < nVP ? ph[n] : czero(); };
-    // ΣΠ over the bubble mesh from the tail sums on both sides of ω = 0
-    const double2* tp = Tpp + (size_t)(2 * (wb + 1)) * row + wb;
-    const double2* th = Tph + (size_t)(2 * (wb + 1)) * row + wb;
-    const double2 spp = cadd(tp[0], tp[1]), sph = cadd(th[0], th[1]);
+    const double2 spp = Tpp[3 * row + 2], sph = Tph[3 * row + 2];   // ΣΠ over the bubble mesh
     // the ν-independent K2 sums: wave 2 l + 0 the p channel's of level l, wave 2 l + 1 those of a and t
     if (wv < 2 * NLEV) {
         const int l = wv >> 1;

@@ -41,7 +41,7 @@ struct SegPrep {
     unsigned wblk;           // first block of the weights, per channel
     unsigned wper;
     F0V f0;
-    int nWP, nVP, wb;
+    int n2b, nWP, nVP, wb;
 };
 __global__ __launch_bounds__(256) void k_seg_prep(SegPrep a) {
     if (blockIdx.x < a.wblk) {
@@ -58,13 +58,13 @@ __global__ __launch_bounds__(256) void k_seg_prep(SegPrep a) {
     const unsigned q = blockIdx.x - a.wblk;
     const int k = (int)(q / a.wper);
     const size_t e = (size_t)(q - k * a.wper) * 256 + threadIdx.x;
-    const int per = 2 * a.wb, NWP = 2 * a.nWP - 1;
-    if (e >= (size_t)per * NWP) return;
-    const int t = (int)(e % per), iW = (int)(e / per), m = iW - (a.nWP - 1), w = t - a.wb, ch = a.wch[k];
+    const int per = 2 * a.wb, NW2 = 2 * a.n2b - 1;
+    if (e >= (size_t)per * NW2) return;
+    const int t = (int)(e % per), m = (int)(e / per) - (a.n2b - 1), w = t - a.wb, ch = a.wch[k];
     const double2 f = ch == PCH ? a.f0.eval(m, bmf(m, w), FDGA_INF, PCH, PSP)
                       : ch == TCH ? a.f0.eval(m, w, FDGA_INF, TCH, DSP)
                                   : a.f0.eval(m, w, FDGA_INF, ACH, PSP);
-    a.W[k][e] = cmul(a.Pi0[k][(size_t)(w + a.nVP) + (size_t)(2 * a.nVP) * iW], f);
+    a.W[k][e] = cmul(a.Pi0[k][(size_t)(w + a.nVP) + (size_t)(2 * a.nVP) * (m + a.nWP - 1)], f);
 }
 
 // the wave's number in its block, in a scalar register: a class's bounds and base are the same for all lanes,
@@ -131,10 +131,10 @@ struct SegK2 {
     SegVtx F, F0;                // F0: REF, the local Vertex of the reference system (BSE_K2! only)
     RefV ref;
     const double2 *Wp, *Wt, *Wa; // weights on the band
-    const double2* tot;          // their totals (BSE_K2!)
+    const double2* ws;           // their sums over the mesh (BSE_K2!; the layout of K1Args)
     const double2 *Lp, *Lt, *La; // FL.K2 (BSE_K2!)
     double2 *Kp, *Kt, *Ka;       // results
-    int n2b, n2f, nWP, nVP, wb;
+    int n2b, n2f, wb;
     double T;
     SymCls sp, sat;
     int np, nat;                 // classes of the p channel, and of the a and t channels
@@ -174,53 +174,6 @@ __device__ __forceinline__ double2 seg_const(const SegK2& A, int m, int v) {
     }
     return x;
 }
-__device__ __forceinline__ double2 wave_sum2(double2 v) { return cmk(wave_sum(v.x), wave_sum(v.y)); }
-// one wave per (channel, Ω of the K2 box): Σ_ω W over the whole mesh, the band and the tails beyond it
-struct SegTot {
-    const double2* W[3];
-    WTail T[3];
-    double2* out;            // [Ω, channel]
-    int n2b, nWP, wb;
-};
-__device__ __forceinline__ void seg_tot(const SegTot& A, int wid, int lane) {
-    const int NW2 = 2 * A.n2b - 1;
-    if (wid >= 3 * NW2) return;
-    const int ch = wid / NW2;
-    const size_t row = (size_t)(wid % NW2 - A.n2b + A.nWP);
-    auto total = [&](const double2* W, const WTail& t) {
-        const double2* Wr = W + (size_t)(2 * A.wb) * row;
-        double2 s = czero();
-        for (int w = lane; w < 2 * A.wb; w += WAVE) s = cadd(s, Wr[w]);
-        s = cadd(wave_sum2(s), cadd(t.at(row, 0, A.wb), t.at(row, 2 * A.wb + 1, A.wb)));
-        if (lane == 0) A.out[wid] = s;
-    };
-    if (ch == PCH) total(A.W[PCH], A.T[PCH]);
-    else if (ch == TCH) total(A.W[TCH], A.T[TCH]);
-    else total(A.W[ACH], A.T[ACH]);
-}
-__global__ __launch_bounds__(256) void k_seg_tot(SegTot A) {
-    seg_tot(A, (int)((blockIdx.x * 256 + threadIdx.x) / WAVE), threadIdx.x & (WAVE - 1));
-}
-
-// BSE_K1! of the three channels in one launch (t from the a channel of the same block), and for the local solver the weight
-// totals that BSE_K2! takes: blocks [0, nb) a and t, [nb, 2 nb) p, the rest the totals
-__global__ __launch_bounds__(256) void k_k1_all(double2* __restrict__ K1p, double2* __restrict__ K1a, double2* __restrict__ K1t,
-                                                const double2* __restrict__ Wp, const double2* __restrict__ Wa,
-                                                const double2* __restrict__ Wt, WTail Tp, WTail Ta, WTail Tt, VtxV F, int n1,
-                                                int nWP, int nVP, int wb, int NP, double T, int NK, SymCls sym, int nb,
-                                                SegTot tot) {
-    const int b = (int)blockIdx.x;
-    if (b < nb) {
-        gemv_k1_block<ACH>(b, K1a, nullptr, Wa, Ta, F, n1, nWP, nVP, wb, NP, T, NK, sym);
-        __syncthreads();   // the block's partial sums are read before the t channel's replace them
-        gemv_k1_block<TCH>(b, K1t, K1a, Wt, Tt, F, n1, nWP, nVP, wb, NP, -T, NK, sym);
-    } else if (b < 2 * nb) {
-        gemv_k1_block<PCH>(b - nb, K1p, nullptr, Wp, Tp, F, n1, nWP, nVP, wb, NP, T, NK, sym);
-    } else {
-        seg_tot(tot, (b - 2 * nb) * (256 / WAVE) + (int)threadIdx.x / WAVE, threadIdx.x & (WAVE - 1));
-    }
-}
-
 constexpr int SEG_NT = 512;
 // One wave per output class, lanes over ω.  The t channel is summed in the density component 2 F(t) - F(a)
 // next to the a channel, whose terms both share.
@@ -239,7 +192,7 @@ __global__ __launch_bounds__(SEG_NT) void k_seg_k2(SegK2 A) {
     const SymCls& sym = pw ? A.sp : A.sat;
     const int NV2 = 2 * A.n2f, cls = sym.ncls ? wid : wid / NV2 + (2 * A.n2b - 1) * (wid % NV2), o0 = sym.rep(cls);
     const int NW2 = 2 * A.n2b - 1, iW = o0 % NW2, iv = o0 / NW2, m = iW - (A.n2b - 1), v = iv - A.n2f;
-    const size_t row = (size_t)(m + A.nWP - 1), ro = (size_t)(2 * A.wb) * row + A.wb;
+    const size_t ro = (size_t)(2 * A.wb) * iW + A.wb;
     const int wl = -A.wb, wh = A.wb - 1;   // the band covers the window or the mesh
     int b, e;
     sym.range(cls, b, e);
@@ -248,7 +201,7 @@ __global__ __launch_bounds__(SEG_NT) void k_seg_k2(SegK2 A) {
         double2 s = czero();
         seg_term<LEFT, REF, PCH>(A, m, v, wl, wh, lane, [&](double2 x, int w) { s = cadd(s, cmul(x, W[w])); });
         s = wave_sum2(s);
-        if (!LEFT) s = cadd(s, cmul(seg_const<REF, PCH>(A, m, v), A.tot[iW]));
+        if (!LEFT) s = cadd(s, cmul(seg_const<REF, PCH>(A, m, v), A.ws[NW2 * (2 + 3 * PCH) + iW]));
         const double2 raw = cscale(s, A.T);
         for (int k = b + lane; k < e; k += WAVE) {
             const int code = sym.member(cls, k), o = code >> 2;
@@ -268,13 +221,13 @@ __global__ __launch_bounds__(SEG_NT) void k_seg_k2(SegK2 A) {
     const double2 ca = LEFT ? czero() : seg_const<REF, ACH>(A, m, v);
     if (A.at & 1) {
         sa = wave_sum2(sa);
-        if (!LEFT) sa = cadd(sa, cmul(ca, A.tot[2 * NW2 + iW]));
+        if (!LEFT) sa = cadd(sa, cmul(ca, A.ws[NW2 * (2 + 3 * ACH) + iW]));
         rawa = cscale(sa, A.T);
     }
     if (A.at & 2) {
         double2 d = wave_sum2(csub(cscale(st, 2.0), sat));
         if (!LEFT)
-            d = cadd(d, cmul(csub(cscale(seg_const<REF, TCH>(A, m, v), 2.0), ca), A.tot[NW2 + iW]));
+            d = cadd(d, cmul(csub(cscale(seg_const<REF, TCH>(A, m, v), 2.0), ca), A.ws[NW2 * (2 + 3 * TCH) + iW]));
         rawt = cscale(d, -A.T);
     }
     for (int k = b + lane; k < e; k += WAVE) {
@@ -298,14 +251,13 @@ __global__ __launch_bounds__(SEG_NT) void k_seg_k2(SegK2 A) {
 // The SDE L-vertices of one Vertex level (src/SDE.jl:79-217), the channels at the fixed bosonic argument Ω:
 //   Lpp(Ω, ν) = T U [(K1p + K2p(ν)) ΣΠpp + Σ_n K2p(n) Πpp(Ω - n - 1) + Σ_n K3p(n, ν) Πpp(Ω - n - 1)]
 //   Lph(Ω, ν) = T U Σ_{r = a, t} [(K1r + K2r(ν)) ΣΠph + Σ_n K2r(n) Πph(n) + Σ_n K3r(ν, n) Πph(n)]
-// One wave per class of SGpp[2] (waves [0, npp)) or of SGph[2], lanes over n; ΣΠ from the tail sums that
-// start at ω = 0.  SIAM boxes as above: 39 us (point by point over the window 92), with groups 17 (34).
+// One wave per class of SGpp[2] (waves [0, npp)) or of SGph[2], lanes over n.  SIAM boxes as above: 39 us (point by point over the window 92), with groups 17 (34).
 struct SegSde {
     SegCh p, t, a;
     const double2 *Pp, *Ph, *Tp, *Th;
     double2 *Lpp, *Lph;
     double2 TU;
-    int n2b, n2f, nWP, nVP, wb;
+    int n2b, n2f, nWP, nVP;
     SymCls sp, sh;
     int npp, nph;
 };
@@ -322,9 +274,8 @@ __global__ __launch_bounds__(256) void k_seg_sde(SegSde A) {
     const int cls = pw ? wid : wid - A.npp, o0 = sym.rep(cls);
     const int NW2 = 2 * A.n2b - 1, iW = o0 % NW2, iv = o0 / NW2, m = iW - (A.n2b - 1), v = iv - A.n2f;
     const size_t row = (size_t)(m + A.nWP - 1);
-    const double2* T = (pw ? A.Tp : A.Th) + (size_t)(2 * (A.wb + 1)) * row;
     const double2* Pi = (pw ? A.Pp : A.Ph) + (size_t)(2 * A.nVP) * row + A.nVP;
-    const double2 tot = cadd(T[A.wb], T[A.wb + 1]);
+    const double2 tot = (pw ? A.Tp : A.Th)[3 * row + 2];
     double2 s = czero(), cst = czero();
     // Π at n (ph) or Ω - n - 1 (pp) on the mesh
     auto add = [&](double2 x, int n) { s = cadd(s, cmul(x, Pi[pw ? m - n - 1 : n])); };
