@@ -354,11 +354,12 @@ def main_c2(args):
     head = "fp32" if max(errs.values()) <= 1e-6 else "fp64"
     P = paths[head]
     # k_bubble_nl as built: G(R) read once (FP32 on the FP32 path), Πpp and Πph stored on the band
-    # chunks, the chunk sums of all 16-ω chunks written (the far regions enter the later stages only
-    # through those sums)
+    # chunks, the chunk sums of the 16-ω chunks that meet G's mesh or the band written (beyond them one
+    # sum per Ω)
     wb, nchunk = c2_band(w)
     b_bubble = ((8.0 if head == "fp32" else 16.0) * 2 * w["nG"] * NP
-                + 16.0 * (2 * nchunk * 16 * NWP * NP + 2 * (NVP // 16) * NWP * NP))
+                + 16.0 * (2 * nchunk * 16 * NWP * NP
+                          + 2 * max(nchunk, min(NVP, 2 * w["nG"]) // 16) * NWP * NP))
     t_bub = P["st"]["bubble_kernel"] * 1e-3
     gemm_peak = FP32_MFMA_PEAK if head == "fp32" else FP64_MFMA_PEAK
     gemm_traffic = recorded_traffic("c2_bse_gemm_traffic.txt", f"{head}_hbm_bytes_per_launch")

@@ -156,7 +156,8 @@ int fdga_sync(fdga_ctx* ctx);
 int fdga_time_iterations(fdga_ctx* ctx, int32_t strategy, int32_t n, double* ms);
 /* per-stage device time accumulated by fdga_iterate while stage timing is on (ms, summed over
  * passes); stage: 0 dyson+bubbles, 1 cache, 2 L_K2, 3 L_K3, 4 K1, 5 K2, 6 K3, 7 update, 8 SDE;
- * 9 and 10: the BSE_L_K3! and BSE_K3! GEMM kernels alone (inside stages 3 and 6); 11: the bubble
+ * 9 and 10: the BSE_L_K3! and BSE_K3! GEMM kernels alone (inside stages 3 and 6); where both run in the one
+ * kernel k_bse3 (lattice :fdPA, below), its time is in 10 and stage 6; 11: the bubble
  * kernel alone (inside stage 0) */
 int fdga_stage_ms(const fdga_ctx* ctx, int32_t stage, double* ms);
 /* enable (1) / disable (0) per-stage event timing inside fdga_iterate (adds a host sync per
@@ -167,6 +168,10 @@ int fdga_set_stage_timing(fdga_ctx* ctx, int32_t on);
  * fdga_init, fdga_init_sym_grp / fdga_reset_sym_grp and after fdga_set of G0, Π0, the RefVertex
  * tables or the reference Vertex.  No counterpart in the reference (execution option). */
 int fdga_set_graph(fdga_ctx* ctx, int32_t on);
+/* The GEMM launches of the next functions serve every iteration and stage call but one: the lattice :fdPA
+ * iteration without K3 groups and with 2 nK3f <= 96 (FP32) or 64 (FP64) runs both contractions of an (Ω, P) in
+ * one kernel, which takes no tile or grid and executes 48 (2 nK3f)^3 flops per (Ω, P), less where the crossing
+ * leaves the box. */
 /* number of 64 x 64 output tiles (each over the full contraction length) that the batched (p, a, t)
  * BSE_L_K3! (left = 1) or BSE_K3! (left = 0) GEMM launch computes; fewer than the dense count
  * when symmetry groups are installed.  No counterpart in the reference (measurement). */
@@ -206,7 +211,8 @@ int fdga_selftest_zgemm_batched(int32_t M, int32_t N, int32_t K, int32_t nbatch,
  * The reference solves one parameter point per solver; a sweep calls solve! per point.  A group
  * iterates several contexts together: each member's stages run on the member's stream, and the
  * BSE_L_K3!/BSE_K3! contractions of all members run as one grouped GEMM launch each (the (Ω, P,
- * channel) blocks of every member as work items, each with the member's own box sizes).  Each
+ * channel) blocks of every member as work items, each with the member's own box sizes), except for
+ * the members whose two contractions are one kernel (above): those run on the members' streams.  Each
  * member's results equal those of fdga_iterate on the member alone.  Members must share the
  * precision, be all local or all lattice solvers and have no K3 symmetry groups; they must not be
  * iterated alone while in a group, and the group must be destroyed before its members.  No
