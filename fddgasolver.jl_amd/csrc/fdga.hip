@@ -393,12 +393,24 @@ std::vector<BubbleFold> bubble_folds(int L, int LG) {
 
 // band tail sums of one array on the bubble mesh (rows of 2 nVP entries)
 // ω entries per block of the lattice bubble (k_bubble_nl): 16 at L = 16 (16 x 256 complex in LDS);
-// 6 at L = 24 (6 x 576 complex + 24 twiddles, 55.7 KB); otherwise up to 8 (a whole line of Π per store, and
-// several blocks a CU on small lattices), as many L x L tiles twice as fit 64 KB
+// 6 at L = 24 (6 x 576 complex + 24 twiddles, 55.7 KB); otherwise up to 8 (up to L = 15 a whole line of Π per
+// store, and several blocks a CU on small lattices), as many L x L tiles twice as fit 64 KB.  The second plane
+// costs entries at large L, and the transform gains more: L = 18, 22, 28, 32 (NB 6, 4, 2, 1), mesh 32, nΩ = 31:
+// 83, 98, 128, 154 us (through private arrays, NB 12, 8, 5, 3: 284, 383, 599, 777)
 int bubble_nb(int L) {
     if (L == 16) return 16;
     if (L == 24) return 6;
     return std::max(1, std::min(8, (65536 / (int)sizeof(double2) - L) / (2 * L * L)));
+}
+
+// the chunks [blo, bhi) that meet the band (k_tail_sums_chunked reads those that it cuts entry by entry) and the
+// inner ones [ilo, ihi), those and the ones that meet G's mesh
+struct BubbleChunks { int blo, bhi, ilo, ihi; };
+BubbleChunks bubble_chunks(const fdga_ctx* c) {
+    const int NB = bubble_nb(c->d.L), nchunk = (int)cdiv(c->NVP, NB);
+    const int blo = (c->nVP - c->wb) / NB, bhi = (c->nVP + c->wb + NB - 1) / NB;
+    return BubbleChunks{blo, bhi, std::min(blo, std::max(0, c->nVP - c->d.nG) / NB),
+                        std::max(bhi, std::min(nchunk, (c->nVP + c->d.nG + NB - 1) / NB))};
 }
 
 int tail_sums(fdga_ctx* c, const double2* X, double2* T) {
@@ -441,31 +453,31 @@ int bubbles_into(fdga_ctx* c, double2* pp, double2* ph, const double2* Gsrc, boo
     const int L = d.L, NB = bubble_nb(L);
     const int nchunk = (int)cdiv(c->NVP, NB);
     double2 *cpp = c->pchunk[0], *cph = c->pchunk[1];
-    // the chunks [wlo, whi) that k_tail_sums_chunked reads entry by entry: those that meet the band
-    const int wlo = band ? (c->nVP - c->wb) / NB : 0;
-    const int whi = band ? (c->nVP + c->wb + NB - 1) / NB : nchunk;
-    // the inner chunks: those and the ones that meet G's mesh
-    const int ilo = std::min(wlo, std::max(0, c->nVP - d.nG) / NB);
-    const int ihi = std::max(whi, std::min(nchunk, (c->nVP + d.nG + NB - 1) / NB));
-    const int nin = ihi - ilo;
+    const BubbleChunks b = bubble_chunks(c);
+    const int ilo = b.ilo, nin = b.ihi - b.ilo, wlo = band ? b.blo : 0, whi = band ? b.bhi : nchunk;
+    const int glo = std::min(wlo, ilo), ng = std::max(whi, b.ihi) - glo;
     double2* fout = nin < nchunk ? c->pfar : nullptr;
-    const dim3 grid(nin + (fout ? 1 : 0), c->NWP);
+    const dim3 grid(ng + (fout ? 1 : 0), c->NWP);
     kernel_begin(c);
     if (L == 16 && d.precision == FDGA_FP32) {
         // the FP32 form: G(R) rounded to FP32 (into tmpG2), the products and the transform in FP32
         float2* GR32 = reinterpret_cast<float2*>(c->tmpG2);
         k_narrow32<<<cdiv(c->nGel, 256), 256, 0, c->run>>>(GR32, c->tmpG1, c->nGel);
         k_bubble_nl<16, 16, 512, float2><<<grid, 512, (size_t)NB * 256 * sizeof(float2), c->run>>>(
-            pp, ph, GR32, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, fout);
+            pp, ph, GR32, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, glo, ng,
+            fout);
     } else if (L == 16) {
         k_bubble_nl<16, 16, 512><<<grid, 512, (size_t)NB * 256 * sizeof(double2), c->run>>>(
-            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, fout);
+            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, glo, ng,
+            fout);
     } else if (L == 24) {
         k_bubble_nl<24, 6><<<grid, 256, (size_t)(NB * 576 + 24) * sizeof(double2), c->run>>>(
-            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, fout);
+            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, glo, ng,
+            fout);
     } else {
         k_bubble_nl<0, 0><<<grid, 256, (size_t)(2 * NB * L * L + L) * sizeof(double2), c->run>>>(
-            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, fout);
+            pp, ph, c->tmpG1, c->folds, d.nG, L, d.nK1, c->nVP, d.T, NB, cpp, cph, wlo, whi, ilo, nin, glo, ng,
+            fout);
     }
     if (pp == c->Pipp) {
         c->pi_band = band ? 3 : 0;
@@ -1532,7 +1544,8 @@ int fdga_create(fdga_ctx** out, const fdga_dims* dims) {
     for (double2** p : {&c->Ptail[0], &c->Ptail[1], &c->Ptail[2], &c->Ptail[3]}) rc |= dalloc(c, p, c->ntail);
     for (double2** p : {&c->Lpp, &c->Lph, &c->tmpL1, &c->tmpL2}) rc |= dalloc(c, p, c->nL);
     if (d.nonlocal) {
-        const size_t nch = (size_t)c->NP * cdiv(c->NVP, bubble_nb(d.L)) * c->NWP;
+        const BubbleChunks b = bubble_chunks(c);
+        const size_t nch = (size_t)c->NP * (b.ihi - b.ilo) * c->NWP;
         rc |= dalloc(c, &c->pchunk[0], nch);
         rc |= dalloc(c, &c->pchunk[1], nch);
         rc |= dalloc(c, &c->pfar, (size_t)4 * c->NWP);

@@ -328,12 +328,12 @@ __device__ __forceinline__ CT bubble_R(const CT* __restrict__ GR, const BubbleFo
     return acc;
 }
 
-// Blocks take the NB-ω chunks ilo + blockIdx.x of the inner range [ilo, ilo + nin); those in [wlo, whi) store
-// their Π values, and all store their chunk sums.  The iteration passes for [wlo, whi) the chunks that hold the
-// band ω ∈ [-wb, wb) (every Π entry a later stage reads outside the band enters only through the chunk sums) and
-// for the inner range those and the ones that meet G's mesh: beyond it every product vanishes except the
-// origin's, which is the same at every momentum, and one block per Ω (blockIdx.x = nin) sums it over all ω of
-// either side (`fout`).  [0, chunks) for both stores all of Π.
+// Blocks take the NB-ω chunks glo + blockIdx.x, blockIdx.x < ng; those in [wlo, whi) store their Π values, those of
+// the inner range [ilo, ilo + nin) their chunk sums.  The inner range holds the chunks that meet the band
+// ω ∈ [-wb, wb) or G's mesh: beyond it every product vanishes except the origin's, which is the same at every
+// momentum, and one block per Ω (blockIdx.x = ng) sums it over all ω of either side (`fout`).  The iteration
+// stores the band's chunks and takes the inner ones (every Π entry a later stage reads outside the band enters
+// only through the sums); to store all of Π the blocks take all chunks, with the same sums, bit for bit.
 // L = 16, G's mesh of 512 in a bubble mesh of 4096, nΩ = 64: 270 us in FP64 (all chunks stored and summed one by
 // one: 712), 176 in FP32 (546).  L = 10, LG = 20, 120 of 296: 49 us (317, with the transform in private arrays);
 // L = 8, 128 of 512: 30 us (275).
@@ -348,17 +348,19 @@ __global__ __launch_bounds__(NT, NT >= 512 ? (sizeof(CT) == 8 ? 6 : 4) : 1) void
                                                    const CT* __restrict__ GR, const BubbleFold* __restrict__ folds,
                                                    int nG, int Lr, int nW, int nV, double T, int NBr,
                                                    double2* __restrict__ cpp, double2* __restrict__ cph, int wlo,
-                                                   int whi, int ilo, int nin, double2* __restrict__ fout) {
+                                                   int whi, int ilo, int nin, int glo, int ng,
+                                                   double2* __restrict__ fout) {
     extern __shared__ double2 sm[];   // NB * L * L (twice for a run-time L; + L twiddles unless L = 16) of CT
     const int L = LT ? LT : Lr, LL = L * L, NB = NBT ? NBT : NBr;
     CT* s = reinterpret_cast<CT*>(sm);
     CT* s2 = s + NB * LL;
     CT* tw = s + (LT ? 1 : 2) * NB * LL;
     const int tid = threadIdx.x;
-    const int chunk = ilo + (int)blockIdx.x, iw0 = chunk * NB, iW = blockIdx.y;
+    const int chunk = glo + (int)blockIdx.x, iw0 = chunk * NB, iW = blockIdx.y;
+    const bool inner = chunk >= ilo && chunk < ilo + nin;
     const int m = iW - (nW - 1);
     const int nb = min(NB, 2 * nV - iw0);
-    if ((int)blockIdx.x == nin) {   // fout[side + 2 (iΩ + NΩ which)]
+    if ((int)blockIdx.x == ng) {   // fout[side + 2 (iΩ + NΩ which)]
         for (int q = 0; q < 4; ++q) {
             const int which = q >> 1, lo = q & 1 ? (ilo + nin) * NB : 0, hi = q & 1 ? 2 * nV : ilo * NB;
             double2 a = czero();
@@ -409,14 +411,14 @@ __global__ __launch_bounds__(NT, NT >= 512 ? (sizeof(CT) == 8 ? 6 : 4) : 1) void
                 }
             }
             double2* cs = which == 0 ? cpp : cph;
-            if (cs)
+            if (inner)
                 for (int P = tid; P < LL; P += blockDim.x) {
                     double sr = 0.0, si = 0.0;
                     for (int j = 0; j < NB; ++j) {   // the order of the transformed block's sums below
                         const int wl = (j + P) % NB;
                         if (wl < nb) { const CT v = s[wl]; sr += v.x; si += v.y; }
                     }
-                    cs[(size_t)P + (size_t)LL * (blockIdx.x + (size_t)nin * iW)] = cmk(sr, si);
+                    cs[(size_t)P + (size_t)LL * ((size_t)(chunk - ilo) + (size_t)nin * iW)] = cmk(sr, si);
                 }
             __syncthreads();   // s is reused by the next products
             continue;
@@ -500,18 +502,18 @@ __global__ __launch_bounds__(NT, NT >= 512 ? (sizeof(CT) == 8 ? 6 : 4) : 1) void
             }
             __syncthreads();
         }
-        // chunk sums C[P + LL (chunk + chunks iΩ)] = Σ_{ω in this block's chunk} Π(ω, Ω, P) for the
+        // chunk sums C[P + LL (chunk - ilo + nin iΩ)] = Σ_{ω in this block's chunk} Π(ω, Ω, P) for the
         // tail sums (k_tail_sums_chunked); each thread a momentum, the ω order rotated by P so that
         // the lanes' LDS reads spread over the banks
         double2* cs = which == 0 ? cpp : cph;
-        if (cs) {
+        if (inner) {
             for (int P = tid; P < LL; P += blockDim.x) {
                 double sr = 0.0, si = 0.0;
                 for (int j = 0; j < NB; ++j) {
                     const int wl = (j + P) % NB;
                     if (wl < nb) { const CT v = s[P * NB + wl]; sr += v.x; si += v.y; }
                 }
-                cs[(size_t)P + (size_t)LL * (blockIdx.x + (size_t)nin * iW)] = cmk(sr, si);
+                cs[(size_t)P + (size_t)LL * ((size_t)(chunk - ilo) + (size_t)nin * iW)] = cmk(sr, si);
             }
             __syncthreads();   // s is reused by the next products
         }
