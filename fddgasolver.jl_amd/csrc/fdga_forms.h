@@ -10,7 +10,7 @@
 // |ω| <= Wc = NK + |Ω| + |ν| + 2 (NK bounds every box of F, F0 and its tables) X and Y are summed
 // point by point; beyond it neither depends on ω any more (every converted or crossed argument lies
 // outside every box, so only bare vertices and K1/K2 classes at the fixed arguments remain), and the
-// far sums are X_far Σ_far Π + Y_far Σ_far Π0 with the sums of Π and Π0 outside the window (tail_left, tail_right).
+// far sums are X_far Σ_far Π + Y_far Σ_far Π0 with the sums of Π and Π0 outside the window (far_terms).
 #pragma once
 #include "fdga_kernels.h"
 
@@ -104,16 +104,14 @@ __device__ __forceinline__ void form_wave(int wid, int lane, const FormArgs& a) 
     form_xy<FORM, CH>(a, m, v, lane == 0 ? -Wc - 1 : Wc + 1, p, X, Y);
     far_pair(X, xl, xr);
     far_pair(Y, yl, yr);
-    sr = wave_sum(sr);
-    si = wave_sum(si);
-    double2 acc = cmk(sr, si);
-    if (lo > 0)
-        acc = cadd(acc, cadd(cmul(xl, tail_left(a.Pt, pi, row, nVP, a.wb, lo, lane)),
-                             cmul(yl, tail_left(a.P0t, pi0, row, nVP, a.wb, lo, lane))));
-    if (hi < 2 * nVP - 1)
-        acc = cadd(acc, cadd(cmul(xr, tail_right(a.Pt, pi, row, nVP, a.wb, hi, lane)),
-                             cmul(yr, tail_right(a.P0t, pi0, row, nVP, a.wb, hi, lane))));
-    const double2 raw = cscale(acc, a.scale);
+    constexpr bool NOX = FORM == FORM_K1_MFRG || FORM == FORM_K2_MFRG;   // X = 0
+    far_terms(nVP, a.wb, lo, hi, lane, [&](int side, int k) {
+        double2 t = cmul(side ? yr : yl, *(k < 0 ? a.P0t + 3 * row + side : pi0 + k));
+        if (!NOX) t = cadd(cmul(side ? xr : xl, *(k < 0 ? a.Pt + 3 * row + side : pi + k)), t);
+        sr += t.x;
+        si += t.y;
+    });
+    const double2 raw = cscale(cmk(wave_sum(sr), wave_sum(si)), a.scale);
     int b, e;
     a.sym.range(wid, b, e);
     for (int k = b + lane; k < e; k += WAVE) {

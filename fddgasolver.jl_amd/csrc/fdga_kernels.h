@@ -2241,17 +2241,18 @@ __global__ __launch_bounds__(256) void k_tail_sums_chunked(const double2* __rest
         }
     }
 }
-// Σ of a row x of Π (one wave) left of the window's first index lo and right of its last one hi, from the sums S
-// outside the band and the band's entries outside the window (nVP - wb <= lo <= nVP < hi + 1 <= nVP + wb)
-__device__ __forceinline__ double2 tail_left(const double2* S, const double2* x, size_t row, int nVP, int wb, int lo, int lane) {
-    double2 s = czero();
-    for (int k = nVP - wb + lane; k < lo; k += WAVE) s = cadd(s, x[k]);
-    return cadd(S[3 * row], wave_sum2(s));
-}
-__device__ __forceinline__ double2 tail_right(const double2* S, const double2* x, size_t row, int nVP, int wb, int hi, int lane) {
-    double2 s = czero();
-    for (int k = hi + 1 + lane; k < nVP + wb; k += WAVE) s = cadd(s, x[k]);
-    return cadd(S[3 * row + 1], wave_sum2(s));
+// A wave's far terms of one row outside the window [lo, hi] (nVP - wb <= lo <= nVP < hi + 1 <= nVP + wb): add(side, k)
+// for the band's entries k left (0) and right (1) of it, and with k = -1 for the sums outside the band, all in one
+// run of lanes.  The callers add into the lane sums that they reduce anyway.  Three channels, SIAM boxes 33 and 128:
+// K1_new 16.0 and 22.0 us, mfRG K2 20.5 and 114 (each of a wave's four sums read and reduced on its own 20.1 and
+// 26.0, 24.5 and 137; sums kept at every ω of the band 17.2 and 21.2, 20.4 and 113).
+template <class ADD>
+__device__ __forceinline__ void far_terms(int nVP, int wb, int lo, int hi, int lane, ADD&& add) {
+    const int nl = lo > 0 ? lo - (nVP - wb) + 1 : 0, nr = hi < 2 * nVP - 1 ? nVP + wb - hi : 0;
+    for (int j = lane; j < nl + nr; j += WAVE) {
+        const int side = j >= nl, k = side ? j - nl : j;
+        add(side, k == 0 ? -1 : (side ? hi : nVP - wb - 1) + k);
+    }
 }
 // Frequency window of the gather-GEMVs.  Every vertex term that depends on the summed
 // frequency ω is supported on |ω| <= Wc = NK + |m| + |n| + 2, where NK bounds every box of the
@@ -2612,16 +2613,12 @@ __device__ __forceinline__ void sde_L_wave(int wid, int lane, double2* __restric
     sde_terms<DP, DH>(ref, m, v, lane == 0 ? -Wc - 1 : Wc + 1, fxp, fxh);
     far_pair(fxp, xpl, xpr);
     far_pair(fxh, xhl, xhr);
+    far_terms(nVP, wb, lo, hi, lane, [&](int side, int k) {
+        if (DP) { double2 a = cmul(*(k < 0 ? Tpp + 3 * row + side : Pipp + base + k), side ? xpr : xpl); ar += a.x; ai += a.y; }
+        if (DH) { double2 b = cmul(*(k < 0 ? Tph + 3 * row + side : Piph + base + k), side ? xhr : xhl); br += b.x; bi += b.y; }
+    });
     ar = wave_sum(ar); ai = wave_sum(ai); br = wave_sum(br); bi = wave_sum(bi);
-    double2 A = cmk(ar, ai), B = cmk(br, bi);
-    if (lo > 0) {
-        if (DP) A = cadd(A, cmul(tail_left(Tpp, Pipp + base, row, nVP, wb, lo, lane), xpl));
-        if (DH) B = cadd(B, cmul(tail_left(Tph, Piph + base, row, nVP, wb, lo, lane), xhl));
-    }
-    if (hi < 2 * nVP - 1) {
-        if (DP) A = cadd(A, cmul(tail_right(Tpp, Pipp + base, row, nVP, wb, hi, lane), xpr));
-        if (DH) B = cadd(B, cmul(tail_right(Tph, Piph + base, row, nVP, wb, hi, lane), xhr));
-    }
+    const double2 A = cmk(ar, ai), B = cmk(br, bi);
     const double2 rawp = cmul(A, TU), rawh = cmul(B, TU);
     int b, e;
     sym.range(wid, b, e);
