@@ -754,6 +754,73 @@ int idx_fbase(int ch) { return ch == PCH ? 7 : ch == ACH ? 8 : 9; }
 // classes of the channel's K2 (SGpp[2] = SGppL[2] for p, SGph[2] = SGphL[2] for a and t)
 static SymCls sym_k2(const fdga_ctx* c, int ch) { return symcls(c, ch == PCH ? SG_PP2 : SG_PH2); }
 
+// the arguments of the K2 weights of the channels in `mask` (bit ch) on the band into Wc, and of BSE_K1! with the
+// sums of these weights (k1 = false: the sums alone)
+static WArgs w_args(fdga_ctx* c, int mask) {
+    WArgs a{};
+    for (int r = 0; r < 3; ++r) {
+        a.W[r] = c->Wc[r];
+        a.L[r] = chanF(c, c->FL[r]);
+    }
+    a.Ppp = c->Pipp; a.Ppp0 = c->Pi0pp; a.Pph = c->Piph; a.Pph0 = c->Pi0ph;
+    a.f0 = f0_view(c);
+    a.n2b = c->d.nK2b; a.nWP = c->d.nK1; a.nVP = c->nVP; a.wb = c->wb; a.NP = c->NP; a.mask = mask;
+    // the momenta of a thread: as many as leave some 512 blocks, at most W_PCH
+    const size_t n = (size_t)2 * c->wb * c->NW2;
+    a.pch = (int)std::max<size_t>(1, std::min<size_t>(W_PCH, n * c->NP / (512 * 256)));
+    return a;
+}
+static dim3 w_grid(const WArgs& a) {
+    return dim3(cdiv((size_t)2 * a.wb, 32), cdiv((size_t)2 * a.n2b - 1, 8), cdiv((size_t)a.NP, (size_t)a.pch));
+}
+static K1Args k1_args(fdga_ctx* c, int mask, bool k1 = true) {
+    K1Args a{};
+    a.F = vtx_F(c);
+    for (int r = 0; r < 3; ++r) a.L[r] = chanF(c, c->FL[r]);
+    a.Ppp = c->Pipp; a.Ppp0 = c->Pi0pp; a.Pph = c->Piph; a.Pph0 = c->Pi0ph;
+    a.Spp = pi_tail(c, c->Pipp); a.Spp0 = pi_tail(c, c->Pi0pp); a.Sph = pi_tail(c, c->Piph); a.Sph0 = pi_tail(c, c->Pi0ph);
+    a.Kp = c->Fb[PCH].K1; a.Kt = c->Fb[TCH].K1; a.Ka = c->Fb[ACH].K1;
+    a.ws = c->wsum;
+    a.n1 = c->d.nK1; a.n2b = c->d.nK2b; a.nWP = c->d.nK1; a.nVP = c->nVP; a.NP = c->NP; a.mask = mask;
+    a.T = c->d.T;
+    a.sym = symcls(c, SG_K1);
+    a.nk = k1 ? (int)nclass(a.sym, c->n1 * c->NP) : 0;
+    a.ntot = !k1 || a.sym.ncls ? c->NW2 * c->NP : 0;
+    return a;
+}
+static unsigned k1_grid(const K1Args& a) { return 8 * cdiv((size_t)2 * (a.nk + a.ntot) * WAVE, 8 * 256); }
+static int launch_w(fdga_ctx* c, int mask) {
+    const WArgs a = w_args(c, mask);
+    k_bse_w<<<w_grid(a), 256, 0, c->run>>>(a);
+    LAUNCHCHK(c);
+    return 0;
+}
+static bool seg_rows(const fdga_ctx* c);
+// of the three channels, for an iteration (the local solver's one-launch form of BSE_K2! makes its own)
+static int launch_w_all(fdga_ctx* c) { return seg_rows(c) ? 0 : launch_w(c, 7); }
+static int launch_k1(fdga_ctx* c, int mask) {
+    const K1Args a = k1_args(c, mask);
+    k_k1<<<k1_grid(a), 256, 0, c->run>>>(a);
+    LAUNCHCHK(c);
+    return 0;
+}
+// what BSE_K2! of the channels in `mask` reads: their weights and the sums of these, unless they are there already
+static int k2_inputs(fdga_ctx* c, int mask) {
+    if (c->w_fresh) return 0;
+    const WArgs w = w_args(c, mask);
+    const K1Args k = k1_args(c, mask, false);
+    const dim3 g = w_grid(w);
+    const unsigned nw = g.x * g.y * g.z;
+    k_k2_inputs<<<nw + k1_grid(k), 256, 0, c->run>>>(w, k, (int)g.x, (int)g.y, (int)nw);
+    LAUNCHCHK(c);
+    return 0;
+}
+
+// BSE_K2! and BSE_L_K2! of the local solver in one launch each (k_seg_k2, ROWS): for bands up to 128, 32 KB of LDS a
+// block, where an iteration takes the same either way (boxes 56, (28, 28), band 115: :scPA 105 and 103 us, with a
+// reference vertex 157 and 153); on boxes 33 it takes 92 against 101 us.
+static bool seg_rows(const fdga_ctx* c) { return !c->d.nonlocal && c->wb <= SEG_WB; }
+
 // the local solver's K2 copies along diagonals (F, and F0 when it is a Vertex; once per iteration), and for the
 // channels in `left` (bit ch) the weights of BSE_L_K2! into Wc, in one launch
 static int launch_seg_prep(fdga_ctx* c, int left) {
@@ -791,17 +858,18 @@ static int launch_seg_prep(fdga_ctx* c, int left) {
 // BSE_K2! (LEFT: BSE_L_K2!) of the local solver for the channels in `chs` (bit ch)
 template <bool LEFT>
 static int launch_seg_k2(fdga_ctx* c, int chs) {
-    if (launch_seg_prep(c, LEFT ? chs : 0)) return -3;
+    const bool rows = seg_rows(c);
+    if (!rows && ((!LEFT && k2_inputs(c, chs)) || launch_seg_prep(c, LEFT ? chs : 0))) return -3;
     const fdga_dims& d = c->d;
     SegK2 a{};
     const F0V f0 = f0_view(c);
     SegCh* dst[2][3] = {{&a.F.p, &a.F.t, &a.F.a}, {&a.F0.p, &a.F0.t, &a.F0.a}};
     for (int r = 0; r < 3; ++r) {
         *dst[0][r] = seg_of(chanF(c, c->F[r]));
-        dst[0][r]->S = c->seg[r];
+        if (!rows) dst[0][r]->S = c->seg[r];
         if (d.ref_kind == 1) {
             *dst[1][r] = seg_of(f0.g[r]);
-            dst[1][r]->S = c->seg[3 + r];
+            if (!rows) dst[1][r]->S = c->seg[3 + r];
         }
     }
     a.ref = f0.ref;
@@ -819,10 +887,23 @@ static int launch_seg_k2(fdga_ctx* c, int chs) {
     a.np = (chs >> PCH & 1) ? (int)nclass(a.sp, c->n2) : 0;
     a.at = (chs >> ACH & 1) | (chs >> TCH & 1) << 1;
     a.nat = a.at ? (int)nclass(a.sat, c->n2) : 0;
-    a.bat = (int)cdiv((size_t)a.nat * WAVE, 8 * SEG_NT);
-    const unsigned nb = 8 * (a.bat + cdiv((size_t)a.np * WAVE, 8 * SEG_NT));
-    if (!LEFT && d.ref_kind == 1) k_seg_k2<false, true><<<nb, SEG_NT, 0, c->run>>>(a);
-    else k_seg_k2<LEFT, false><<<nb, SEG_NT, 0, c->run>>>(a);
+    const int nt = seg_nt(rows);
+    a.bat = (int)cdiv((size_t)a.nat * WAVE, (size_t)8 * nt);
+    const unsigned nb = 8 * (a.bat + cdiv((size_t)a.np * WAVE, (size_t)8 * nt));
+    const bool ref = !LEFT && d.ref_kind == 1;
+    if (rows) {
+        a.L1p = c->FL[PCH].K1; a.L1t = c->FL[TCH].K1; a.L1a = c->FL[ACH].K1;
+        a.Ppp = c->Pipp; a.Ppp0 = c->Pi0pp; a.Pph = c->Piph; a.Pph0 = c->Pi0ph;
+        a.Spp = pi_tail(c, c->Pipp); a.Spp0 = pi_tail(c, c->Pi0pp); a.Sph = pi_tail(c, c->Piph); a.Sph0 = pi_tail(c, c->Pi0ph);
+        a.nWP = d.nK1; a.nVP = c->nVP; a.vtx0 = d.ref_kind == 1;
+        const size_t lds = (size_t)(nt / WAVE) * 4 * c->wb * sizeof(double2);
+        if (ref) k_seg_k2<false, true, true><<<nb, nt, lds, c->run>>>(a);
+        else k_seg_k2<LEFT, false, true><<<nb, nt, lds, c->run>>>(a);
+    } else if (ref) {
+        k_seg_k2<false, true, false><<<nb, nt, 0, c->run>>>(a);
+    } else {
+        k_seg_k2<LEFT, false, false><<<nb, nt, 0, c->run>>>(a);
+    }
     LAUNCHCHK(c);
     return 0;
 }
@@ -852,46 +933,6 @@ static int launch_lk2(fdga_ctx* c) {
 static int launch_lk2_all(fdga_ctx* c) {
     if (c->d.nonlocal) return launch_lk2<PCH>(c) || launch_lk2<ACH>(c) || launch_lk2<TCH>(c);
     return launch_seg_k2<true>(c, 7);
-}
-
-// the K2 weights of the channels in `mask` (bit ch) on the band into Wc
-static int launch_w(fdga_ctx* c, int mask) {
-    WArgs a{};
-    for (int r = 0; r < 3; ++r) {
-        a.W[r] = c->Wc[r];
-        a.L[r] = chanF(c, c->FL[r]);
-    }
-    a.Ppp = c->Pipp; a.Ppp0 = c->Pi0pp; a.Pph = c->Piph; a.Pph0 = c->Pi0ph;
-    a.f0 = f0_view(c);
-    a.n2b = c->d.nK2b; a.nWP = c->d.nK1; a.nVP = c->nVP; a.wb = c->wb; a.NP = c->NP; a.mask = mask;
-    // the momenta of a thread: as many as leave some 512 blocks, at most W_PCH
-    const size_t n = (size_t)2 * c->wb * c->NW2;
-    a.pch = (int)std::max<size_t>(1, std::min<size_t>(W_PCH, n * c->NP / (512 * 256)));
-    k_bse_w<<<dim3(cdiv(2 * c->wb, 32), cdiv(c->NW2, 8), cdiv(c->NP, a.pch)), 256, 0, c->run>>>(a);
-    LAUNCHCHK(c);
-    return 0;
-}
-// BSE_K1! of the channels in `mask` and the sums of their weights for BSE_K2!; k1 = false: the sums alone
-static int launch_k1(fdga_ctx* c, int mask, bool k1 = true) {
-    K1Args a{};
-    a.F = vtx_F(c);
-    for (int r = 0; r < 3; ++r) a.L[r] = chanF(c, c->FL[r]);
-    a.Ppp = c->Pipp; a.Ppp0 = c->Pi0pp; a.Pph = c->Piph; a.Pph0 = c->Pi0ph;
-    a.Spp = pi_tail(c, c->Pipp); a.Spp0 = pi_tail(c, c->Pi0pp); a.Sph = pi_tail(c, c->Piph); a.Sph0 = pi_tail(c, c->Pi0ph);
-    a.Kp = c->Fb[PCH].K1; a.Kt = c->Fb[TCH].K1; a.Ka = c->Fb[ACH].K1;
-    a.ws = c->wsum;
-    a.n1 = c->d.nK1; a.n2b = c->d.nK2b; a.nWP = c->d.nK1; a.nVP = c->nVP; a.NP = c->NP; a.mask = mask;
-    a.T = c->d.T;
-    a.sym = symcls(c, SG_K1);
-    a.nk = k1 ? (int)nclass(a.sym, c->n1 * c->NP) : 0;
-    a.ntot = !k1 || a.sym.ncls ? c->NW2 * c->NP : 0;
-    k_k1<<<8 * cdiv((size_t)2 * (a.nk + a.ntot) * WAVE, 8 * 256), 256, 0, c->run>>>(a);
-    LAUNCHCHK(c);
-    return 0;
-}
-// what BSE_K2! of the channels in `mask` reads: their weights and the sums of these, unless they are there already
-static int k2_inputs(fdga_ctx* c, int mask) {
-    return c->w_fresh ? 0 : launch_w(c, mask) || launch_k1(c, mask, false) ? -3 : 0;
 }
 
 // lattice BSE_K2!: X table, GEMM X W per Ω over the band, finish per (Ω, P)
@@ -938,14 +979,12 @@ static int launch_k2_nl(fdga_ctx* c) {
 template <int CH>
 static int launch_k2(fdga_ctx* c) {
     if (c->d.nonlocal) return launch_k2_nl<CH>(c);
-    if (k2_inputs(c, 1 << CH)) return -3;
     return launch_seg_k2<false>(c, 1 << CH);
 }
 
 // BSE_K2! of the three channels: one launch for the local solver
 static int launch_k2_all(fdga_ctx* c) {
     if (c->d.nonlocal) return launch_k2<PCH>(c) || launch_k2<ACH>(c) || launch_k2<TCH>(c);
-    if (k2_inputs(c, 7)) return -3;
     return launch_seg_k2<false>(c, 7);
 }
 
@@ -2162,7 +2201,7 @@ static int iterate_two_chains(fdga_ctx* c, int32_t strategy, int32_t update_sigm
         rc = launch_lk2_all(c);
         c->seg_fresh = 1;
     }
-    rc = rc ? rc : launch_w(c, 7);
+    rc = rc ? rc : launch_w_all(c);
     c->w_fresh = 1;
     rc = rc ? rc : launch_k1(c, 7);
     rc = rc ? rc : launch_k2_all(c);
@@ -2289,7 +2328,7 @@ static int iterate_eager(fdga_ctx* c, int32_t strategy, int32_t update_sigma, in
     }
     stage_begin(c);
     // the K1/K2 weights depend on Π, Π0, FL and F0 only: computed once for both stages
-    if (launch_w(c, 7)) return -3;
+    if (launch_w_all(c)) return -3;
     c->w_fresh = 1;
     int rc = launch_k1(c, 7);
     stage_end(c, 4);
@@ -2919,7 +2958,7 @@ int group_iterate_eager(fdga_group* g, int strategy, int update_sigma) {
     }
     for (size_t j = 0; j < fused.size(); ++j) {
         fdga_ctx* c = g->m[j];
-        if (launch_w(c, 7)) return member_err(g, c);
+        if (launch_w_all(c)) return member_err(g, c);
         c->w_fresh = 1;
         c->seg_fresh = fd;
         int rc = launch_k1(c, 7);

@@ -2099,10 +2099,10 @@ struct WArgs {
     int n2b, nWP, nVP, wb, NP, mask, pch;
 };
 constexpr int W_PCH = 8;
-__global__ __launch_bounds__(256) void k_bse_w(WArgs a) {
+__device__ __forceinline__ void bse_w_block(const WArgs& a, int bx, int by, int bz) {
     const int per = 2 * a.wb, NW2 = 2 * a.n2b - 1, NWP = 2 * a.nWP - 1;
-    const int t = (int)(blockIdx.x * 32 + threadIdx.x % 32), iW = (int)(blockIdx.y * 8 + threadIdx.x / 32);
-    const int p0 = (int)blockIdx.z * a.pch;
+    const int t = bx * 32 + (int)threadIdx.x % 32, iW = by * 8 + (int)threadIdx.x / 32;
+    const int p0 = bz * a.pch;
     if (t >= per || iW >= NW2) return;
     const int m = iW - (a.n2b - 1), w = t - a.wb, wc = crossing(m, w, PCH);
     const bool dp = a.mask >> PCH & 1, dt = a.mask >> TCH & 1, da = a.mask >> ACH & 1;
@@ -2125,6 +2125,10 @@ __global__ __launch_bounds__(256) void k_bse_w(WArgs a) {
             if (da) a.W[ACH][o] = cadd(cmul(d, fa), cmul(P, cadd(own_k1<ACH>(a.L, m, p), own_k2<ACH>(a.L, m, w, p))));
         }
     }
+}
+
+__global__ __launch_bounds__(256) void k_bse_w(WArgs a) {
+    bse_w_block(a, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
 }
 
 // Sums of one row (Ω, P) of Π over the bubble mesh: S[3 row + 0, 1, 2] left of the band |ω| < wb, right of it,
@@ -2350,9 +2354,10 @@ __device__ __forceinline__ void k1_store(const K1Args& a, int ch, int m, int p, 
         w[2 * nq] = o.tot;
     }
 }
-__global__ __launch_bounds__(256) void k_k1(K1Args a) {
+// block q of nb (a multiple of 8)
+__device__ __forceinline__ void k1_block(const K1Args& a, int q, int nb) {
     const int lane = threadIdx.x & (WAVE - 1);
-    const int blk = (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8);
+    const int blk = q % 8 * (nb / 8) + q / 8;
     const int wid = blk * (256 / WAVE) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
     const bool pw = wid & 1;
     const int cls = wid >> 1;
@@ -2391,6 +2396,13 @@ __global__ __launch_bounds__(256) void k_k1(K1Args a) {
         if (ma) a.Ka[o] = ka;
         if (mt) a.Kt[o] = cscale(cadd(sym_apply(code & 3, rt.raw), ka), 0.5);   // src/BSE_templates.jl:29-33
     }
+}
+__global__ __launch_bounds__(256) void k_k1(K1Args a) { k1_block(a, (int)blockIdx.x, (int)gridDim.x); }
+// the weights (blocks [0, nw), wx along ω, wy along Ω) and the sums that BSE_K2! called on its own takes, in one launch
+__global__ __launch_bounds__(256) void k_k2_inputs(WArgs w, K1Args k, int wx, int wy, int nw) {
+    const int b = (int)blockIdx.x;
+    if (b < nw) bse_w_block(w, b % wx, b / wx % wy, b / (wx * wy));
+    else k1_block(k, b - nw, (int)gridDim.x - nw);
 }
 
 // BSE_K2!: K2(Ω, ν, P) = T s Σ_ω [F(Ω,ν,ω) - F(Ω,∞,ω)] W(ω) + FL.K2 (t: 2 FLt - FLa).

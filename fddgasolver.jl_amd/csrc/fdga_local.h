@@ -17,7 +17,7 @@
 namespace fdga {
 
 // one channel's classes; S: K2 along its diagonals, S[ν + n2f + 2 n2f row] with row = Ω + ν (t, a) or
-// Ω - ν (p) counted from its smallest value, zero outside the box
+// Ω - ν (p) counted from its smallest value, zero outside the box (null: K2 is read in place)
 struct SegCh {
     const double2 *K1, *K2, *K3;
     double2* S;
@@ -75,8 +75,9 @@ template <class ACC>
 __device__ __forceinline__ void seg_run(const double2* X, int s, int l, int h, int lane, ACC&& acc) {
     for (int w = l + lane; w <= h; w += WAVE) acc(X[(ptrdiff_t)s * w], w);
 }
-// the classes of channel TO in the evaluation F(m, v, ω) of channel CH (CH != TO) on the mesh wl <= ω <= wh
-template <int CH, int TO, class ACC>
+// the classes of channel TO in the evaluation F(m, v, ω) of channel CH (CH != TO) on the mesh wl <= ω <= wh; DIAG: K2
+// along its diagonals from S, else in place
+template <int CH, int TO, bool DIAG, class ACC>
 __device__ __forceinline__ void seg_cross(const SegCh& g, int m, int v, int wl, int wh, int lane, ACC&& acc) {
     // Ω' = al (ω - w0); ν1 = f1 fixed (F1) or ω + f1, ν2 likewise
     constexpr int al = (TO == PCH || CH == TCH) ? 1 : -1;
@@ -87,13 +88,17 @@ __device__ __forceinline__ void seg_cross(const SegCh& g, int m, int v, int wl, 
     seg_run(g.K1 + (g.n1 - 1) - (ptrdiff_t)al * w0, al, max(wl, w0 - (g.n1 - 1)), min(wh, w0 + (g.n1 - 1)), lane, acc);
     const int l2 = max(wl, w0 - (g.n2b - 1)), h2 = min(wh, w0 + (g.n2b - 1)), NW2 = 2 * g.n2b - 1, NV2 = 2 * g.n2f;
     auto k2 = [&](bool fixed, int f) {
+        const double2* K2 = g.K2 + (g.n2b - 1) - (ptrdiff_t)al * w0 + (ptrdiff_t)NW2 * (f + g.n2f);
         if (fixed) {
-            if (in_f(f, g.n2f))
-                seg_run(g.K2 + (g.n2b - 1) - (ptrdiff_t)al * w0 + (ptrdiff_t)NW2 * (f + g.n2f), al, l2, h2, lane, acc);
+            if (in_f(f, g.n2f)) seg_run(K2, al, l2, h2, lane, acc);
+            return;
+        }
+        const int l = max(l2, -g.n2f - f), h = min(h2, g.n2f - 1 - f);
+        if (!DIAG) {
+            seg_run(K2, al + NW2, l, h, lane, acc);
         } else {   // Ω' + ν = w0 + f (al = -1) or Ω' - ν = -w0 - f (al = 1) along the class
             const int row = al < 0 ? w0 + f + (g.n2b - 1) + g.n2f : -w0 - f + (g.n2b - 1) + (g.n2f - 1);
-            if (row >= 0 && row < g.rows())
-                seg_run(g.S + (ptrdiff_t)NV2 * row + (g.n2f + f), 1, max(l2, -g.n2f - f), min(h2, g.n2f - 1 - f), lane, acc);
+            if (row >= 0 && row < g.rows()) seg_run(g.S + (ptrdiff_t)NV2 * row + (g.n2f + f), 1, l, h, lane, acc);
         }
     };
     k2(F1, f1);
@@ -128,11 +133,14 @@ __device__ __forceinline__ void seg_tab(const RefV& r, int k, bool swapped, int 
 
 // Arguments of BSE_K2! (src/BSEa/BSEa_K2.jl:43-100) and BSE_L_K2! (BSEa_K2.jl:1-41)
 struct SegK2 {
-    SegVtx F, F0;                // F0: REF, the local Vertex of the reference system (BSE_K2! only)
+    SegVtx F, F0;                // F0: the local Vertex of the reference system (vtx0)
     RefV ref;
     const double2 *Wp, *Wt, *Wa; // weights on the band
     const double2* ws;           // their sums over the mesh (BSE_K2!; the layout of K1Args)
     const double2 *Lp, *Lt, *La; // FL.K2 (BSE_K2!)
+    const double2 *L1p, *L1t, *L1a;                                              // ROWS: FL.K1,
+    const double2 *Ppp, *Ppp0, *Pph, *Pph0, *Spp, *Spp0, *Sph, *Sph0;            // Π, Π0 and their sums
+    int nWP, nVP, vtx0;
     double2 *Kp, *Kt, *Ka;       // results
     int n2b, n2f, wb;
     double T;
@@ -143,16 +151,16 @@ struct SegK2 {
 };
 // the part of Σ_ω [F(Ω, ν, ω) - F(Ω, ∞, ω)] W(ω) that depends on ω under the sum (LEFT: of Σ Γ W with Γ free of
 // F0 and of the own channel)
-template <bool LEFT, bool REF, int CH, class ACC>
+template <bool LEFT, bool REF, int CH, bool DIAG, class ACC>
 __device__ __forceinline__ void seg_term(const SegK2& A, int m, int v, int wl, int wh, int lane, ACC&& acc) {
     constexpr int C1 = CH == PCH ? TCH : PCH, C2 = CH == ACH ? TCH : ACH;
-    seg_cross<CH, C1>(seg_ch<C1>(A.F), m, v, wl, wh, lane, acc);
-    seg_cross<CH, C2>(seg_ch<C2>(A.F), m, v, wl, wh, lane, acc);
+    seg_cross<CH, C1, DIAG>(seg_ch<C1>(A.F), m, v, wl, wh, lane, acc);
+    seg_cross<CH, C2, DIAG>(seg_ch<C2>(A.F), m, v, wl, wh, lane, acc);
     if (LEFT) return;
     seg_own(seg_ch<CH>(A.F), m, v, wl, wh, lane, acc);
     if (REF) {
-        seg_cross<CH, C1>(seg_ch<C1>(A.F0), m, v, wl, wh, lane, acc);
-        seg_cross<CH, C2>(seg_ch<C2>(A.F0), m, v, wl, wh, lane, acc);
+        seg_cross<CH, C1, DIAG>(seg_ch<C1>(A.F0), m, v, wl, wh, lane, acc);
+        seg_cross<CH, C2, DIAG>(seg_ch<C2>(A.F0), m, v, wl, wh, lane, acc);
         seg_own(seg_ch<CH>(A.F0), m, v, wl, wh, lane, acc);
     }
     if (A.ref.tb) {
@@ -174,7 +182,53 @@ __device__ __forceinline__ double2 seg_const(const SegK2& A, int m, int v) {
     }
     return x;
 }
-constexpr int SEG_NT = 512;
+// threads of a block, and the largest band of the one-launch form
+constexpr int seg_nt(bool rows) { return rows ? 256 : 512; }
+constexpr int SEG_WB = 128;
+__device__ __forceinline__ double2 seg_k1(const SegCh& g, const double2* K1, int m) {
+    return in_b(m, g.n1) ? K1[m + g.n1 - 1] : czero();
+}
+__device__ __forceinline__ double2 seg_k2(const SegCh& g, const double2* K2, int m, int n) {
+    return in_b(m, g.n2b) && in_f(n, g.n2f) ? K2[(size_t)(m + g.n2b - 1) + (size_t)(2 * g.n2b - 1) * (n + g.n2f)] : czero();
+}
+// A wave's row of weights in LDS: the terms of k_bse_w (LEFT: Π0(Ω, ω) F0(Ω, ω~, ∞)) at the class's Ω; returns Σ W
+// over the mesh (BSE_K2!)
+template <bool LEFT, int CH>
+__device__ __forceinline__ double2 seg_row(const SegK2& A, int m, int lane, double2* row) {
+    const SegCh &f0 = seg_ch<CH>(A.F0), &g = seg_ch<CH>(A.F);
+    const double2 *L1 = CH == PCH ? A.L1p : CH == TCH ? A.L1t : A.L1a, *L2 = CH == PCH ? A.Lp : CH == TCH ? A.Lt : A.La;
+    double2 c = A.ref.U, l = czero();   // F0 and FL without their K2
+    if (A.vtx0) {
+        c = cadd(c, CH == TCH ? csub(cscale(seg_k1(f0, f0.K1, m), 2.0), seg_k1(A.F0.a, A.F0.a.K1, m)) : seg_k1(f0, f0.K1, m));
+    }
+    if (!LEFT) l = CH == TCH ? csub(cscale(seg_k1(g, L1, m), 2.0), seg_k1(g, A.L1a, m)) : seg_k1(g, L1, m);
+    const size_t r = (size_t)(m + A.nWP - 1), o = (size_t)(2 * A.nVP) * r + A.nVP;
+    const double2 *P = (CH == PCH ? A.Ppp : A.Pph) + o, *P0 = (CH == PCH ? A.Ppp0 : A.Pph0) + o;
+    double2 s = czero();
+    for (int t = lane; t < 2 * A.wb; t += WAVE) {
+        const int w = t - A.wb, wc = crossing(m, w, CH);
+        double2 f = c, x = P0[w];
+        if (A.vtx0) {
+            double2 k = seg_k2(f0, f0.K2, m, wc);
+            if (CH == TCH) k = csub(cscale(k, 2.0), seg_k2(A.F0.a, A.F0.a.K2, m, wc));
+            f = cadd(f, k);
+        }
+        if (LEFT) {
+            x = cmul(x, f);
+        } else {
+            double2 k = seg_k2(g, L2, m, wc);
+            if (CH == TCH) k = csub(cscale(k, 2.0), seg_k2(g, A.La, m, wc));
+            const double2 p = P[w];
+            x = cadd(cmul(csub(p, x), f), cmul(p, cadd(l, k)));
+            s = cadd(s, x);
+        }
+        row[t] = x;
+    }
+    if (LEFT) return s;
+    const double2 *S = (CH == PCH ? A.Spp : A.Sph) + 3 * r, *S0 = (CH == PCH ? A.Spp0 : A.Sph0) + 3 * r;
+    auto far = [&](int q) { return cadd(cmul(csub(S[q], S0[q]), c), cmul(S[q], l)); };
+    return cadd(wave_sum2(s), cadd(far(0), far(1)));
+}
 // One wave per output class, lanes over ω.  The t channel is summed in the density component 2 F(t) - F(a)
 // next to the a channel, whose terms both share.
 // Blocks of 8 waves on consecutive ν of one Ω (shared lines of W), each XCD on a range of Ω of its own.  Bound
@@ -182,26 +236,53 @@ constexpr int SEG_NT = 512;
 // the card, without symmetry groups BSE_L_K2! 92 us and BSE_K2! 125 us (point by point: 240 and 292), with them
 // 31 and 58 (61 and 164).  Tried: loops unrolled twice (the registers cost more occupancy than the second load
 // in flight gives: 160 -> 209 us), the wave's number in a vector register (160 against 92 us).
-template <bool LEFT, bool REF>
-__global__ __launch_bounds__(SEG_NT) void k_seg_k2(SegK2 A) {
+// ROWS: each wave forms its weights in LDS and K2 is read in place, so that nothing has to be prepared: one launch
+// instead of two (BSE_L_K2!) or three, for boxes whose kernels are not longer than a launch.  Called alone, p
+// channel, SIAM boxes 33, (16, 16): BSE_K2! 8.1 us (prepared 15.2), BSE_L_K2! 7.1 (9.0).  Blocks of four waves, so that
+// few classes spread over the card (eight: 8.6 and 7.4).
+template <bool LEFT, bool REF, bool ROWS>
+__global__ __launch_bounds__(seg_nt(ROWS)) void k_seg_k2(SegK2 A) {
     const int lane = threadIdx.x & (WAVE - 1), bq = (int)blockIdx.x / 8, xcd = (int)blockIdx.x % 8, per = (int)gridDim.x / 8;
     const bool pw = bq >= A.bat;
     const int n = pw ? A.np : A.nat;
-    const int wid = (pw ? xcd * (per - A.bat) + bq - A.bat : xcd * A.bat + bq) * (SEG_NT / WAVE) + seg_wave();
-    if (wid >= n) return;
+    const int wid = (pw ? xcd * (per - A.bat) + bq - A.bat : xcd * A.bat + bq) * (seg_nt(ROWS) / WAVE) + seg_wave();
+    if (!ROWS && wid >= n) return;
     const SymCls& sym = pw ? A.sp : A.sat;
-    const int NV2 = 2 * A.n2f, cls = sym.ncls ? wid : wid / NV2 + (2 * A.n2b - 1) * (wid % NV2), o0 = sym.rep(cls);
+    const int wq = ROWS ? min(wid, n - 1) : wid;   // (every wave reaches the barrier)
+    const int NV2 = 2 * A.n2f, cls = sym.ncls ? wq : wq / NV2 + (2 * A.n2b - 1) * (wq % NV2), o0 = sym.rep(cls);
     const int NW2 = 2 * A.n2b - 1, iW = o0 % NW2, iv = o0 / NW2, m = iW - (A.n2b - 1), v = iv - A.n2f;
     const size_t ro = (size_t)(2 * A.wb) * iW + A.wb;
     const int wl = -A.wb, wh = A.wb - 1;   // the band covers the window or the mesh
     int b, e;
     sym.range(cls, b, e);
+    const double2 *W0, *W1;                // the weights of p, or of a and t
+    double2 tot0 = czero(), tot1 = czero();
+    if constexpr (ROWS) {
+        extern __shared__ double2 seg_rows[];
+        double2* row = seg_rows + (size_t)(4 * A.wb) * seg_wave();
+        W0 = row + A.wb;
+        W1 = row + 3 * A.wb;
+        if (pw) {
+            tot0 = seg_row<LEFT, PCH>(A, m, lane, row);
+        } else {
+            if (A.at & 1) tot0 = seg_row<LEFT, ACH>(A, m, lane, row);
+            if (A.at & 2) tot1 = seg_row<LEFT, TCH>(A, m, lane, row + 2 * A.wb);
+        }
+        __syncthreads();
+        if (wid >= n) return;
+    } else {
+        W0 = (pw ? A.Wp : A.Wa) + ro;
+        W1 = A.Wt + ro;
+        if (!LEFT) {
+            tot0 = A.ws[NW2 * (2 + 3 * (pw ? PCH : ACH)) + iW];
+            if (!pw) tot1 = A.ws[NW2 * (2 + 3 * TCH) + iW];
+        }
+    }
     if (pw) {
-        const double2* W = A.Wp + ro;
         double2 s = czero();
-        seg_term<LEFT, REF, PCH>(A, m, v, wl, wh, lane, [&](double2 x, int w) { s = cadd(s, cmul(x, W[w])); });
+        seg_term<LEFT, REF, PCH, !ROWS>(A, m, v, wl, wh, lane, [&](double2 x, int w) { s = cadd(s, cmul(x, W0[w])); });
         s = wave_sum2(s);
-        if (!LEFT) s = cadd(s, cmul(seg_const<REF, PCH>(A, m, v), A.ws[NW2 * (2 + 3 * PCH) + iW]));
+        if (!LEFT) s = cadd(s, cmul(seg_const<REF, PCH>(A, m, v), tot0));
         const double2 raw = cscale(s, A.T);
         for (int k = b + lane; k < e; k += WAVE) {
             const int code = sym.member(cls, k), o = code >> 2;
@@ -210,24 +291,24 @@ __global__ __launch_bounds__(SEG_NT) void k_seg_k2(SegK2 A) {
         }
         return;
     }
-    const double2 *Wa = A.Wa + ro, *Wt = A.Wt + ro;
     double2 sa = czero(), st = czero(), sat = czero();   // Σ Xa Wa, Σ Xt Wt, Σ Xa Wt
-    seg_term<LEFT, REF, ACH>(A, m, v, wl, wh, lane, [&](double2 x, int w) {
-        sa = cadd(sa, cmul(x, Wa[w]));
-        sat = cadd(sat, cmul(x, Wt[w]));
+    seg_term<LEFT, REF, ACH, !ROWS>(A, m, v, wl, wh, lane, [&](double2 x, int w) {
+        sa = cadd(sa, cmul(x, W0[w]));
+        sat = cadd(sat, cmul(x, W1[w]));
     });
-    if (A.at & 2) seg_term<LEFT, REF, TCH>(A, m, v, wl, wh, lane, [&](double2 x, int w) { st = cadd(st, cmul(x, Wt[w])); });
+    if (A.at & 2)
+        seg_term<LEFT, REF, TCH, !ROWS>(A, m, v, wl, wh, lane, [&](double2 x, int w) { st = cadd(st, cmul(x, W1[w])); });
     double2 rawa = czero(), rawt = czero();
     const double2 ca = LEFT ? czero() : seg_const<REF, ACH>(A, m, v);
     if (A.at & 1) {
         sa = wave_sum2(sa);
-        if (!LEFT) sa = cadd(sa, cmul(ca, A.ws[NW2 * (2 + 3 * ACH) + iW]));
+        if (!LEFT) sa = cadd(sa, cmul(ca, tot0));
         rawa = cscale(sa, A.T);
     }
     if (A.at & 2) {
         double2 d = wave_sum2(csub(cscale(st, 2.0), sat));
         if (!LEFT)
-            d = cadd(d, cmul(csub(cscale(seg_const<REF, TCH>(A, m, v), 2.0), ca), A.ws[NW2 * (2 + 3 * TCH) + iW]));
+            d = cadd(d, cmul(csub(cscale(seg_const<REF, TCH>(A, m, v), 2.0), ca), tot1));
         rawt = cscale(d, -A.T);
     }
     for (int k = b + lane; k < e; k += WAVE) {
