@@ -2874,15 +2874,19 @@ hipError_t group_gemm_launch(fdga_group* g, int which, const GemmSchedGroup& sc,
                      b, ep);
 }
 
+// the grouped BSE_K3!'s functors hold one F/Fbuff state of all members: members at another one are refused, also where
+// every contraction runs on its member's own arrays
+int group_state(fdga_group* g) {
+    const int s = g->m[0]->swap_state;
+    for (const fdga_ctx* c : g->m)
+        if (c->swap_state != s) return gfail(g, "group members are not at the same iteration (F/Fbuff state)");
+    return 0;
+}
+
 // the grouped contraction `which` (0 BSE_L_K3!, 1 BSE_K3!) on the group's stream: one launch, or for
 // lattice groups the p and a channels and then the t channel; unfused: of the members outside k_bse3
 int group_gemm(fdga_group* g, int which, bool unfused = false) {
     const GroupItems& gi = unfused && g->nfused ? g->giu[g->tile[which]] : g->gi[g->tile[which]];
-    if (which == 1) {
-        const int s = g->m[0]->swap_state;
-        for (const fdga_ctx* c : g->m)
-            if (c->swap_state != s) return gfail(g, "group members are not at the same iteration (F/Fbuff state)");
-    }
     if (g->timing) GHIPCHK(g, hipEventRecord(g->tev[0], g->st));
     hipError_t e = group_gemm_launch(g, which, GemmSchedGroup{gi.items, gi.geo, gi.nitems},
                                      group_grid(g, which, (size_t)gi.nitems));
@@ -2939,6 +2943,7 @@ int group_iterate_eager(fdga_group* g, int strategy, int update_sigma) {
     const int all[3] = {PCH, ACH, TCH};
     const bool fd = strategy == FDGA_FDPA;
     std::vector<char> fused;
+    if (group_state(g)) return -1;
     for (fdga_ctx* c : g->m) {
         if (has_k3_groups(c)) return gfail(g, "group members must not have K3 symmetry groups installed");
         c->run = c->st;
@@ -2962,7 +2967,7 @@ int group_iterate_eager(fdga_group* g, int strategy, int update_sigma) {
         c->w_fresh = 1;
         c->seg_fresh = fd;
         int rc = launch_k1(c, 7);
-            rc = rc ? rc : launch_k2_all(c);
+        rc = rc ? rc : launch_k2_all(c);
         c->w_fresh = c->seg_fresh = 0;
         if (rc) return member_err(g, c);
         if (fused[j]) {
@@ -3185,6 +3190,7 @@ int fdga_group_autotune(fdga_group* g, int32_t reps) {
     const int all[3] = {PCH, ACH, TCH};
     for (int t = 0; t < TILE_N; ++t)
         if (group_build_items(g, t)) return -2;
+    if (group_state(g)) return -1;
     if (fdga_group_sync(g) || group_fork(g)) return -2;
     for (fdga_ctx* c : g->m) {
         c->run = c->st;
