@@ -2333,8 +2333,9 @@ static int iterate_eager(fdga_ctx* c, int32_t strategy, int32_t update_sigma, in
     int rc = launch_k1(c, 7);
     stage_end(c, 4);
     stage_begin(c);
+    c->seg_fresh = strategy == FDGA_FDPA;   // BSE_L_K2! has made the K2 copies, as in the untimed iteration
     rc = rc ? rc : launch_k2_all(c);
-    c->w_fresh = 0;
+    c->w_fresh = c->seg_fresh = 0;
     if (rc) return -3;
     stage_end(c, 5);
     stage_begin(c);
