@@ -3183,9 +3183,10 @@ int fdga_group_set_tiles(fdga_group* g, int32_t which, int32_t tile, int64_t gri
 }
 
 // Times every tile shape and grid (one workgroup per item; 4, 8 or 16 workgroups per CU) of both
-// contractions on the members' current operands and keeps the fastest.  The contractions'
-// outputs are scratch until the next iteration recomputes them; F, Fbuff's inputs and Σ are left
-// as they are.
+// contractions on the members' current operands and keeps the fastest: BSE_L_K3! over the members whose :fdPA
+// iterations launch it (none: its settings stay), BSE_K3! over all, as :scPA does.  Fbuff.K3 is scratch until the next
+// iteration overwrites it; FL.K3, which :scPA reads, is kept there while BSE_L_K3! writes it, so that the solvers'
+// state is left as it is.
 int fdga_group_autotune(fdga_group* g, int32_t reps) {
     if (!g || reps < 1) return -1;
     const int all[3] = {PCH, ACH, TCH};
@@ -3196,7 +3197,7 @@ int fdga_group_autotune(fdga_group* g, int32_t reps) {
     for (fdga_ctx* c : g->m) {
         c->run = c->st;
         // the operand forms the group's launches were made for (those of the members' iterations)
-        if (fl_prepare(c) || fdga_build_k3_cache(c) || k3_rhs(c, k3_set(c, all, 3, false, false), 3))
+        if (fl_prepare(c) || fdga_build_k3_cache(c) || (g->nfused == g->n && k3_rhs(c, k3_set(c, all, 3, false, false), 3)))
             return member_err(g, c);
     }
     if (group_join(g) || fdga_group_sync(g)) return -2;
@@ -3207,20 +3208,29 @@ int fdga_group_autotune(fdga_group* g, int32_t reps) {
     }
     const int keep_timing = g->timing;
     g->timing = 0;
-    for (int which = 0; which < 2; ++which) {
+    auto copy_FL = [&](bool back) -> int {
+        for (fdga_ctx* c : g->m)
+            for (int r = 0; r < 3; ++r)
+                GHIPCHK(g, hipMemcpyAsync(back ? c->FL[r].K3 : c->Fb[r].K3, back ? c->Fb[r].K3 : c->FL[r].K3,
+                                          c->n3 * c->NP * sizeof(double2), hipMemcpyDeviceToDevice, g->st));
+        return 0;
+    };
+    for (int which = g->nfused < g->n ? 0 : 1; which < 2; ++which) {
+        const GroupItems* list = which == 0 && g->nfused ? g->giu : g->gi;
+        if (which == 0 && copy_FL(false)) return -2;
         float best = 1e30f;
         int bt = g->tile[which];
         size_t bg = g->grid[which];
         for (int t = 0; t < TILE_N; ++t)
             for (int per : {0, 4, 8, 16}) {
                 const size_t grid = per ? (size_t)((ncu * per + 7) / 8 * 8) : 0;
-                if (grid && grid >= (size_t)g->gi[t].nitems) continue;
+                if (grid && grid >= (size_t)list[t].nitems) continue;
                 g->tile[which] = t;
                 g->grid[which] = grid;
-                if (group_gemm(g, which)) return -3;   // warm-up
+                if (group_gemm(g, which, which == 0)) return -3;   // warm-up
                 GHIPCHK(g, hipEventRecord(g->tev[0], g->st));
                 for (int r = 0; r < reps; ++r)
-                    if (group_gemm(g, which)) return -3;
+                    if (group_gemm(g, which, which == 0)) return -3;
                 GHIPCHK(g, hipEventRecord(g->tev[1], g->st));
                 GHIPCHK(g, hipEventSynchronize(g->tev[1]));
                 float ms = 0.f;
@@ -3229,6 +3239,14 @@ int fdga_group_autotune(fdga_group* g, int32_t reps) {
             }
         g->tile[which] = bt;
         g->grid[which] = bg;
+        if (which == 0) {
+            if (copy_FL(true)) return -2;
+            // the FP32 lattice BSE_L_K3! has written right operands of its own
+            if (group_fork(g)) return -2;
+            for (fdga_ctx* c : g->m)
+                if (k3_rhs(c, k3_set(c, all, 3, false, false), 3)) return member_err(g, c);
+            if (group_join(g)) return -2;
+        }
     }
     g->timing = keep_timing;
     group_graphs_invalidate(g);
