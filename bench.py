@@ -19,7 +19,7 @@ Anderson loop over 1.6 GB state vectors is outside the timed path).  `value` is 
 iterations/s when every error is <= 1e-6, else the FP64 path's (`config.value_path`).
 
 `roofline` is the BSE contraction, the iteration's largest kernel (k_bse3: BSE_L_K3! and BSE_K3! of the three
-channels in one launch): MFMA-bound (executed flops 8 BM BN Nν3 per computed tile over the launch's HIP-event
+channels in one launch): MFMA-bound (executed flops of its 16 x 16 tiles, bse3_flops, over the launch's HIP-event
 time), with its algorithmic bytes beside (gemm_roofline) and `traffic` the rocprofv3 FETCH + WRITE bytes per
 launch (profiles/c2_bse_gemm_traffic.txt).  `roofline_bubble` is the lattice bubble kernel
 (k_bubble_nl, bubbles_real_space!): G(R) read once, Πpp and Πph written on the band chunks and the
@@ -269,33 +269,33 @@ def c2_band(w):
     return wb, (nVP + wb + 15) // 16 - (nVP - wb) // 16
 
 
-def tune_gemm_grid(S, grids=(0, 256, 512, 768, 1024), lk3_grids=(0, 160, 192, 224), reps=4):
-    """Workgroup counts of the contraction launches by whole-iteration time (hipGraph replay): a persistent
-    grid leaves compute units to the iteration's other chain (BSE_L_K2!, weights, BSE_K1!, BSE_K2!),
-    which the launch-by-launch autotuner cannot see.  First one count for both contractions, then
-    BSE_L_K3!'s alone (the FP32 lattice form runs one workgroup per compute unit: counts below 256 leave
-    some free).  The state is restored afterwards; results do not depend on the grids.  Returns
-    (BSE_L_K3!, BSE_K3!) counts."""
+def tune_gemm_grid(S, grids=(0, 256, 512, 768, 1024), reps=4):
+    """Workgroup count of the fused contraction (k_bse3 takes BSE_K3!'s) by whole-iteration time (hipGraph replay): a
+    persistent grid leaves compute units to the iteration's other chain (BSE_L_K2!, weights, BSE_K1!, BSE_K2!).  The
+    state is restored afterwards; results do not depend on the grid."""
     import fdga
     x = fdga.flatten(S)
     S.set_graph(True)
 
-    def timed(gl, gk):
-        S.set_gemm_grid(True, gl)
-        S.set_gemm_grid(False, gk)
+    def timed(g):
+        S.set_gemm_grid(False, g)
         fdga.unflatten(S, x)
         fdga.iterate_solver(S, "fdPA")   # capture
         S.sync()
         return S.time_iterations("fdPA", reps)
-    best = min((timed(g, g), g) for g in grids)
-    gk = best[1]
-    best = min((timed(g, gk), g) for g in lk3_grids if g != gk or g == 0)
-    gl = best[1]
-    S.set_gemm_grid(True, gl)
-    S.set_gemm_grid(False, gk)
+    grid = min((timed(g), g) for g in grids)[1]
+    S.set_gemm_grid(False, grid)
     S.set_graph(False)
     fdga.unflatten(S, x)
-    return gl, gk
+    return grid
+
+
+def bse3_flops(w):
+    """Executed flops of k_bse3: per (Ω, P) six products (two equations, three channels) of 16 x 16 tiles over
+    the rows and columns of the K3 box, the summed frequency in steps of 4 (48 Nν3³ at multiples of 16)."""
+    N = 2 * w["nK3"][1]
+    T = 16 * ((N + 15) // 16)
+    return 6 * 8.0 * T * T * 4 * ((N + 3) // 4) * (2 * w["nK3"][0] - 1) * w["L"] ** 2
 
 
 def gemm_roofline(head, P, gemm_peak, traffic, n3P):
@@ -334,11 +334,9 @@ def main_c2(args):
             fdga.iterate_solver(S, "fdPA")
         obs = observables(S)
         fdga.unflatten(S, x0)
-        S.autotune(reps=3)   # tile shapes of the contraction launches (results do not depend on them)
-        grid = tune_gemm_grid(S)
-        log(f"bench c2[{prec}]: autotuned tile shapes (BSE_L_K3!, BSE_K3!): {S.gemm_tiles()}, grid {grid}")
+        log(f"bench c2[{prec}]: contraction grid {tune_gemm_grid(S)}")
         ms, st = time_path(S, args, STAGES)
-        f_exec = S.gemm_flops(True) + S.gemm_flops(False)
+        f_exec = bse3_flops(w)
         t_gemm = (st["gemm_L_K3"] + st["gemm_K3"]) * 1e-3
         log(f"bench c2[{prec}]: {ms:.3f} ms/iteration; stages " + ", ".join(f"{k}={v:.3f}" for k, v in st.items()))
         paths[prec] = dict(ms=ms, st=st, obs=obs, f_exec=f_exec, t_gemm=t_gemm, bse_tflops=f_exec / t_gemm / 1e12,
@@ -420,9 +418,9 @@ def build_c4_point(k, precision):
 
 def main_c4(args):
     """The batched sweep: one parquet iteration of all 8 points per step, every member's stages on
-    its own stream and the BSE contractions of all points in one grouped persistent launch each,
-    tile shapes and grids from the autotuner, the group iteration replayed from a hipGraph; FP32
-    MFMA contraction.  Compared with the same points iterated one after the other."""
+    its own stream, its contractions in one launch there (every point's K3 box is within the fused
+    contraction's limit), the group iteration replayed from a hipGraph; FP32 MFMA contraction.  Compared
+    with the same points iterated one after the other."""
     import fdga
     t0 = time.perf_counter()
     S, ws = [], []
@@ -434,10 +432,6 @@ def main_c4(args):
     G = fdga.SolverGroup(S)
     G.iterate("fdPA")   # first iteration eagerly (caches each point's reference SDE)
     G.sync()
-    t1 = time.perf_counter()
-    G.autotune(reps=2)
-    tuned = {("L_K3", "K3")[wh]: dict(zip(("tile", "grid", "computed_tiles"), G.tiles(wh))) for wh in (0, 1)}
-    log(f"bench c4: autotuned in {time.perf_counter() - t1:.1f} s: {tuned}")
     G.set_graph(True)
     for _ in range(max(1, args.warmup)):
         G.iterate("fdPA")
@@ -466,8 +460,7 @@ def main_c4(args):
         "sweep_ms_per_iteration": ms, "sweep_iters_per_s": 1000.0 / ms,
         "points_one_after_another_ms": sum(solo),
         "contractions": {"ms": gl + gk, "flops": 2 * f_launch, "tflops": tf, "peak_tflops_fp32": peak,
-                         "roofline_frac": tf / peak},
-        "autotuned": tuned}), flush=True)
+                         "roofline_frac": tf / peak}}), flush=True)
 
 
 def main_c3(args):
@@ -658,7 +651,7 @@ def main():
                     help="c2: the headline NL Hubbard lattice workload (the metric's JSON line); c1: the local SIAM fdPA "
                          "workload at its fixed point (separate JSON line); c0: the small SIAM solve (hipGraph replay and "
                          "Newton–Krylov vs mixing, separate JSON line); c4: the 8-point lattice sweep in one solver group "
-                         "(grouped GEMM launches, autotuned tiles, hipGraph; separate JSON line); c3: the tangent and adjoint of "
+                         "(hipGraph; separate JSON line); c3: the tangent and adjoint of "
                          "build_K3_cache! + BSE_K3! on the c2 lattice (separate JSON line)")
     ap.add_argument("--acc-iters", type=int, default=5,
                     help="c2: iterations from the initial state after which the FP32 path is compared with FP64")

@@ -2658,10 +2658,10 @@ int fdga_set_stage_timing(fdga_ctx* c, int32_t on) {
 
 // =========================================================================================
 // Groups of solver contexts (a parameter sweep on one device).  Each member runs its own stages
-// on its own stream, concurrently with the other members; the BSE_L_K3! and BSE_K3! contractions
-// of all members run as one grouped GEMM launch each on the group's stream (the (Ω, P, channel)
-// blocks of every member as work items, with the member's own box sizes), persistent over a
-// chosen grid and with a chosen tile shape.  Each member's results are those of fdga_iterate on
+// on its own stream, concurrently with the other members, the fused :fdPA contraction (k_bse3) among
+// them; the BSE_L_K3! and BSE_K3! contractions of the other members (:scPA: of all) run as one
+// grouped GEMM launch each on the group's stream (the (Ω, P, channel) blocks of every member as work
+// items, with the member's own box sizes), persistent over a chosen grid and with a chosen tile shape.  Each member's results are those of fdga_iterate on
 // the member alone.  No counterpart in the reference, which solves one parameter point per solver.
 struct GroupItems {   // work items of one tile shape
     int* items = nullptr;     // lattice groups: the p and a channels' items; else all three channels'

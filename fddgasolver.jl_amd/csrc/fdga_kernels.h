@@ -1181,10 +1181,11 @@ typedef LK3_EpT<true> LK3R_Ep;
 // BSE_L_K3! of the FP32 lattice contraction with its momentum-independent operands kept on chip: one
 // workgroup per (channel slot, Ω, LK3P_G momenta).  Γr(Ω), the left operand rounded to FP32, stays in
 // LDS; each thread keeps F0r(Ω) at its output positions in registers, so a momentum reads only its Π0
-// and Π rows (and Γ~(Ω), from L2, in the epilogue) and forms B = Π0 F0r into LDS.  The tile is zgemm_tiles_t's 64 x 64 (four
-// waves of 32 x 32, the same MFMA sequence and K order) and the epilogue is LK3BoundR's, so every
-// element rounds exactly as in the GEMM engine.  FL.K3 in FP32 (out32) and the FP32 right operand
-// (R32) are written; Nν3 <= 64.
+// and Π rows (and Γ~(Ω), from L2, in the epilogue) and forms B = Π0 F0r into LDS.  The tile is
+// zgemm_tiles_t's 64 x 64 (four waves of 32 x 32, the same MFMA sequence and K order) and the epilogue is
+// LK3BoundR's, so every element rounds exactly as in the GEMM engine.  FL.K3 in FP32 (out32) and the
+// FP32 right operand (R32) are written; Nν3 <= 64.  Launched by the mfRG map (the :fdPA iterations that
+// meet its conditions run k_bse3).
 constexpr int LK3P_G = 8;
 __global__ __launch_bounds__(256, 2) void k_lk3_pbatch(K3Geom g, LK3Chan c0, LK3Chan c1, int nslot) {
     typedef MfmaT<true> MT;
@@ -2277,9 +2278,9 @@ __device__ __forceinline__ void far_pair(double2 t, double2& left, double2& righ
 //   Σ W = c0 (ΣΠ - ΣΠ0) + kL ΣΠ + Σ_ω x(ω),   x(ω) = (Π - Π0) K2_0(Ω, ω~) + Π K2_L(Ω, ω~, P)
 //   K1  = T s [(c0 + K1(Ω, P)) ΣW + Σ_ω (K2_0(Ω, ω) + K2(Ω, ω, P)) W(ω)]
 // with sums over the K2 boxes alone and ΣΠ from the tail sums; W(ω) is formed in place.  Two waves per class of
-// (Ω, P), one for p and one for a and t (one load of Π and of each K2 for both), lanes over ω; without groups they also store Σ W left and right of the
-// band and in all for the rows of the K2 mesh, ws[iΩ + Nω2 (P + NP (part + 3 ch))], under groups the waves after
-// the nk classes do.  Each XCD takes a range of classes of its own: neighbours in Ω share the lines of K2.
+// (Ω, P), one for p and one for a and t (one load of Π and of each K2 for both), lanes over ω; without groups they
+// also store Σ W left and right of the band and in all for the rows of the K2 mesh, ws[iΩ + Nω2 (P + NP (part +
+// 3 ch))], under groups the waves after the nk classes do.  Each XCD takes a range of classes of its own: neighbours in Ω share the lines of K2.
 // Bound by the address rate of the K2 loads (Ω is fastest there, a line per lane).  L = 16, nΩ = 64, K2 (32, 32):
 // 119 us for the three channels (F evaluated at every ω of the window, two launches: 333); L = 24, 72, (36, 36):
 // 235 us (503).  Blocks of 8 neighbours in Ω of one kind measured 286 against 160 us, a and t apart 160 to 119.

@@ -332,7 +332,8 @@ __global__ __launch_bounds__(seg_nt(ROWS)) void k_seg_k2(SegK2 A) {
 // The SDE L-vertices of one Vertex level (src/SDE.jl:79-217), the channels at the fixed bosonic argument Ω:
 //   Lpp(Ω, ν) = T U [(K1p + K2p(ν)) ΣΠpp + Σ_n K2p(n) Πpp(Ω - n - 1) + Σ_n K3p(n, ν) Πpp(Ω - n - 1)]
 //   Lph(Ω, ν) = T U Σ_{r = a, t} [(K1r + K2r(ν)) ΣΠph + Σ_n K2r(n) Πph(n) + Σ_n K3r(ν, n) Πph(n)]
-// One wave per class of SGpp[2] (waves [0, npp)) or of SGph[2], lanes over n.  SIAM boxes as above: 39 us (point by point over the window 92), with groups 17 (34).
+// One wave per class of SGpp[2] (waves [0, npp)) or of SGph[2], lanes over n.  SIAM boxes as above: 39 us (point by
+// point over the window 92), with groups 17 (34).
 struct SegSde {
     SegCh p, t, a;
     const double2 *Pp, *Ph, *Tp, *Th;

@@ -165,12 +165,12 @@ class Solver:
         return tuple(self.lib.fdga_gemm_grid(self.h, left) for left in (1, 0))
 
     def set_gemm_grid(self, left, grid):
-        """A persistent grid of `grid` workgroups (a multiple of 8) for that launch, or 0; results do
-        not depend on it."""
+        """A persistent grid of `grid` workgroups (a multiple of 8) for that launch, or 0; the fused lattice
+        contraction takes BSE_K3!'s.  Results do not depend on it."""
         self._check(self.lib.fdga_set_gemm_grid(self.h, int(left), int(grid)))
 
     def gemm_flops(self, left):
-        """Executed flops of one batched BSE_L_K3! (left) or BSE_K3! launch."""
+        """Executed flops of one batched BSE_L_K3! (left) or BSE_K3! launch (not of the fused lattice contraction)."""
         return self.lib.fdga_gemm_flops(self.h, int(left))
 
     def set_stage_timing(self, on):
@@ -192,8 +192,9 @@ class Solver:
 
 class SolverGroup:
     """Several solvers on one device iterated together (a parameter sweep): each member's stages
-    run on its own stream, and the BSE_L_K3!/BSE_K3! contractions of all members run as one
-    grouped GEMM launch each.  Members keep their own boxes and lattices; they must share the
+    run on its own stream, and the BSE_L_K3!/BSE_K3! contractions as one grouped GEMM launch each over
+    the members, or in :fdPA for a lattice member without K3 boxes beyond the fused contraction's limit
+    (include/fdga.h, fdga_gemm_blocks) in one kernel on its stream.  Members keep their own boxes and lattices; they must share the
     contraction precision and be all local or all lattice solvers, without K3 symmetry groups.
     No counterpart in the reference (one solver per parameter point); each member ends where
     `iterate_solver` on the member alone would.  Close the group before its members."""
@@ -245,7 +246,8 @@ class SolverGroup:
         self._check(self.lib.fdga_group_set_timing(self.h, int(on)))
 
     def gemm_ms(self):
-        """Accumulated times of the grouped BSE_L_K3! and BSE_K3! launches while timing is on."""
+        """Accumulated times of the grouped BSE_L_K3! and BSE_K3! launches while timing is on; members in the
+        fused contraction count with BSE_K3!."""
         out = []
         for w in (0, 1):
             ms = ctypes.c_double(0.0)
@@ -265,7 +267,7 @@ class SolverGroup:
         self._check(self.lib.fdga_group_set_tiles(self.h, which, self.TILES[tile], grid))
 
     def autotune(self, reps=3):
-        """Time every tile shape and grid of both contractions and keep the fastest."""
+        """Time every tile shape and grid of both grouped contractions and keep the fastest."""
         self._check(self.lib.fdga_group_autotune(self.h, reps))
 
 

@@ -168,10 +168,11 @@ int fdga_set_stage_timing(fdga_ctx* ctx, int32_t on);
  * fdga_init, fdga_init_sym_grp / fdga_reset_sym_grp and after fdga_set of G0, Π0, the RefVertex
  * tables or the reference Vertex.  No counterpart in the reference (execution option). */
 int fdga_set_graph(fdga_ctx* ctx, int32_t on);
-/* The GEMM launches of the next functions serve every iteration and stage call but one: the lattice :fdPA
- * iteration without K3 groups and with 2 nK3f <= 96 (FP32) or 64 (FP64) runs both contractions of an (Ω, P) in
- * one kernel, which takes no tile or grid and executes 48 (2 nK3f)^3 flops per (Ω, P), less where the crossing
- * leaves the box. */
+/* The GEMM launches of the next functions serve the stage calls and every iteration but one: the lattice (L > 1)
+ * :fdPA and :fdPA_new iterations without K3 groups, with 2 nK3f <= 64 in FP64, or in FP32 with 2 nK3f <= 96 and
+ * (2 nK3b - 1) L^2 >= 512, run both contractions of an (Ω, P) in one kernel.  It takes no tile, and BSE_K3!'s
+ * workgroup count (0: one per work item; results do not depend on it).  It executes 48 N^3 flops per (Ω, P) where
+ * N = 2 nK3f is a multiple of 16, more otherwise (rows and columns in tiles of 16, the sum in steps of 4). */
 /* number of 64 x 64 output tiles (each over the full contraction length) that the batched (p, a, t)
  * BSE_L_K3! (left = 1) or BSE_K3! (left = 0) GEMM launch computes; fewer than the dense count
  * when symmetry groups are installed.  No counterpart in the reference (measurement). */
@@ -183,8 +184,8 @@ int     fdga_gemm_tile(const fdga_ctx* ctx, int32_t left);
 int     fdga_set_gemm_tile(fdga_ctx* ctx, int32_t left, int32_t tile);
 /* workgroup count of that launch: 0 = one workgroup per output tile (the default), otherwise a
  * persistent grid of `grid` workgroups (a multiple of 8, so that every workgroup stays on one XCD)
- * looping over the tiles (the FP32 lattice BSE_L_K3!: over its (channel, Ω, momentum group) tasks); a
- * smaller grid leaves compute units to the other chain of the iteration.
+ * looping over the tiles (the FP32 lattice BSE_L_K3! of the three channels, which the mfRG map launches: over its
+ * (channel, Ω, momentum group) tasks); a smaller grid leaves compute units to the other chain of the iteration.
  * Results do not depend on it.  No counterpart in the reference (execution option). */
 int     fdga_gemm_grid(const fdga_ctx* ctx, int32_t left);
 int     fdga_set_gemm_grid(fdga_ctx* ctx, int32_t left, int32_t grid);
@@ -195,8 +196,8 @@ int     fdga_set_gemm_grid(fdga_ctx* ctx, int32_t left, int32_t grid);
 int     fdga_autotune(fdga_ctx* ctx, int32_t reps);
 
 /* Self-test of the batched complex GEMM engine used by BSE_L_K3!/BSE_K3!: C = A B for dense
- * column-major M x K and K x N ComplexF64 matrices on the FP64 (precision 0) or FP32 (1) MFMA path.  No counterpart in the reference; it exists
- * so that the library's tests can check the MFMA tiling directly. */
+ * column-major M x K and K x N ComplexF64 matrices on the FP64 (precision 0) or FP32 (1) MFMA path.  No
+ * counterpart in the reference; it exists so that the library's tests can check the MFMA tiling directly. */
 int fdga_selftest_zgemm(int32_t M, int32_t N, int32_t K, int32_t precision, const double* A, const double* B, double* C);
 /* The same through tile shape `tile` (FDGA_TILE_*) over `grid` workgroups (0: one per output tile;
  * otherwise a multiple of 8, the workgroups looping over the tiles).  No counterpart in the reference. */
@@ -227,14 +228,16 @@ int fdga_group_sync(fdga_group* g);
 int fdga_group_time_iterations(fdga_group* g, int32_t strategy, int32_t n, double* ms);
 /* replay fdga_group_iterate(strategy, 1) from captured hipGraphs (as fdga_set_graph) */
 int fdga_group_set_graph(fdga_group* g, int32_t on);
-/* event timing of the two grouped contractions (which: 0 BSE_L_K3!, 1 BSE_K3!), ms summed */
+/* event timing of the two grouped contractions (which: 0 BSE_L_K3!, 1 BSE_K3!), ms summed; the members whose two
+ * contractions are one kernel count with 1 */
 int fdga_group_set_timing(fdga_group* g, int32_t on);
 int fdga_group_gemm_ms(const fdga_group* g, int32_t which, double* ms);
 /* tile shape and grid of contraction `which`; `computed`: non-idle output tiles of one launch */
 int fdga_group_tiles(fdga_group* g, int32_t which, int32_t* tile, int64_t* grid, int64_t* computed);
 int fdga_group_set_tiles(fdga_group* g, int32_t which, int32_t tile, int64_t grid);
-/* autotuner: times every tile shape and grid of both contractions (`reps` launches each) on the
- * members' current operands and keeps the fastest; the solver state is left as it was */
+/* autotuner: times every tile shape and grid of both contractions (`reps` launches each) on the members' current
+ * operands and keeps the fastest, BSE_L_K3! over the members that launch it (with none its settings stay); the
+ * solver state is left as it was (Fbuff.K3 is overwritten) */
 int fdga_group_autotune(fdga_group* g, int32_t reps);
 
 #ifdef __cplusplus
