@@ -1797,7 +1797,21 @@ int fdga_get(fdga_ctx* c, int32_t which, double* host) {
         if (!c->pi_band_G)
             return fail(c, "Πpp/Πph are stored on the band only and G has changed since the bubbles were computed: "
                            "call fdga_bubbles first");
-        if (bubbles_into(c, c->Pipp, c->Piph, c->G, false)) return -3;
+        // the other one may have been set since: it is kept
+        const bool pp = which == FDGA_PIPP;
+        double2 *other = pp ? c->Piph : c->Pipp, *keep = nullptr;
+        if (!(c->pi_band & (pp ? 2 : 1))) {
+            HIPCHK(c, hipMalloc((void**)&keep, c->nPiel * sizeof(double2)));
+            HIPCHK(c, hipMemcpyAsync(keep, other, c->nPiel * sizeof(double2), hipMemcpyDeviceToDevice, c->run));
+        }
+        const int rc = bubbles_into(c, c->Pipp, c->Piph, c->G, false);
+        if (keep) {
+            HIPCHK(c, hipMemcpyAsync(other, keep, c->nPiel * sizeof(double2), hipMemcpyDeviceToDevice, c->run));
+            if (tail_sums(c, other, pi_tail(c, other))) return -3;
+            HIPCHK(c, hipStreamSynchronize(c->run));
+            (void)hipFree(keep);
+        }
+        if (rc) return -3;
     }
     const size_t bytes = a.n * sizeof(double2);
     if (a.kind == 0) {
