@@ -77,8 +77,8 @@ __device__ __forceinline__ void b3_st(V* base, unsigned lane, V v) {
 // ms); not where it would spill (FP32 N = 72: 2.50 -> 2.63 ms).
 // Measured alone, 31 Ω x 256 P: FP32 N = 64 1.26 ms (79 TFLOP/s, matrix cores busy 56 % of the time; 4.0 GB of
 // traffic beyond L2), N = 72 2.50 ms, N = 80 2.33 ms (84 TFLOP/s), N = 96 3.94 ms (86); FP64 N = 64 1.91 ms
-// (52 TFLOP/s; 2.14 beside the iteration's K2 chain).  The separate equations took, at N = 64, 2.07 ms in FP32 (left equation 0.72, summed left
-// operand 0.37, full equation 0.97) and 4.2 ms in FP64.  What is left to the matrix rate is latency: a
+// (52 TFLOP/s; up to 2.07 on other cards).  The separate equations took, at N = 64, 2.07 ms in FP32 (left equation
+// 0.72, summed left operand 0.37, full equation 0.97) and 4.2 ms in FP64.  What is left to the matrix rate is latency: a
 // workgroup's phases are separated by four barriers per channel.
 template <bool F32, int NT, bool EXACT>
 __global__ __launch_bounds__(64 * (NT < 4 ? NT : 4), F32 && NT <= 4 ? 3 : 2) void k_bse3(Bse3Args A) {
