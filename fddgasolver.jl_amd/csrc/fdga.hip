@@ -87,7 +87,7 @@ struct fdga_ctx {
     std::string err;
     int NP = 1, NkG = 1, NG = 0;
     int NW1 = 0, NW2 = 0, NV2 = 0, NW3 = 0, NV3 = 0, NWP = 0, NVP = 0, nVP = 0;
-    int wb = 0;   // half-width of the band of the bubble mesh that the gathers read (W, tail sums)
+    int wb = 0;   // half-width of the band of the bubble mesh that the sums read entry by entry (Π, W)
     size_t nGel = 0, nPiel = 0, n1 = 0, n2 = 0, n3 = 0, nL = 0;
     double2 *Gbare = nullptr, *G0 = nullptr, *Sig0 = nullptr, *G = nullptr, *Sig = nullptr;
     double2 *Pi0pp = nullptr, *Pi0ph = nullptr, *Pipp = nullptr, *Piph = nullptr;
@@ -524,7 +524,6 @@ double2* pi_of(fdga_ctx* c, int ch, bool zero) {
     return ch == PCH ? c->Pipp : c->Piph;
 }
 
-// bound of every box of F, F0 and the RefVertex tables (frequency window of the gather-GEMVs)
 // Window bound of the SDE L-vertex sums: their channel evaluations keep the bosonic argument Ω
 // fixed (src/SDE.jl:79-217), so K1 is a constant there and the summand depends on ω only through the
 // K2 and K3 boxes (target and reference Vertex) and the RefVertex tables.
@@ -534,6 +533,7 @@ int sde_box_bound(const fdga_ctx* c) {
     if (d.ref_kind == 1) nk = std::max({nk, d.r_nK2f, d.r_nK3f});
     return nk + 1;
 }
+// bound of every box of F, F0 and the RefVertex tables (the window of the other sums evaluated point by point)
 int box_bound(const fdga_ctx* c) {
     const fdga_dims& d = c->d;
     int nk = std::max({d.nK1, d.nK2b, d.nK2f, d.nK3b, d.nK3f, d.tab_nb, d.tab_nf});
@@ -1563,8 +1563,8 @@ int fdga_create(fdga_ctx** out, const fdga_dims* dims) {
     c->NWP = 2 * d.nK1 - 1;
     c->nVP = d.nK1 * d.mPinu;
     c->NVP = 2 * c->nVP;
-    // the gathers read W and the tail sums only for |ω| <= Wc = NK + |Ω| + |ν| + 2 with Ω, ν in the
-    // K1 or K2 box (BSE_K1!, BSE_K2!, SDE L-vertices)
+    // every sum over ω depends on it only for |ω| <= Wc = NK + |Ω| + |ν| + 2 with Ω, ν in the K1 or K2 box
+    // (BSE_K1!, BSE_K2!, SDE L-vertices): the rest enters through the sums of Π outside the band
     c->wb = std::min(c->nVP, box_bound(c) + std::max(d.nK1 - 1, d.nK2b - 1 + d.nK2f) + 3);
     c->nGel = (size_t)c->NG * c->NkG;
     c->nPiel = (size_t)c->NVP * c->NWP * c->NP;

@@ -6,7 +6,7 @@
 //   bubbles_real_space!    k_dft2_rows (G -> G(R)) + k_bubble_nl (products and bfft over R' in LDS)
 //   s-wave averages        k_pavg_multi
 //   build_K3_cache!        k_cache               gather: Γ_irr / F0 / F-base caches
-//   BSE_L_K3!, BSE_K3!     zgemm_tiles<...>      batched complex GEMM on v_mfma_f64_16x16x4f64
+//   BSE_L_K3!, BSE_K3!     lattice :fdPA k_bse3 (fdga_bse3.h); else zgemm_tiles_t<...>, batched complex GEMMs on MFMA
 //   BSE_K1!                k_k1                  sums over the K2 boxes, the rest from the sums of Π
 //   BSE_K2!, BSE_L_K2!     local solver fdga_local.h; lattice k_k2nl_*, k_lk2nl_table and GEMMs
 //   SDE!                   k_seg_sde (fdga_local.h), k_sde_L_nl, k_sde_L, k_sde_sigma_*, k_u2_*, k_occupation
@@ -2259,7 +2259,7 @@ __device__ __forceinline__ void far_terms(int nVP, int wb, int lo, int hi, int l
         add(side, k == 0 ? -1 : (side ? hi : nVP - wb - 1) + k);
     }
 }
-// Frequency window of the gather-GEMVs.  Every vertex term that depends on the summed
+// Frequency window of the sums that are evaluated point by point (forms, RefVertex SDE, lattice K2 tables).  Every vertex term that depends on the summed
 // frequency ω is supported on |ω| <= Wc = NK + |m| + |n| + 2, where NK bounds every box of the
 // vertex (K1 boxes reach furthest: their bosonic argument is a sum or difference of Ω, ν, ω).
 // Beyond the window the summand is T(ω_far) W(ω) with T(ω_far) the same value for every ω on

@@ -401,7 +401,8 @@ autotune!(S::HipSolver; reps::Integer = 3) =
     check(context(S), ccall((:fdga_autotune, libfdga), Cint, (Ptr{Cvoid}, Int32), context(S), Int32(reps)))
 
 # solver groups: several solvers (a parameter sweep) iterated together, the contractions of all of
-# them in one launch each; destroy the group before its members
+# them in one launch each (:fdPA within the fused contraction's limit: one per member); destroy the group
+# before its members
 function group(solvers::Vector{<:HipSolver})
     ctxs = [context(S) for S in solvers]
     g = Ref{Ptr{Cvoid}}(C_NULL)
