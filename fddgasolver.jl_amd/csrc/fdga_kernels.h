@@ -2296,8 +2296,8 @@ struct K1Args {
     int nk, ntot;
 };
 struct K1Row { double2 raw, l, r, tot; };
-// o: p, or a and then t
-template <bool PH>
+// o: p, or a and then t; K1 false: the sums of W alone
+template <bool PH, bool K1>
 __device__ __forceinline__ void k1_row(const K1Args& a, int m, int p, int lane, K1Row& oa, K1Row& ot) {
     const size_t row = (size_t)(m + a.nWP - 1) + (size_t)(2 * a.nWP - 1) * p;
     const double2* pi = (PH ? a.Pph : a.Ppp) + (size_t)(2 * a.nVP) * row + a.nVP;
@@ -2317,22 +2317,22 @@ __device__ __forceinline__ void k1_row(const K1Args& a, int m, int p, int lane, 
         for (int w = lo + lane; w < hi; w += WAVE) {
             const int wc = PH ? w : crossing(m, w, PCH);
             const double2 P = pi[w], d = csub(P, pi0[w]);
-            const double2 l = box_k2(a.L[C], m, wc, p), f = box_k2(a.F.g[C], m, w, p);
+            const double2 l = box_k2(a.L[C], m, wc, p), f = K1 ? box_k2(a.F.g[C], m, w, p) : czero();
             double2 gc = czero(), gw = czero();
             if (f0.kind == 1) {
                 gc = box_k2(f0.g[C], m, wc, 0);
-                gw = PH ? gc : box_k2(f0.g[C], m, w, 0);
+                if (K1) gw = PH ? gc : box_k2(f0.g[C], m, w, 0);
             }
             const double2 x = cadd(cmul(d, gc), cmul(P, l));
             tot = cadd(tot, x);
-            k = cadd(k, cmul(cadd(gw, f), cadd(x, cadd(cmul(d, c0), cmul(P, kL)))));
+            if (K1) k = cadd(k, cmul(cadd(gw, f), cadd(x, cadd(cmul(d, c0), cmul(P, kL)))));
             if (PH) {
                 const double2 lt = csub(cscale(box_k2(a.L[TCH], m, w, p), 2.0), l);
-                const double2 ft = csub(cscale(box_k2(a.F.g[TCH], m, w, p), 2.0), f);
+                const double2 ft = K1 ? csub(cscale(box_k2(a.F.g[TCH], m, w, p), 2.0), f) : czero();
                 const double2 gt = f0.kind == 1 ? csub(cscale(box_k2(f0.g[TCH], m, w, 0), 2.0), gc) : czero();
                 const double2 xt = cadd(cmul(d, gt), cmul(P, lt));
                 tott = cadd(tott, xt);
-                kt = cadd(kt, cmul(cadd(gt, ft), cadd(xt, cadd(cmul(d, c0t), cmul(P, kLt)))));
+                if (K1) kt = cadd(kt, cmul(cadd(gt, ft), cadd(xt, cadd(cmul(d, c0t), cmul(P, kLt)))));
             }
         }
     }
@@ -2341,7 +2341,7 @@ __device__ __forceinline__ void k1_row(const K1Args& a, int m, int p, int lane, 
         o.l = far(0);
         o.r = far(1);
         o.tot = cadd(wave_sum2(sum), far(2));
-        o.raw = cscale(cadd(cmul(cadd(c, k1), o.tot), wave_sum2(kk)), sc);
+        if (K1) o.raw = cscale(cadd(cmul(cadd(c, k1), o.tot), wave_sum2(kk)), sc);
     };
     finish(oa, c0, kL, tot, k, own_k1<C>(a.F.g, m, p), a.T);
     if (PH) finish(ot, c0t, kLt, tott, kt, own_k1<TCH>(a.F.g, m, p), -a.T);
@@ -2356,6 +2356,7 @@ __device__ __forceinline__ void k1_store(const K1Args& a, int ch, int m, int p, 
     }
 }
 // block q of nb (a multiple of 8)
+template <bool K1>
 __device__ __forceinline__ void k1_block(const K1Args& a, int q, int nb) {
     const int lane = threadIdx.x & (WAVE - 1);
     const int blk = q % 8 * (nb / 8) + q / 8;
@@ -2379,7 +2380,7 @@ __device__ __forceinline__ void k1_block(const K1Args& a, int q, int nb) {
     const bool st = sums || (!a.sym.ncls && in_b(m, a.n2b));
     K1Row ra{}, rt{};
     if (pw) {
-        k1_row<false>(a, m, p, lane, ra, rt);
+        k1_row<false, K1>(a, m, p, lane, ra, rt);
         if (st) k1_store(a, PCH, m, p, ra, lane);
         for (int k = b + lane; k < e; k += WAVE) {
             const int code = a.sym.member(cls, k);
@@ -2387,7 +2388,7 @@ __device__ __forceinline__ void k1_block(const K1Args& a, int q, int nb) {
         }
         return;
     }
-    k1_row<true>(a, m, p, lane, ra, rt);
+    k1_row<true, K1>(a, m, p, lane, ra, rt);
     const bool ma = a.mask >> ACH & 1, mt = a.mask >> TCH & 1;
     if (st && ma) k1_store(a, ACH, m, p, ra, lane);
     if (st && mt) k1_store(a, TCH, m, p, rt, lane);
@@ -2398,12 +2399,12 @@ __device__ __forceinline__ void k1_block(const K1Args& a, int q, int nb) {
         if (mt) a.Kt[o] = cscale(cadd(sym_apply(code & 3, rt.raw), ka), 0.5);   // src/BSE_templates.jl:29-33
     }
 }
-__global__ __launch_bounds__(256) void k_k1(K1Args a) { k1_block(a, (int)blockIdx.x, (int)gridDim.x); }
+__global__ __launch_bounds__(256) void k_k1(K1Args a) { k1_block<true>(a, (int)blockIdx.x, (int)gridDim.x); }
 // the weights (blocks [0, nw), wx along ω, wy along Ω) and the sums that BSE_K2! called on its own takes, in one launch
 __global__ __launch_bounds__(256) void k_k2_inputs(WArgs w, K1Args k, int wx, int wy, int nw) {
     const int b = (int)blockIdx.x;
     if (b < nw) bse_w_block(w, b % wx, b / wx % wy, b / (wx * wy));
-    else k1_block(k, b - nw, (int)gridDim.x - nw);
+    else k1_block<false>(k, b - nw, (int)gridDim.x - nw);
 }
 
 // BSE_K2!: K2(Ω, ν, P) = T s Σ_ω [F(Ω,ν,ω) - F(Ω,∞,ω)] W(ω) + FL.K2 (t: 2 FLt - FLa).
