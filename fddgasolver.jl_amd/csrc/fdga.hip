@@ -926,7 +926,14 @@ static int launch_lk2(fdga_ctx* c) {
         return sym_fill(c, c->FL[CH].K2, sym_k2(c, CH).ncls ? c->sg[CH == PCH ? SG_PP2 : SG_PH2].repop : nullptr,
                         c->n2 * c->NP);
     }
-    return launch_seg_k2<true>(c, 1 << CH);
+    const SymCls sym = sym_k2(c, CH);
+    const size_t n = nclass(sym, c->n2);
+    if (n * 2 * c->wb > LK2_POINTS) return launch_seg_k2<true>(c, 1 << CH);
+    k_point_lk2<CH><<<cdiv(n * WAVE, 256), 256, 0, c->run>>>(c->FL[CH].K2, c->FL[ACH].K2, pi_of(c, CH, true), vtx_F(c),
+                                                            c->d.nK2b, c->d.nK2f, c->d.nK1, c->nVP, c->d.T * kSign[CH],
+                                                            box_bound(c), sym);
+    LAUNCHCHK(c);
+    return 0;
 }
 
 // BSE_L_K2! of the three channels: one launch for the local solver

@@ -329,6 +329,36 @@ __global__ __launch_bounds__(seg_nt(ROWS)) void k_seg_k2(SegK2 A) {
     }
 }
 
+// BSE_L_K2! of one channel point by point: Σ_ω Γ(Ω, ν, ω) Π0(ω) F0(Ω, ω~, ∞) over the window, Γ without F0 and the own
+// channel (zero outside it).  One wave per output class, lanes over ω: all of a point's loads are in flight together,
+// which for a call on its own is worth more than k_seg_k2's fewer instructions until these set the time.  p channel
+// (the three channels), against k_seg_k2: SIAM boxes 33, 0.1 M points, 6.0 us (in one launch 7.0); boxes 60, 1.8 M,
+// 12.5 (15.4) and 53.0 (58.8), with a reference vertex 13.7 (15.8) and 59.8 (61.2); boxes 128 with groups, 2.7 M, 16.0
+// (16.4) and 62.6 (64.9), with a reference vertex 17.4 (17.2) and 70.6 (67.8); without groups, 8.4 M, 38.8 (35.2).
+constexpr size_t LK2_POINTS = (size_t)2 << 20;   // the line between the two: even from there on
+template <int CH>
+__global__ __launch_bounds__(256) void k_point_lk2(double2* __restrict__ out, const double2* __restrict__ outa,
+                                                   const double2* __restrict__ Pi0, VtxV F, int n2b, int n2f, int nWP,
+                                                   int nVP, double scale, int NK, SymCls sym) {
+    constexpr int SP = ChSpin<CH>::SP, FLG = FL_ALL & ~FL_F0 & ~(FL_GP << CH);
+    const int wid = (int)blockIdx.x * (256 / WAVE) + seg_wave(), lane = threadIdx.x & (WAVE - 1);
+    const int NW2 = 2 * n2b - 1;
+    if (wid >= sym.count(NW2 * 2 * n2f)) return;
+    const int o0 = sym.rep(wid), m = o0 % NW2 - (n2b - 1), v = o0 / NW2 - n2f, Wc = window(NK, m, v);
+    const double2* P0 = Pi0 + (size_t)(2 * nVP) * (m + nWP - 1) + nVP;
+    double2 s = czero();
+    for (int w = max(-nVP, -Wc) + lane; w <= min(nVP - 1, Wc); w += WAVE)
+        s = cadd(s, cmul(cmul(F.eval(m, v, w, 0, CH, SP, FLG), P0[w]), F.f0.eval(m, crossing(m, w, CH), FDGA_INF, CH, SP)));
+    const double2 raw = cscale(wave_sum2(s), scale);
+    int b, e;
+    sym.range(wid, b, e);
+    for (int k = b + lane; k < e; k += WAVE) {
+        const int code = sym.member(wid, k), o = code >> 2;
+        const double2 x = sym_apply(code & 3, raw);
+        out[o] = CH == TCH ? cscale(cadd(x, outa[o]), 0.5) : x;
+    }
+}
+
 // The SDE L-vertices of one Vertex level (src/SDE.jl:79-217), the channels at the fixed bosonic argument Ω:
 //   Lpp(Ω, ν) = T U [(K1p + K2p(ν)) ΣΠpp + Σ_n K2p(n) Πpp(Ω - n - 1) + Σ_n K3p(n, ν) Πpp(Ω - n - 1)]
 //   Lph(Ω, ν) = T U Σ_{r = a, t} [(K1r + K2r(ν)) ΣΠph + Σ_n K2r(n) Πph(n) + Σ_n K3r(ν, n) Πph(n)]
